@@ -437,6 +437,18 @@ int ssc_kernel_combine_f32(const float *weight, const float *basis,
                            int32_t kernel_volume, int32_t c_in, int32_t c_out,
                            float *out /* [K,c_in,c_out] */, ssc_stream_t stream);
 
+/* Its gradient with respect to the weights (the reference differentiates the einsums,
+ * ss_conv/utils/kernel.py:267-299): d_weight, laid out as `weight`, from d_dense[K,c_in,c_out].
+ *   first_out[n_fields_out], first_in[n_fields_in]: first channel of every field (i,u) / (j,v);
+ *   entries of d_weight that no block owns are not written. */
+int ssc_kernel_combine_bwd_f32(const float *d_dense, const float *basis,
+                               const int32_t *chan_out, const int32_t *chan_in,
+                               const int32_t *blocks, const int32_t *first_out,
+                               int32_t n_fields_out, const int32_t *first_in,
+                               int32_t n_fields_in, int32_t n_irreps_in,
+                               int32_t kernel_volume, int32_t c_in, int32_t c_out,
+                               float *d_weight, ssc_stream_t stream);
+
 /* The same synthesis with the filters also written in the convolution kernel's packed order
  * (what ssc_conv_pack_filters_f32 makes of `out` read as [K, Cin, Cout]; `packed` of
  * ssc_conv_packed_bytes(kernel_volume, c_in, c_out) bytes): a layer that synthesises its

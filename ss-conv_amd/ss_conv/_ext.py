@@ -102,6 +102,8 @@ _SIGNATURES = {
                                              ctypes.POINTER(_i32)]),
     "ssc_kernel_combine_f32": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32,
                                               _vp, _vp]),
+    "ssc_kernel_combine_bwd_f32": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32,
+                                                  _i32, _i32, _i32, _i32, _vp, _vp]),
     "ssc_kernel_combine_packed_f32": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
                                                      _i32, _vp, _vp, _sz, _vp]),
     "ssc_pool_workspace_bytes": (_sz, [_i64, _i32]),
@@ -1369,6 +1371,20 @@ def kernel_combine(weight, basis, chan_out, chan_in, blocks, n_irreps_in, kernel
         return out, buf
     _check(_lib.ssc_kernel_combine_packed_f32(*args, buf.data_ptr(), buf.numel(), _stream(weight)))
     return out, buf
+
+
+def kernel_combine_backward(d_dense, basis, chan_out, chan_in, blocks, first_out, first_in,
+                            n_irreps_in, kernel_volume, n_weight):
+    """Gradient of the flat weight vector [n_weight] from that of the dense kernel
+    [K, Cin, Cout] (the contraction of kernel_combine against the same basis)."""
+    _need_gpu(d_dense, basis, chan_out, chan_in, blocks)
+    d_dense = d_dense.float().contiguous()
+    d_weight = torch.empty((n_weight,), dtype=torch.float32, device=d_dense.device)
+    _check(_lib.ssc_kernel_combine_bwd_f32(
+        _ptr(d_dense), _ptr(basis), _ptr(chan_out), _ptr(chan_in), _ptr(blocks), _ptr(first_out),
+        first_out.numel(), _ptr(first_in), first_in.numel(), int(n_irreps_in), int(kernel_volume),
+        d_dense.size(1), d_dense.size(2), _ptr(d_weight), _stream(d_dense)))
+    return d_weight
 
 
 def flush_combine():

@@ -125,12 +125,13 @@ def orthogonal_(tensor, gain=1):
 class _Combine(torch.autograd.Function):
     """dense[k, (j,v,b), (i,u,a)] = sum_n weight_ij[u,v,n] * basis_ij[n,a,b,k] in one native
     launch; the gradient with respect to the weights is the same contraction against the
-    fixed basis, block by block (the blocks are small: torch einsum)."""
+    fixed basis, one launch as well."""
 
     @staticmethod
     def forward(ctx, weight, module, pack):
-        basis, chan_out, chan_in, blocks, _ = module._tables
+        basis, chan_out, chan_in, blocks = module._tables[:4]
         ctx.module = module
+        ctx.tables = module._tables
         out = _ext.kernel_combine(weight.detach().float().contiguous(), basis, chan_out, chan_in,
                                   blocks, len(module.multiplicities_in), module.size ** 3,
                                   module.n_in, module.n_out, packed=bool(pack),
@@ -141,23 +142,24 @@ class _Combine(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):  # grad: [K, Cin, Cout]
-        m = ctx.module
-        K = m.size ** 3
-        grads = []
-        o_off = 0
-        for i, (mi, di) in enumerate(zip(m.multiplicities_out, m.dims_out)):
-            i_off = 0
-            for j, (mj, dj) in enumerate(zip(m.multiplicities_in, m.dims_in)):
-                kij = getattr(m, "kernel_{}_{}".format(i, j))
-                if kij is not None:
-                    nb = kij.size(0)
-                    g = grad[:, i_off:i_off + mj * dj, o_off:o_off + mi * di]
-                    g = g.reshape(K, mj, dj, mi, di)
-                    basis = kij.to(grad.dtype).reshape(nb, di, dj, K)
-                    grads.append(torch.einsum("kvbua,nabk->uvn", g, basis).reshape(-1))
-                i_off += mj * dj
-            o_off += mi * di
-        return torch.cat(grads), None, None
+        return _CombineGrad.apply(grad, ctx.module, ctx.tables), None, None
+
+
+class _CombineGrad(torch.autograd.Function):
+    """The gradient above as a function of its own: linear in `grad`, so that it can be
+    differentiated again, by the synthesis itself."""
+
+    @staticmethod
+    def forward(ctx, grad, module, tables):
+        basis, chan_out, chan_in, blocks, _, first_out, first_in = tables
+        ctx.module = module
+        return _ext.kernel_combine_backward(grad, basis, chan_out, chan_in, blocks, first_out,
+                                            first_in, len(module.multiplicities_in),
+                                            module.size ** 3, module.weight.numel())
+
+    @staticmethod
+    def backward(ctx, grad):
+        return _Combine.apply(grad, ctx.module, False), None, None
 
 
 class SE3Kernel(torch.nn.Module):
@@ -242,9 +244,16 @@ class SE3Kernel(torch.nn.Module):
                 w_off += mi * mj * nb
                 b_off += nb * self.dims_out[i] * self.dims_in[j] * K
         assert w_off == self.weight.numel()
-        as_i32 = lambda rows: torch.tensor(rows, dtype=torch.int32, device=device).contiguous()
-        self._tables = (torch.cat(pieces).contiguous(), as_i32(chan_out), as_i32(chan_in),
-                        as_i32(blocks), device)
+        # (the first channel of every field is for the gradient)
+        tables = [chan_out, chan_in, blocks,
+                  [(c,) for c, (_, _, a) in enumerate(chan_out) if a == 0],
+                  [(c,) for c, (_, _, b) in enumerate(chan_in) if b == 0]]
+        flat = torch.tensor([x for rows in tables for row in rows for x in row],
+                            dtype=torch.int32, device=device)  # one copy to the device for all
+        out, ins, blk, first_out, first_in = (
+            piece.view(len(rows), -1) for piece, rows in
+            zip(flat.split([len(rows) * len(rows[0]) for rows in tables]), tables))
+        self._tables = (torch.cat(pieces).contiguous(), out, ins, blk, device, first_out, first_in)
 
     def combination(self, weight, pack=False):
         """[Cout, Cin, k, k, k] view of the natively contracted [K, Cin, Cout] kernel

@@ -1005,6 +1005,47 @@ def test_kernel_combine_matches_einsum(oracle, device):
         assert torch.equal(fused, packed)
 
 
+@pytest.mark.parametrize("rs_in,rs_out,size", [
+    ([(1, 0)], [(1, 0)], 1),                             # one element, one basis function
+    ([(3, 0)], [(2, 0), (1, 1), (1, 2)], 3),             # blocks without a basis function
+    ([(1, 0), (2, 2)], [(2, 1), (1, 4)], 5),             # > 256 elements of a basis function
+    ([(16, 0), (16, 1)], [(5, 0), (3, 1), (2, 3)], 3),
+    ([(2, 3)], [(1, 4), (3, 3)], 7),                     # more than 8 basis functions
+])
+def test_kernel_combine_gradient(device, rs_in, rs_out, size):
+    """The weight gradient of the synthesis against the contraction in float64, block by block."""
+    from ss_conv.utils.kernel import SE3Kernel
+    torch.manual_seed(1)
+    ker = SE3Kernel(rs_in, rs_out, size).to(device)
+    dense = ker()
+    d_out = torch.randn(dense.shape, device=device, requires_grad=True)
+    grad, = torch.autograd.grad(dense, ker.weight, d_out, create_graph=True)
+    d_dense = d_out.detach().cpu().reshape(ker.n_out, ker.n_in, size ** 3).permute(2, 1, 0)
+    want, scale = [], []
+    g64 = d_dense.double()
+    o_off = 0
+    for i, (mi, di) in enumerate(zip(ker.multiplicities_out, ker.dims_out)):
+        i_off = 0
+        for j, (mj, dj) in enumerate(zip(ker.multiplicities_in, ker.dims_in)):
+            kij = getattr(ker, "kernel_%d_%d" % (i, j))
+            if kij is not None:
+                b64 = kij.cpu().double().reshape(-1, di, dj, size ** 3)
+                g = g64[:, i_off:i_off + mj * dj, o_off:o_off + mi * di]
+                g = g.reshape(size ** 3, mj, dj, mi, di)
+                for dst, x, b in ((want, g, b64), (scale, g.abs(), b64.abs())):
+                    dst.append(torch.einsum("kvbua,nabk->uvn", x, b).reshape(-1))
+            i_off += mj * dj
+        o_off += mi * di
+    want, scale = torch.cat(want), torch.cat(scale)
+    got = grad.detach().cpu().double()
+    # fp32 sums of at most 9 * 9 * 343 products: a thread adds 109 of them, then 8 levels
+    assert bool(((got - want).abs() <= 128 * 2.0 ** -24 * scale + 1e-30).all())
+    # linear in d_out, so its own derivative along t is the synthesis of t
+    t = torch.randn_like(ker.weight)
+    again, = torch.autograd.grad(grad, d_out, t)
+    assert torch.equal(again, ker.combination(t))
+
+
 def test_convolution_layer_end_to_end(oracle, device):
     """Point2Voxel -> Convolution against the oracle pipeline and against dense conv3d."""
     import torch.nn.functional as F
