@@ -829,6 +829,27 @@ int ssc_bnact_bwd_sums_f32(const float *x, const float *dy /* [n,c_out] */, int6
                            size_t workspace_bytes /* ssc_bn_workspace_bytes(n, c_in) */,
                            ssc_stream_t stream);
 
+/* pre_bias[c] of the calls above: scalar_bias on the first n_scalar columns, gate_bias on the
+ * n_gates columns from gate_first on, 0 elsewhere. */
+int ssc_bnact_pre_bias_f32(int32_t c, const float *scalar_bias /* [n_scalar] */, int32_t n_scalar,
+                           const float *gate_bias /* [n_gates] */, int32_t gate_first,
+                           int32_t n_gates, float *pre_bias /* [c] */, ssc_stream_t stream);
+
+/* From the sums of ssc_bnact_bwd_sums_f32 over n >= 1 rows, each output optional (NULL):
+ *   d_scalar_bias[n_scalar], d_gate_bias[n_gates]: the sums of their columns;
+ *   d_weight[f] = field_rstd[f] * A[f], A[f] = sum of sums[c + ...] over the field's columns;
+ *   d_bias[scalar] = sums[column];
+ *   dz_mean[c] = sums[c] / n for scalar columns, 0 elsewhere;
+ *   coef[c] = scale[c] * field_rstd[f]^2 * A[f] / n.
+ * field_of NULL: no batch normalisation, the first two only. */
+int ssc_bnact_bwd_coef_f32(int64_t n, int32_t c, const float *sums /* [2*c] */,
+                           const int32_t *field_of, const int32_t *scalar_idx,
+                           const int32_t *field_first, const int32_t *field_dim,
+                           const float *scale, const float *field_rstd, int32_t n_scalar,
+                           int32_t gate_first, int32_t n_gates, float *d_weight, float *d_bias,
+                           float *d_scalar_bias, float *d_gate_bias, float *dz_mean, float *coef,
+                           ssc_stream_t stream);
+
 int ssc_bnact_bwd_f32(const float *x, const float *dy, int64_t n, int32_t c_in, int32_t c_out,
                       const float *shift, const float *scale, const float *add,
                       const float *pre_bias, const int32_t *out_mode, const int32_t *gate_col,

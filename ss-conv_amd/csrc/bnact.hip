@@ -235,6 +235,51 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Bias in front of the activations, one entry per input column: the scalar biases on the
+// leading columns, the gates' biases from gate_first on, 0 elsewhere.
+__global__ void __launch_bounds__(256)
+    bnact_pre_bias_kernel(int C, const float *__restrict__ scalar_bias, int n_scalar,
+                          const float *__restrict__ gate_bias, int gate_first, int n_gates,
+                          float *__restrict__ pre_bias) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= C) return;
+  float v = 0.f;
+  if (c < n_scalar) v = scalar_bias[c];
+  if (c >= gate_first && c < gate_first + n_gates) v = gate_bias[c - gate_first];
+  pre_bias[c] = v;
+}
+
+// Everything the backward pass derives from the column sums: the parameter gradients and what
+// the batch statistics contribute to dx.  A thread per column; it adds up its field's columns
+// (at most a few) itself, in order, so one launch needs no barrier.  The work is nothing, the
+// launch is all: as 14 tensor operations this took 75 us of a block's backward pass with the
+// queue full (a dependent launch every 5 us) and up to 250 us where the host was behind; one
+// launch takes 5 us.
+__global__ void __launch_bounds__(256)
+    bnact_bwd_coef_kernel(int C, float inv_n, const float *__restrict__ sums /* [2C] */,
+                          const int32_t *__restrict__ field_of,
+                          const int32_t *__restrict__ scalar_idx,
+                          const int32_t *__restrict__ field_first,
+                          const int32_t *__restrict__ field_dim, const float *__restrict__ scale,
+                          const float *__restrict__ rstd, int n_scalar, int gate_first,
+                          int n_gates, float *__restrict__ d_weight, float *__restrict__ d_bias,
+                          float *__restrict__ d_scalar_bias, float *__restrict__ d_gate_bias,
+                          float *__restrict__ dz_mean, float *__restrict__ coef) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= C) return;
+  const float dz = sums[c];
+  if (d_scalar_bias && c < n_scalar) d_scalar_bias[c] = dz;
+  if (d_gate_bias && c >= gate_first && c < gate_first + n_gates) d_gate_bias[c - gate_first] = dz;
+  if (!field_of) return;
+  const int f = field_of[c], first = field_first[f], si = scalar_idx[c];
+  float a = 0.f;
+  for (int j = 0; j < field_dim[f]; ++j) a += sums[C + first + j];
+  if (d_weight && c == first) d_weight[f] = rstd[f] * a;
+  if (d_bias && si >= 0) d_bias[si] = dz;
+  if (dz_mean) dz_mean[c] = si >= 0 ? dz * inv_n : 0.f;
+  if (coef) coef[c] = scale[c] * (rstd[f] * rstd[f] * a) * inv_n;
+}
+
 // Per-column constants of the normalisation (identity when the pointers are null).
 struct ColAffine {
   const float *shift, *scale, *add, *pre_bias;
@@ -938,6 +983,42 @@ int ssc_bnact_bwd_sums_f32(const float *x, const float *dy, int64_t n, int32_t c
   hipLaunchKernelGGL(bn_colsum_kernel, dim3((unsigned)ceil_div(2 * c_in, kColsumCols)), dim3(256), 0, s,
                      partial, sh.blocks, 2 * c_in, 1.0, (const int32_t *)nullptr, sums);
   SSC_LAUNCH_CHECK("bnact_bwd_sums");
+  return SSC_OK;
+}
+
+int ssc_bnact_pre_bias_f32(int32_t c, const float *scalar_bias, int32_t n_scalar,
+                           const float *gate_bias, int32_t gate_first, int32_t n_gates,
+                           float *pre_bias, ssc_stream_t stream) {
+  SSC_CHECK(c >= 1 && n_scalar >= 0 && n_scalar <= c && n_gates >= 0 && gate_first >= 0 &&
+                gate_first <= c - n_gates,
+            SSC_EINVAL, "bad shape: c %d, %d scalars, gates %d + %d", c, n_scalar, gate_first,
+            n_gates);
+  SSC_CHECK(pre_bias && (scalar_bias || n_scalar == 0) && (gate_bias || n_gates == 0), SSC_EINVAL,
+            "NULL pointer argument");
+  hipLaunchKernelGGL(bnact_pre_bias_kernel, dim3((unsigned)ceil_div(c, 256)), dim3(256), 0,
+                     (hipStream_t)stream, c, scalar_bias, n_scalar, gate_bias, gate_first, n_gates,
+                     pre_bias);
+  SSC_LAUNCH_CHECK("bnact_pre_bias");
+  return SSC_OK;
+}
+
+int ssc_bnact_bwd_coef_f32(int64_t n, int32_t c, const float *sums, const int32_t *field_of,
+                           const int32_t *scalar_idx, const int32_t *field_first,
+                           const int32_t *field_dim, const float *scale, const float *field_rstd,
+                           int32_t n_scalar, int32_t gate_first, int32_t n_gates, float *d_weight,
+                           float *d_bias, float *d_scalar_bias, float *d_gate_bias, float *dz_mean,
+                           float *coef, ssc_stream_t stream) {
+  SSC_CHECK(n >= 1 && c >= 1 && n_scalar >= 0 && n_gates >= 0 && gate_first >= 0, SSC_EINVAL,
+            "bad shape: n %lld, c %d", (long long)n, c);
+  SSC_CHECK(sums, SSC_EINVAL, "NULL pointer argument");
+  SSC_CHECK(field_of ? scalar_idx && field_first && field_dim && scale && field_rstd
+                     : !d_weight && !d_bias && !dz_mean && !coef,
+            SSC_EINVAL, "the field tables are incomplete");
+  hipLaunchKernelGGL(bnact_bwd_coef_kernel, dim3((unsigned)ceil_div(c, 256)), dim3(256), 0,
+                     (hipStream_t)stream, c, (float)(1.0 / (double)n), sums, field_of, scalar_idx,
+                     field_first, field_dim, scale, field_rstd, n_scalar, gate_first, n_gates,
+                     d_weight, d_bias, d_scalar_bias, d_gate_bias, dz_mean, coef);
+  SSC_LAUNCH_CHECK("bnact_bwd_coef");
   return SSC_OK;
 }
 

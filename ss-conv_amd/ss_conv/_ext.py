@@ -102,6 +102,9 @@ _SIGNATURES = {
                                              ctypes.POINTER(_i32)]),
     "ssc_kernel_combine_f32": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32,
                                               _vp, _vp]),
+    "ssc_bnact_pre_bias_f32": (ctypes.c_int, [_i32, _vp, _i32, _vp, _i32, _i32, _vp, _vp]),
+    "ssc_bnact_bwd_coef_f32": (ctypes.c_int, [_i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32,
+                                              _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "ssc_kernel_combine_bwd_f32": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32,
                                                   _i32, _i32, _i32, _i32, _vp, _vp]),
     "ssc_kernel_combine_packed_f32": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
@@ -1717,6 +1720,46 @@ def bnact_backward_sums(x, dy, shift, scale, add, pre_bias, out_mode, gate_col, 
         _ptr(pre_bias), _ptr(out_mode), _ptr(gate_col), _ptr(gated_first), _ptr(gated_dim),
         int(act_scalar), int(act_gate), sums.data_ptr(), ws.data_ptr(), ws.numel(), _stream(x)))
     return sums
+
+
+def bnact_pre_bias(c, scalar_bias, gate_bias, n_scalar, gate_first, n_gates, device):
+    """[c] float32: scalar_bias [n_scalar] on the leading columns, gate_bias [n_gates] from
+    gate_first on (either may be None), zeros elsewhere."""
+    def given(bias, n):
+        if bias is None or n == 0:
+            return None, 0
+        bias = bias.detach().to(device=device, dtype=torch.float32).expand(n).contiguous()
+        return bias, n
+    scalar_bias, n_scalar = given(scalar_bias, n_scalar)
+    gate_bias, n_gates = given(gate_bias, n_gates)
+    out = torch.empty(c, dtype=torch.float32, device=device)
+    _check(_lib.ssc_bnact_pre_bias_f32(c, _ptr(scalar_bias), n_scalar, _ptr(gate_bias),
+                                       gate_first if n_gates else 0, n_gates, out.data_ptr(),
+                                       _stream(out)))
+    return out
+
+
+def bnact_backward_coef(n, sums, layout, scale, rstd, n_scalar_act, c_out, n_gates, want, training):
+    """What follows from the column sums of a backward pass over n rows.  want: which of the
+    gradients of (weight, bias, scalar bias, gate bias) are asked for; training: the batch's
+    own statistics were used.  Returns those four, dz_mean and coef, None where not wanted.
+    layout None: no batch norm."""
+    c = sums.size(1)
+    made = lambda n, yes: sums.new_empty(n) if yes else None  # noqa: E731
+    want_w, want_b, want_sb, want_gb = want
+    d_sb, d_gb = made(n_scalar_act, want_sb), made(n_gates, want_gb)
+    d_weight = d_bias = dz_mean = coef = None
+    tables = (None,) * 4
+    if layout is not None:
+        tables = tuple(layout[k] for k in ("field_of", "scalar_idx", "field_first", "field_dim"))
+        d_weight = made(rstd.numel(), want_w)
+        d_bias = made(layout["n_scalar"], want_b)
+        dz_mean, coef = made(c, training), made(c, training)
+    _check(_lib.ssc_bnact_bwd_coef_f32(
+        n, c, sums.data_ptr(), *[_ptr(t) for t in tables], _ptr(scale), _ptr(rstd),
+        n_scalar_act, c_out, n_gates, _ptr(d_weight), _ptr(d_bias), _ptr(d_sb), _ptr(d_gb),
+        _ptr(dz_mean), _ptr(coef), _stream(sums)))
+    return d_weight, d_bias, d_sb, d_gb, dz_mean, coef
 
 
 def bnact_backward(x, dy, shift, scale, add, pre_bias, out_mode, gate_col, gated_first, gated_dim,

@@ -52,10 +52,7 @@ def field_layout(Rs):
     as_t = lambda v: torch.tensor(v, dtype=torch.int32)  # noqa: E731
     return {"field_of": as_t(field_of), "scalar_idx": as_t(scalar_idx),
             "field_first": as_t(field_first), "field_dim": as_t(field_dim),
-            # index tensors of the same layout for the few torch ops of the backward pass
-            "field_of_long": torch.tensor(field_of, dtype=torch.long),
-            "scalar_cols": torch.tensor([c for c, s in enumerate(scalar_idx) if s >= 0],
-                                        dtype=torch.long)}
+            "n_scalar": s}
 
 
 def gate_layout(Rs, has_scalar_act, has_gate_act):
@@ -180,11 +177,8 @@ class _BnAct(torch.autograd.Function):
                 plan.running_var)
         pre_bias = None
         if scalar_bias is not None or gate_bias is not None:
-            pre_bias = x.new_zeros(c_in)
-            if scalar_bias is not None:
-                pre_bias[:plan.n_scalar_act] = scalar_bias.detach()
-            if gate_bias is not None:
-                pre_bias[plan.c_out:plan.c_out + plan.n_gates] = gate_bias.detach()
+            pre_bias = _ext.bnact_pre_bias(c_in, scalar_bias, gate_bias, plan.n_scalar_act,
+                                           plan.c_out, plan.n_gates, x.device)
         act = plan.act or {}
         y = _ext.bnact_forward(x, shift, scale, add, pre_bias, act.get("out_mode"),
                                act.get("gate_col"), plan.act_scalar, plan.act_gate, plan.c_out)
@@ -192,6 +186,7 @@ class _BnAct(torch.autograd.Function):
         ctx.was_training = plan.bn is not None and plan.training
         ctx.has = (weight is not None, bias is not None, scalar_bias is not None,
                    gate_bias is not None)
+        ctx.sizes = [0 if t is None else t.numel() for t in (weight, bias, scalar_bias, gate_bias)]
         ctx.save_for_backward(x, shift, scale, add, rstd, pre_bias)
         return y
 
@@ -204,29 +199,17 @@ class _BnAct(torch.autograd.Function):
                 act.get("gated_first"), act.get("gated_dim"), plan.act_scalar, plan.act_gate)
         dy = dy.contiguous()
         n = x.size(0)
-        has_w, has_b, has_sb, has_gb = ctx.has
-        need_sums = ctx.was_training or any(ctx.has)
-        d_weight = d_bias = d_sb = d_gb = None
-        dz_mean = coef = None
-        if need_sums:
+        d_weight = d_bias = d_sb = d_gb = dz_mean = coef = None
+        if ctx.was_training or any(ctx.has):
             sums = _ext.bnact_backward_sums(x, dy, *args)
-            col_b, col_a = sums[0], sums[1]
-            if has_sb:
-                d_sb = col_b[:plan.n_scalar_act].clone()
-            if has_gb:
-                d_gb = col_b[plan.c_out:plan.c_out + plan.n_gates].clone()
-            if plan.bn is not None:
-                field_of = plan.bn["field_of_long"]
-                scalar_cols = plan.bn["scalar_cols"]
-                field_a = torch.zeros_like(rstd).index_add_(0, field_of, col_a)
-                if has_b:
-                    d_bias = col_b[scalar_cols].clone()
-                if has_w:
-                    d_weight = rstd * field_a
-                if ctx.was_training:
-                    dz_mean = torch.zeros_like(col_b)
-                    dz_mean[scalar_cols] = col_b[scalar_cols] / n
-                    coef = scale * (rstd * rstd * field_a)[field_of] / n
+            if n > 0:
+                d_weight, d_bias, d_sb, d_gb, dz_mean, coef = _ext.bnact_backward_coef(
+                    n, sums, plan.bn, scale, rstd, plan.n_scalar_act, plan.c_out, plan.n_gates,
+                    ctx.has, ctx.was_training)
+            else:  # no rows: zero gradients (batch statistics of no rows are refused before)
+                d_weight, d_bias, d_sb, d_gb = [
+                    sums.new_zeros(size) if has else None
+                    for has, size in zip(ctx.has, ctx.sizes)]
         dx = _ext.bnact_backward(x, dy, *args, dz_mean, coef) if ctx.needs_input_grad[0] else None
         return dx, d_weight, d_bias, d_sb, d_gb, None
 
@@ -259,4 +242,4 @@ def canonical(Rs):
 
 
 def to_device(tables, device):
-    return {k: v.to(device) for k, v in tables.items()}
+    return {k: v.to(device) if torch.is_tensor(v) else v for k, v in tables.items()}

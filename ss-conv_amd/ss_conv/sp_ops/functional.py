@@ -87,6 +87,8 @@ class SparseConvRulebookFunction(Function):
         ctx.save_for_backward(pairs, num, features, filters)
         ctx.ssc_meta = getattr(pairs, "_ssc_meta", None)
         ctx.subm = bool(subm)
+        # no zero gradients for the index outputs: the pairs' alone are as large as the pairs
+        ctx.set_materialize_grads(False)
         if subm:  # the outputs are the inputs: nothing new to return
             ctx.mark_non_differentiable(pairs, num)
             return out, None, pairs, num
@@ -96,6 +98,8 @@ class SparseConvRulebookFunction(Function):
     @staticmethod
     def backward(ctx, grad_output, *unused):
         indice_pairs, indice_pair_num, features, filters = ctx.saved_tensors
+        if grad_output is None:
+            return (torch.zeros_like(features), torch.zeros_like(filters)) + (None,) * 9
         if ctx.ssc_meta is not None and getattr(indice_pairs, "_ssc_meta", None) is None:
             indice_pairs._ssc_meta = ctx.ssc_meta
         input_bp, filters_bp = ops.indice_conv_backward(

@@ -2597,3 +2597,46 @@ def test_voxel2point_one_call_equals_the_separate_steps(oracle, device):
                                             st.features.detach().cpu().numpy(), [grid] * 3,
                                             vp.cpu().numpy(), vi.cpu().numpy(), **kw)
             assert rel_l2(out.detach().cpu().numpy(), want) < 1e-6
+
+
+@pytest.mark.parametrize("fields,gates,rows", [
+    ([(1, 0)], 0, 1), ([(0, 0), (3, 2)], 3, 7), ([(5, 0), (2, 1), (0, 2), (1, 4)], 3, 1000),
+    ([(256, 0)], 0, 65), ([(100, 0), (51, 1), (1, 1)], 52, 33), ([(8, 0), (218, 3)], 2, 5)])
+@pytest.mark.parametrize("norm", [True, False])
+def test_bnact_column_constants(fields, gates, rows, norm, device):
+    """The activations' bias vector, and what the backward pass derives from its column sums,
+    against the formulas in float64 (a field adds at most nine float32 terms: 9 * 2^-24)."""
+    from ss_conv import _ext, bnact
+    gen = torch.Generator(device=device).manual_seed(rows)
+    rand = lambda *n: torch.randn(*n, device=device, generator=gen)  # noqa: E731
+    layout = bnact.to_device(bnact.field_layout(fields + [(gates, 0)]), device)
+    of, c, n_fields = layout["field_of"].long(), layout["field_of"].numel(), layout["field_dim"].numel()
+    c_out, n_act = c - gates, fields[0][0]
+    sb, gb = rand(n_act), rand(gates)
+    for s, g in ((sb, gb), (None, gb), (sb, None)):
+        want = torch.zeros(c, device=device)
+        if s is not None:
+            want[:n_act] = s
+        if g is not None:
+            want[c_out:] = g
+        assert torch.equal(_ext.bnact_pre_bias(c, s, g, n_act, c_out, gates, want.device), want)
+    sums, scale, rstd = rand(2, c), rand(c), rand(n_fields).abs() + 0.1
+    for training in ((False, True) if norm else (False,)):
+        want_all = (norm, norm, True, True)
+        got = _ext.bnact_backward_coef(rows, sums, layout if norm else None, scale, rstd, n_act,
+                                       c_out, gates, want_all, training)
+        dz, r = sums[0].double(), rstd.double()
+        a = torch.zeros(n_fields, dtype=torch.float64, device=device).index_add_(0, of, sums[1].double())
+        size = torch.zeros_like(a).index_add_(0, of, sums[1].double().abs())  # of what is added up
+        scalar = layout["scalar_idx"] >= 0
+        want = (r * a, dz[scalar], dz[:n_act], dz[c_out:], torch.where(scalar, dz / rows, 0.),
+                scale.double() * (r * r * a)[of] / rows)
+        bound = (r * size, None, None, None, dz.abs() / rows,
+                 (scale.double().abs() * (r * r * size)[of] / rows))
+        asked = (norm, norm, True, True, norm and training, norm and training)
+        for x, y, b, yes in zip(got, want, bound, asked):
+            assert (x is not None) == yes
+            if yes and b is None:
+                assert torch.equal(x.double(), y)
+            elif yes:
+                assert ((x.double() - y).abs() <= 16 * 2.0 ** -24 * b).all()
