@@ -563,6 +563,13 @@ int ssc_segment_max_f32(const float *feats, const int32_t *offsets, float *out,
                         int32_t *out_idx /* [b,c] */, int32_t n_segments, int32_t channels,
                         ssc_stream_t stream);
 
+/* offsets[b] = number of rows of indices [n,4] (batch, x, y, z) with batch index in [0, b), for
+ * b = 0 .. n_batch (SparseTensor.get_offsets, ss_conv/sp_ops/tensor.py:60-69).
+ * state[2 * n_batch + 3]: the offsets, then a word that is not 0 if a batch index is negative
+ * (the offsets then miss those rows), then scratch. */
+int ssc_batch_offsets(const int32_t *indices, int64_t n, int32_t n_batch, int32_t *state,
+                      ssc_stream_t stream);
+
 /* Backward of the segment pools -- replaces global_avgpool_bp / global_maxpool_bp
  * (src/pool/global_avgpool_cuda_kernel.cu:44-62, global_maxpool_cuda_kernel.cu:45-60).
  * in_grad [n_rows, channels] is written completely (rows outside every segment get 0). */

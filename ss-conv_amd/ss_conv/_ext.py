@@ -121,6 +121,7 @@ _SIGNATURES = {
     "ssc_pool_avg_f16": (ctypes.c_int, [_vp, _i32, _vp, _i64, _vp, _i32, _vp, _vp, _i64, _vp,
                                         _sz, _vp]),
     "ssc_summary_rf": (ctypes.c_int, [_vp, _i64, _vp, _i32, _vp, _i64, _vp, _sz, _vp]),
+    "ssc_batch_offsets": (ctypes.c_int, [_vp, _i64, _i32, _vp, _vp]),
     "ssc_segment_avg_f32": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _vp]),
     "ssc_segment_max_f32": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "ssc_voxel_coords": (ctypes.c_int, [_vp, _vp, _i64, ctypes.POINTER(ctypes.c_float),
@@ -1173,6 +1174,19 @@ def _seg_args(feats, offsets, out, n_seg, c):
         raise RuntimeError("segment pooling needs contiguous tensors")
     if offsets.numel() != n_seg + 1 or feats.size(1) != c or out.numel() != n_seg * c:
         raise RuntimeError("segment pooling: inconsistent sizes")
+
+
+def batch_offsets(indices, batch_size):
+    """int32 [batch_size + 1] row offsets of the batch elements from int32 rows [N, 4] of
+    (batch, x, y, z); a negative batch index is refused, which costs the host a wait."""
+    _need_gpu(indices)
+    indices = indices.contiguous()
+    state = torch.empty(2 * batch_size + 3, dtype=torch.int32, device=indices.device)
+    _check(_lib.ssc_batch_offsets(_ptr(indices), indices.size(0), batch_size, state.data_ptr(),
+                                  _stream(indices)))
+    if indices.size(0) > 0 and state[batch_size + 1].item() != 0:
+        raise RuntimeError("the batch indices of a sparse tensor must not be negative")
+    return state[:batch_size + 1]
 
 
 def global_avgpool_fp(feats, offsets, out, out_maxidx, n_proposal, c):

@@ -2640,3 +2640,24 @@ def test_bnact_column_constants(fields, gates, rows, norm, device):
                 assert torch.equal(x.double(), y)
             elif yes:
                 assert ((x.double() - y).abs() <= 16 * 2.0 ** -24 * b).all()
+
+
+@pytest.mark.parametrize("n", [0, 1, 63, 64, 1023, 1025, 300001])
+@pytest.mark.parametrize("batch", [1, 3, 257, 4096, 4097])
+def test_batch_offsets(n, batch, device):
+    """Row offsets of the batch elements, rows in order or not, elements without rows and rows
+    of elements beyond the batch among them; a negative batch index is refused."""
+    from ss_conv.sp_ops.tensor import SparseTensor
+    rng = np.random.default_rng([n, batch])
+    b = rng.integers(0, batch + 2, n).astype(np.int32)
+    for ids in (np.sort(b), b):
+        idx = np.stack([ids] + [rng.integers(-5, 9, n).astype(np.int32)] * 3, 1)
+        t = torch.from_numpy(idx).to(device)
+        got = SparseTensor(torch.zeros(n, 1, device=device), t, [8] * 3, batch).get_offsets()
+        want = np.concatenate([[0], np.cumsum(np.bincount(ids, minlength=batch)[:batch])])
+        assert got.dtype == torch.int32 and got.is_contiguous()
+        assert np.array_equal(got.cpu().numpy(), want)
+    if n > 0:
+        t[n // 2, 0] = -1
+        with pytest.raises(RuntimeError):
+            SparseTensor(torch.zeros(n, 1, device=device), t, [8] * 3, batch).get_offsets()
