@@ -2661,3 +2661,26 @@ def test_batch_offsets(n, batch, device):
         t[n // 2, 0] = -1
         with pytest.raises(RuntimeError):
             SparseTensor(torch.zeros(n, 1, device=device), t, [8] * 3, batch).get_offsets()
+
+
+@pytest.mark.parametrize("c", [1, 3, 4, 37, 64, 68])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_three_interpolate_channel_counts(c, shift, device):
+    """Rows of four channels at a time and one at a time (channel counts that are no multiple
+    of four, rows that are not 16-byte aligned): the same three products and two sums."""
+    from ss_conv import _ext
+    rng = np.random.default_rng(c)
+    m, n = 50, 257
+    feats = rng.standard_normal((m, c)).astype(np.float32)
+    idx = rng.integers(0, m, (n, 3)).astype(np.int32)
+    w = rng.random((n, 3)).astype(np.float32)
+    room = torch.empty(m * c + 1, device=device)
+    f = room[shift:shift + m * c].view(m, c)
+    f.copy_(torch.from_numpy(feats))
+    i, wt = torch.from_numpy(idx).to(device), torch.from_numpy(w).to(device)
+    room_out = torch.empty(n * c + 1, device=device)
+    out = room_out[shift:shift + n * c].view(n, c)
+    _ext._check(_ext._lib.ssc_three_interp_f32(c, m, n, f.data_ptr(), i.data_ptr(), wt.data_ptr(),
+                                               out.data_ptr(), _ext._stream(f)))
+    p = [w[:, j:j + 1] * feats[idx[:, j]] for j in range(3)]
+    assert np.array_equal(out.cpu().numpy(), (p[0] + p[1]) + p[2])
