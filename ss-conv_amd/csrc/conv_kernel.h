@@ -945,12 +945,18 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
       const char *ab = a_base + par * kStage * kRowB;
       const int base_cur = w_soff0 + cur.cc * kFragB;
       const int base_next = w_soff0 + next.cc * kFragB;
-      Frag a[2][NF];
+      // Staged rows in registers: of this block and the next.  Half: of all four blocks, read
+      // as the stage begins -- two MFMAs are shorter than an LDS read takes, so a block's rows
+      // read during the block before would be waited for in every block instead of once.
+      constexpr int kARing = kHalf ? 4 : 2;
+      Frag a[kARing][NF];
       auto load_a = [&](int m, int q, Frag (&av)[NF]) {
         av[q] = *reinterpret_cast<const Frag *>(ab + m * 16 * kRowB + q * 64);
       };
 #pragma unroll
-      for (int q = 0; q < NF; ++q) load_a(0, q, a[0]);
+      for (int m = 0; m < (kHalf ? 4 : 1); ++m)
+#pragma unroll
+        for (int q = 0; q < NF; ++q) load_a(m, q, a[m]);
       // gaps of the pieces of a block (see above); with fewer than 16 MFMAs they move
       // closer together, in the same order
       // half: two MFMAs a block, so the pieces sit behind the first or the second
@@ -981,7 +987,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
           __builtin_amdgcn_sched_barrier(0);
           if constexpr (kHalf) {
             d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8v, w[slot][i]),
-                                                       __builtin_bit_cast(half8v, a[m & 1][i]), d,
+                                                       __builtin_bit_cast(half8v, a[m][i]), d,
                                                        0, 0, 0);
           } else {
             const int q = i >> 2, j = i & 3;
@@ -1005,7 +1011,9 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
 #pragma unroll
           for (int qq = 1; qq < NF; ++qq)
             if (i == kGapW[qq]) fetch_w(soff, tslot, qq);
-          if (m < 3) {
+          if constexpr (kHalf) {
+            // (read already)
+          } else if (m < 3) {
 #pragma unroll
             for (int qq = 0; qq < NF; ++qq)
               if (i == kGapA[qq]) load_a(m + 1, qq, a[(m + 1) & 1]);
