@@ -947,7 +947,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
       const int base_next = w_soff0 + next.cc * kFragB;
       // Staged rows in registers: of this block and the next.  Half: of all four blocks, read
       // as the stage begins -- two MFMAs are shorter than an LDS read takes, so a block's rows
-      // read during the block before would be waited for in every block instead of once.
+      // read during the block before would be waited for in every block instead of once
+      // (64 -> 128 channels, 1.54 M pairs: 166 -> 160 us).
       constexpr int kARing = kHalf ? 4 : 2;
       Frag a[kARing][NF];
       auto load_a = [&](int m, int q, Frag (&av)[NF]) {
