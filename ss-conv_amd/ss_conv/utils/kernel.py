@@ -125,41 +125,48 @@ def orthogonal_(tensor, gain=1):
 class _Combine(torch.autograd.Function):
     """dense[k, (j,v,b), (i,u,a)] = sum_n weight_ij[u,v,n] * basis_ij[n,a,b,k] in one native
     launch; the gradient with respect to the weights is the same contraction against the
-    fixed basis, one launch as well."""
+    fixed basis, one launch as well.  Derivatives of any order use the tables of the forward
+    pass: the module may have dropped its own since (load_state_dict, .to())."""
 
     @staticmethod
     def forward(ctx, weight, module, pack):
-        basis, chan_out, chan_in, blocks = module._tables[:4]
         ctx.module = module
         ctx.tables = module._tables
-        out = _ext.kernel_combine(weight.detach().float().contiguous(), basis, chan_out, chan_in,
-                                  blocks, len(module.multiplicities_in), module.size ** 3,
-                                  module.n_in, module.n_out, packed=bool(pack),
-                                  defer=pack == "defer")
+        out = _synthesise(weight, module, ctx.tables, packed=bool(pack), defer=pack == "defer")
         if pack:
             out, module.packed = out
         return out
 
     @staticmethod
     def backward(ctx, grad):  # grad: [K, Cin, Cout]
-        return _CombineGrad.apply(grad, ctx.module, ctx.tables), None, None
+        return _Contract.apply(grad, ctx.module, ctx.tables, True), None, None
 
 
-class _CombineGrad(torch.autograd.Function):
-    """The gradient above as a function of its own: linear in `grad`, so that it can be
-    differentiated again, by the synthesis itself."""
+def _synthesise(weight, module, tables, **pack):
+    basis, chan_out, chan_in, blocks = tables[:4]
+    return _ext.kernel_combine(weight.detach().float().contiguous(), basis, chan_out, chan_in,
+                               blocks, len(module.multiplicities_in), module.size ** 3,
+                               module.n_in, module.n_out, **pack)
+
+
+class _Contract(torch.autograd.Function):
+    """Either contraction on its own, linear in `x`: the weight gradient of a dense kernel's
+    gradient (to_weight), or the dense kernel of a weight vector.  Each is the derivative of
+    the other."""
 
     @staticmethod
-    def forward(ctx, grad, module, tables):
+    def forward(ctx, x, module, tables, to_weight):
+        ctx.of = (module, tables, not to_weight)
+        if not to_weight:
+            return _synthesise(x, module, tables)
         basis, chan_out, chan_in, blocks, _, first_out, first_in = tables
-        ctx.module = module
-        return _ext.kernel_combine_backward(grad, basis, chan_out, chan_in, blocks, first_out,
+        return _ext.kernel_combine_backward(x, basis, chan_out, chan_in, blocks, first_out,
                                             first_in, len(module.multiplicities_in),
                                             module.size ** 3, module.weight.numel())
 
     @staticmethod
     def backward(ctx, grad):
-        return _Combine.apply(grad, ctx.module, False), None, None
+        return _Contract.apply(grad, *ctx.of), None, None, None
 
 
 class SE3Kernel(torch.nn.Module):

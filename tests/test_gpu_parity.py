@@ -1046,6 +1046,23 @@ def test_kernel_combine_gradient(device, rs_in, rs_out, size):
     assert torch.equal(again, ker.combination(t))
 
 
+def test_kernel_combine_second_gradient_of_an_older_graph(device):
+    """The synthesis is differentiated twice over a graph whose module has dropped its device
+    tables since (load_state_dict, .to()): the derivative is that of the same basis."""
+    from ss_conv.utils.kernel import SE3Kernel
+    torch.manual_seed(2)
+    ker = SE3Kernel([(2, 0), (1, 1)], [(1, 0), (2, 1)], 3).to(device)
+    dense = ker()
+    d_out = torch.randn(dense.shape, device=device, requires_grad=True)
+    grad, = torch.autograd.grad(dense, ker.weight, d_out, create_graph=True)
+    t = torch.randn_like(ker.weight)
+    want = ker.combination(t)
+    for forget in (lambda: ker.load_state_dict(ker.state_dict()), lambda: ker.to(device)):
+        forget()
+        again, = torch.autograd.grad(grad, d_out, t, retain_graph=True)
+        assert torch.equal(again, want)
+
+
 def test_convolution_layer_end_to_end(oracle, device):
     """Point2Voxel -> Convolution against the oracle pipeline and against dense conv3d."""
     import torch.nn.functional as F
