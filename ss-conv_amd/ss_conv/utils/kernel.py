@@ -139,7 +139,7 @@ class _Combine(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):  # grad: [K, Cin, Cout]
-        return _Contract.apply(grad, ctx.module, ctx.tables, True), None, None
+        return _Contract.apply(grad, ctx.module, _Tables(ctx.tables), True), None, None
 
 
 def _synthesise(weight, module, tables, **pack):
@@ -152,21 +152,44 @@ def _synthesise(weight, module, tables, **pack):
 class _Contract(torch.autograd.Function):
     """Either contraction on its own, linear in `x`: the weight gradient of a dense kernel's
     gradient (to_weight), or the dense kernel of a weight vector.  Each is the derivative of
-    the other."""
+    the other; tangents (forward mode) and vmapped gradients go through the same launch, one
+    per tangent or element."""
 
     @staticmethod
-    def forward(ctx, x, module, tables, to_weight):
-        ctx.of = (module, tables, not to_weight)
+    def forward(x, module, tables, to_weight):
         if not to_weight:
-            return _synthesise(x, module, tables)
-        basis, chan_out, chan_in, blocks, _, first_out, first_in = tables
+            return _synthesise(x, module, tables.of)
+        basis, chan_out, chan_in, blocks, _, first_out, first_in = tables.of
         return _ext.kernel_combine_backward(x, basis, chan_out, chan_in, blocks, first_out,
                                             first_in, len(module.multiplicities_in),
                                             module.size ** 3, module.weight.numel())
 
     @staticmethod
+    def setup_context(ctx, inputs, output):
+        ctx.rest = inputs[1:]
+
+    @staticmethod
     def backward(ctx, grad):
-        return _Contract.apply(grad, *ctx.of), None, None, None
+        module, tables, to_weight = ctx.rest
+        return _Contract.apply(grad, module, tables, not to_weight), None, None, None
+
+    @staticmethod
+    def jvp(ctx, tangent, *_):
+        return _Contract.apply(tangent, *ctx.rest)
+
+    @staticmethod
+    def vmap(info, in_dims, x, *rest):
+        rows = x.movedim(in_dims[0], 0).unbind(0)
+        return torch.stack([_Contract.apply(row, *rest) for row in rows]), 0
+
+
+class _Tables:
+    """A module's device tables as one opaque argument (a tuple of tensors would be taken
+    apart by the function transforms)."""
+    __slots__ = ("of",)
+
+    def __init__(self, of):
+        self.of = of
 
 
 class SE3Kernel(torch.nn.Module):

@@ -1063,6 +1063,36 @@ def test_kernel_combine_second_gradient_of_an_older_graph(device):
         assert torch.equal(again, want)
 
 
+def test_kernel_combine_gradient_under_transforms(device):
+    """The weight gradient is linear in the arriving one: its forward-mode derivative along t
+    is the weight gradient of t, it maps over stacked gradients, and torch.func.grad goes
+    through it in either order with them."""
+    import torch.autograd.forward_ad as fw
+    from ss_conv.utils.kernel import SE3Kernel
+    torch.manual_seed(3)
+    ker = SE3Kernel([(2, 0), (1, 1)], [(1, 0), (2, 1)], 3).to(device)
+    dense = ker()
+    d = torch.randn((3,) + dense.shape, device=device)
+
+    def grad(g, again=False):
+        with torch.enable_grad():
+            return torch.autograd.grad(dense, ker.weight, g, retain_graph=True, create_graph=again)[0]
+
+    want = torch.stack([grad(g) for g in d])
+    with fw.dual_level():
+        value, tangent = fw.unpack_dual(grad(fw.make_dual(d[0], d[1])))
+    assert torch.equal(value, want[0]) and torch.equal(tangent, want[1])
+    value, tangent = torch.func.jvp(grad, (d[0],), (d[1],))
+    assert torch.equal(value, want[0]) and torch.equal(tangent, want[1])
+    assert torch.equal(torch.func.vmap(grad)(d), want)
+    assert torch.equal(torch.func.vmap(grad, in_dims=2)(d.movedim(0, 2)), want)
+    # d(|grad|^2)/dg = 2 * synthesis of grad
+    twice = torch.stack([ker.combination(2 * w.detach()).detach() for w in want])
+    square = lambda g: grad(g, True).pow(2).sum()  # noqa: E731
+    assert torch.allclose(torch.func.grad(square)(d[0]), twice[0], rtol=1e-6, atol=1e-6)
+    assert torch.allclose(torch.func.vmap(torch.func.grad(square))(d), twice, rtol=1e-6, atol=1e-6)
+
+
 def test_convolution_layer_end_to_end(oracle, device):
     """Point2Voxel -> Convolution against the oracle pipeline and against dense conv3d."""
     import torch.nn.functional as F
