@@ -53,6 +53,12 @@ class BatchNorm(nn.Module):
         self._layout_cpu = bnact.field_layout(Rs)
         self._layout_dev = {}
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        if "n_scalar" not in self._layout_cpu:  # (modules saved whole before it was kept)
+            self._layout_cpu = bnact.field_layout(self.Rs)
+            self._layout_dev = {}
+
     def layout(self, device):
         """Channel tables of the kernels on `device`."""
         key = str(device)

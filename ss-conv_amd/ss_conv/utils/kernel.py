@@ -250,6 +250,12 @@ class SE3Kernel(torch.nn.Module):
         self._tables = None
         return super()._load_from_state_dict(*args, **kwargs)
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        # (modules saved whole before the gradient had tables of its own)
+        if self._tables is not None and len(self._tables) != 7:
+            self._tables = None
+
     def _apply(self, fn, *args, **kwargs):
         self._tables = None
         return super()._apply(fn, *args, **kwargs)

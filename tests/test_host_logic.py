@@ -470,3 +470,28 @@ def test_epilogue_layout_keeps_gates_with_their_columns():
     assert lay["src"].tolist() == list(range(10)) + [-1, -1]
     assert lay["mode"].tolist() == [0] * 10 + [3, 3]
     assert lay["gate_run"].tolist() == [12, 0]
+
+
+def test_modules_saved_whole_before_their_tables_grew():
+    """A module that was pickled with the device tables of an earlier form (five tables of the
+    kernel synthesis; channel tables without the number of scalar columns) builds them anew;
+    tables of the present form come along."""
+    import pickle
+    from ss_conv import bnact
+    from ss_conv.batchnorm import BatchNorm
+    from ss_conv.utils.kernel import SE3Kernel
+    rs = [(2, 0), (1, 1)]
+    ker = SE3Kernel(rs, rs, 3)
+    ker._tables = tuple(range(5))
+    assert pickle.loads(pickle.dumps(ker))._tables is None
+    ker._tables = tuple(range(7))
+    assert pickle.loads(pickle.dumps(ker))._tables == tuple(range(7))
+    norm = BatchNorm(rs)
+    of_now = norm.layout("cpu")
+    again = pickle.loads(pickle.dumps(norm))
+    assert set(again._layout_dev["cpu"]) == set(of_now)
+    for tables in (norm._layout_cpu, of_now):
+        del tables["n_scalar"]
+    again = pickle.loads(pickle.dumps(norm))
+    assert again._layout_cpu["n_scalar"] == again.layout("cpu")["n_scalar"] == 2
+    assert set(again.layout("cpu")) == set(bnact.field_layout(rs))
