@@ -1,4 +1,6 @@
 """Sparse tensor container (reference: ss_conv/sp_ops/tensor.py:22-69)."""
+import operator
+
 import numpy as np
 import torch
 
@@ -59,9 +61,15 @@ class SparseTensor(object):
         """int32 [batch_size + 1] row offsets of the batch elements (rows must be
         grouped by batch index in ascending order)."""
         idx = self.indices
-        if (idx.is_cuda and idx.dtype == torch.int32 and idx.dim() == 2 and idx.size(1) == 4
-                and idx.device == self.features.device and 1 <= int(self.batch_size) < 2 ** 20):
-            return _ext.batch_offsets(idx, int(self.batch_size))
+        try:  # whole numbers only; what is none is left for bincount to refuse
+            batch = 0 if isinstance(self.batch_size, bool) else operator.index(self.batch_size)
+        except TypeError:
+            batch = 0
+        # (a native launch goes to the current device, tensor operations to the tensors' own)
+        if (1 <= batch < 2 ** 20 and idx.is_cuda and idx.dtype == torch.int32 and idx.dim() == 2
+                and idx.size(1) == 4 and idx.device == self.features.device
+                and idx.device.index == torch.cuda.current_device()):
+            return _ext.batch_offsets(idx, batch)
         counts = torch.bincount(self.indices[:, 0].long(), minlength=self.batch_size)
         offsets = torch.zeros(self.batch_size + 1, dtype=torch.int32, device=self.features.device)
         offsets[1:] = torch.cumsum(counts[:self.batch_size], 0).to(torch.int32)

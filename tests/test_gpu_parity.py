@@ -2710,6 +2710,24 @@ def test_batch_offsets(n, batch, device):
             SparseTensor(torch.zeros(n, 1, device=device), t, [8] * 3, batch).get_offsets()
 
 
+def test_batch_offsets_only_for_what_bincount_takes(device, monkeypatch):
+    """Batch sizes that are no whole numbers are refused as by torch.bincount, those that only
+    count as one (0-d tensors, numpy scalars) are not; tensors of another device than the
+    current one go to tensor operations, which follow their tensors."""
+    from ss_conv import _ext
+    from ss_conv.sp_ops.tensor import SparseTensor
+    idx = torch.tensor([[0, 1, 2, 3], [2, 1, 1, 1], [2, 0, 0, 0]], dtype=torch.int32, device=device)
+    offsets = lambda b: SparseTensor(idx.float(), idx, [8] * 3, b).get_offsets()  # noqa: E731
+    for refused in (3.0, np.float32(3), True, None, "3"):
+        with pytest.raises(TypeError):
+            offsets(refused)
+    for whole in (3, np.int64(3), torch.tensor(3), np.array(3)):
+        assert offsets(whole).tolist() == [0, 1, 1, 3]
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: idx.device.index + 1)
+    monkeypatch.setattr(_ext, "batch_offsets", None)
+    assert offsets(3).tolist() == [0, 1, 1, 3]
+
+
 @pytest.mark.parametrize("c", [1, 3, 4, 37, 64, 68])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_three_interpolate_channel_counts(c, shift, device):
