@@ -13,6 +13,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 namespace ssc {
@@ -313,16 +314,21 @@ static int static_table(int32_t **table) {
 // look at `bad` (a negative index, which the caller refuses): 1.6 MB of indices for 100 k rows.
 // As tensor operations (minimum, maximum, histogram, scan, each with its buffers, and two
 // values copied to the host) it took 12 launches, 230 us of a training step.
+// With more elements than bins (SUMS false) the rows are counted in memory, and the counts
+// are added up by the two kernels below: one block alone would wait for n_batch / 128 loads
+// one behind the other.  Host's wait included, rows in order: 1000 rows of 20 k elements 39 us
+// (one block 71, tensor operations 81), of 2^20 elements 45 us (1970, 83); 3 M rows of 4097
+// elements 80 us (113, 127).
 constexpr int kCountBins = 4096;
+template <bool SUMS>
 __global__ void __launch_bounds__(256)
     batch_offsets_kernel(const int32_t *__restrict__ indices, int64_t n, int n_batch,
                          int32_t *__restrict__ state) {
-  __shared__ int32_t bins[kCountBins];
+  __shared__ int32_t bins[SUMS ? kCountBins : 1];
   __shared__ int32_t part[256];
   __shared__ bool last;
   int32_t *bad = state + n_batch + 1, *done = bad + 1, *counts = done + 1;
-  const bool in_lds = n_batch <= kCountBins;
-  if (in_lds) {
+  if constexpr (SUMS) {
     for (int b = threadIdx.x; b < n_batch; b += 256) bins[b] = 0;
     __syncthreads();
   }
@@ -336,13 +342,12 @@ __global__ void __launch_bounds__(256)
     if (b < 0)
       atomicOr(bad, 1);
     else if (b < n_batch && add != 0)
-      atomicAdd(in_lds ? &bins[b] : &counts[b], add);
+      atomicAdd(SUMS ? &bins[b] : &counts[b], add);
   }
-  if (in_lds) {
-    __syncthreads();
-    for (int b = threadIdx.x; b < n_batch; b += 256)
-      if (bins[b] != 0) atomicAdd(&counts[b], bins[b]);
-  }
+  if constexpr (!SUMS) return;
+  __syncthreads();
+  for (int b = threadIdx.x; b < n_batch; b += 256)
+    if (bins[b] != 0) atomicAdd(&counts[b], bins[b]);
   __threadfence();
   __syncthreads();
   if (threadIdx.x == 0) last = atomicAdd(done, 1) == (int)gridDim.x - 1;
@@ -361,6 +366,40 @@ __global__ void __launch_bounds__(256)
   for (int b = lo; b < hi; ++b) {
     at += __hip_atomic_load(&counts[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     state[b + 1] = at;
+  }
+}
+
+// Many elements: a block turns kCountBins counts into the sums up to each of them, in place;
+// then each block adds the last sums of the blocks before it and writes its offsets.
+constexpr int kCountRun = kCountBins / kScanThreads;
+__global__ void __launch_bounds__(kScanThreads)
+    batch_count_sums_kernel(int n_batch, int32_t *__restrict__ counts) {
+  __shared__ int lds[kScanThreads / 64 + 1];
+  const int lo = blockIdx.x * kCountBins + (int)threadIdx.x * kCountRun;
+  int c[kCountRun], v = 0, all;
+#pragma unroll
+  for (int i = 0; i < kCountRun; ++i) {
+    c[i] = lo + i < n_batch ? counts[lo + i] : 0;
+    v += c[i];
+  }
+  int at = block_exclusive_scan(v, lds, &all);
+#pragma unroll
+  for (int i = 0; i < kCountRun; ++i) {
+    at += c[i];
+    if (lo + i < n_batch) counts[lo + i] = at;
+  }
+}
+__global__ void __launch_bounds__(kScanThreads)
+    batch_sums_offsets_kernel(int n_batch, const int32_t *__restrict__ sums,
+                              int32_t *__restrict__ offsets) {
+  __shared__ int lds[kScanThreads / 64 + 1];
+  int before = 0, base;
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += kScanThreads)
+    before += sums[(b + 1) * kCountBins - 1];
+  block_exclusive_scan(before, lds, &base);
+  for (int i = threadIdx.x; i < kCountBins; i += kScanThreads) {
+    const int b = blockIdx.x * kCountBins + i;
+    if (b < n_batch) offsets[b + 1] = base + sums[b];
   }
 }
 
@@ -500,11 +539,27 @@ int ssc_batch_offsets(const int32_t *indices, int64_t n, int32_t n_batch, int32_
   SSC_CHECK(state && (indices || n == 0), SSC_EINVAL, "NULL pointer argument");
   int rc = fill_i32(state, 2 * (int64_t)n_batch + 3, 0, (hipStream_t)stream);
   if (rc != SSC_OK || n == 0) return rc;
-  // four rows to a thread, one block per CU at most
-  const int64_t blocks = ceil_div(n, 1024) < 256 ? ceil_div(n, 1024) : 256;
-  hipLaunchKernelGGL(batch_offsets_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                     (hipStream_t)stream, indices, n, n_batch, state);
+  // four rows to a thread, one block per CU at most where every block adds its bins to the
+  // counts; without bins the blocks wait for their own atomics only
+  const bool few = n_batch <= kCountBins;
+  const int64_t blocks = std::min(ceil_div(n, 1024), (int64_t)(few ? 256 : 2048));
+  if (few)
+    hipLaunchKernelGGL(batch_offsets_kernel<true>, dim3((unsigned)blocks), dim3(256), 0,
+                       (hipStream_t)stream, indices, n, n_batch, state);
+  else
+    hipLaunchKernelGGL(batch_offsets_kernel<false>, dim3((unsigned)blocks), dim3(256), 0,
+                       (hipStream_t)stream, indices, n, n_batch, state);
   SSC_LAUNCH_CHECK("batch_offsets");
+  if (!few) {
+    int32_t *counts = state + n_batch + 3;
+    const unsigned groups = (unsigned)ceil_div(n_batch, kCountBins);
+    hipLaunchKernelGGL(batch_count_sums_kernel, dim3(groups), dim3(kScanThreads), 0,
+                       (hipStream_t)stream, n_batch, counts);
+    SSC_LAUNCH_CHECK("batch_count_sums");
+    hipLaunchKernelGGL(batch_sums_offsets_kernel, dim3(groups), dim3(kScanThreads), 0,
+                       (hipStream_t)stream, n_batch, (const int32_t *)counts, state);
+    SSC_LAUNCH_CHECK("batch_sums_offsets");
+  }
   return SSC_OK;
 }
 

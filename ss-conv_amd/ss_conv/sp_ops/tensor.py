@@ -65,6 +65,8 @@ class SparseTensor(object):
             batch = 0 if isinstance(self.batch_size, bool) else operator.index(self.batch_size)
         except TypeError:
             batch = 0
+        # The native form is the faster one as far as it was measured (1000 to 3 M rows in order:
+        # 30 to 184 us where tensor operations take 80 to 252).
         # (a native launch goes to the current device, tensor operations to the tensors' own)
         if (1 <= batch < 2 ** 20 and idx.is_cuda and idx.dtype == torch.int32 and idx.dim() == 2
                 and idx.size(1) == 4 and idx.device == self.features.device

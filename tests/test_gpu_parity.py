@@ -2710,6 +2710,23 @@ def test_batch_offsets(n, batch, device):
             SparseTensor(torch.zeros(n, 1, device=device), t, [8] * 3, batch).get_offsets()
 
 
+@pytest.mark.parametrize("batch", [4097, 8192, 8193, 300000, 2 ** 20 - 1, 2 ** 20])
+@pytest.mark.parametrize("n", [1, 2500, 700001])
+def test_batch_offsets_of_many_elements(batch, n, device):
+    """More elements than the counting kernel has bins for (its counts then lie in memory and
+    are added up in groups of 4096), rows in order and not, in a few elements and in all."""
+    from ss_conv.sp_ops.tensor import SparseTensor
+    rng = np.random.default_rng([n, batch])
+    for ids in (rng.integers(0, batch, n), np.sort(rng.integers(0, batch + 2, n)),
+                rng.choice([0, 4095, 4096, batch - 1, batch], n)):
+        idx = torch.zeros(n, 4, dtype=torch.int32)
+        idx[:, 0] = torch.from_numpy(ids)
+        idx = idx.to(device)
+        got = SparseTensor(torch.zeros(n, 1, device=device), idx, [8] * 3, batch).get_offsets()
+        want = np.concatenate([[0], np.cumsum(np.bincount(ids, minlength=batch)[:batch])])
+        assert np.array_equal(got.cpu().numpy(), want)
+
+
 def test_batch_offsets_only_for_what_bincount_takes(device, monkeypatch):
     """Batch sizes that are no whole numbers are refused as by torch.bincount, those that only
     count as one (0-d tensors, numpy scalars) are not; tensors of another device than the
