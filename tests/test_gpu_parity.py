@@ -1046,6 +1046,48 @@ def test_kernel_combine_gradient(device, rs_in, rs_out, size):
     assert torch.equal(again, ker.combination(t))
 
 
+@pytest.mark.parametrize("rs_in,rs_out,size,empty", [
+    ([(3, 0), (2, 1)], [(2, 0), (1, 3), (2, 1)], 1, 4),        # blocks without a basis function
+    ([(3, 0)], [(2, 0), (1, 3), (1, 4)], 3, 1),
+    ([(5, 1), (2, 3)], [(3, 2), (2, 3)], 5, 0),                # more than 8 functions, kernel 5
+    # tiles of 16 output by 4 input fields: one offset, few of them, many
+    ([(120, 0)], [(121, 0)], 1, 0),
+    ([(150, 0), (2, 1)], [(100, 0), (1, 3), (2, 1)], 1, 4),
+    ([(33, 0), (90, 1)], [(119, 0), (1, 2)], 2, 0),
+    ([(130, 0)], [(113, 0)], 3, 0),
+    ([(17, 0), (30, 1), (14, 2)], [(40, 0), (21, 1), (9, 2)], 7, 0),
+    ([(70000, 0)], [(1, 0)], 1, 0),                            # more fields than a grid has rows
+])
+def test_kernel_combine_gradient_of_many_fields(device, rs_in, rs_out, size, empty):
+    """The weight gradient at the edges of its two kernels, against the contraction in float64."""
+    from ss_conv.utils.kernel import SE3Kernel
+    torch.manual_seed(1)
+    ker = SE3Kernel(rs_in, rs_out, size).to(device)
+    dense = ker()
+    d_out = torch.randn(dense.shape, device=device)
+    got, = torch.autograd.grad(dense, ker.weight, d_out)
+    d_dense = d_out.cpu().reshape(ker.n_out, ker.n_in, size ** 3).permute(2, 1, 0).double()
+    want, scale, none = [], [], 0
+    o_off = 0
+    for i, (mi, di) in enumerate(zip(ker.multiplicities_out, ker.dims_out)):
+        i_off = 0
+        for j, (mj, dj) in enumerate(zip(ker.multiplicities_in, ker.dims_in)):
+            kij = getattr(ker, "kernel_%d_%d" % (i, j))
+            none += kij is None
+            if kij is not None:
+                basis = kij.cpu().double().reshape(-1, di, dj, size ** 3)
+                g = d_dense[:, i_off:i_off + mj * dj, o_off:o_off + mi * di]
+                g = g.reshape(size ** 3, mj, dj, mi, di)
+                for dst, x, b in ((want, g, basis), (scale, g.abs(), basis.abs())):
+                    dst.append(torch.einsum("kvbua,nabk->uvn", x, b).reshape(-1))
+            i_off += mj * dj
+        o_off += mi * di
+    assert none == empty
+    want, scale = torch.cat(want), torch.cat(scale)
+    # fp32: a thread adds at most 25 products, then the sums of at most 22 offsets; then 8 levels
+    assert bool(((got.cpu().double() - want).abs() <= 80 * 2.0 ** -24 * scale + 1e-30).all())
+
+
 def test_kernel_combine_second_gradient_of_an_older_graph(device):
     """The synthesis is differentiated twice over a graph whose module has dropped its device
     tables since (load_state_dict, .to()): the derivative is that of the same basis."""
