@@ -11,6 +11,7 @@ import math
 
 import numpy as np
 import torch
+from torch.autograd.forward_ad import unpack_dual
 
 from ss_conv import _ext
 from .SO3 import irr_repr, real_sh_np, basis_transformation_Q_J
@@ -122,6 +123,10 @@ def orthogonal_(tensor, gain=1):
 
 
 # ---- kernel module ----------------------------------------------------------------------
+# whether a torch.func transform is running (taken to be where torch does not tell)
+_transforms_active = getattr(torch._C, "_are_functorch_transforms_active", lambda: True)
+
+
 class _Combine(torch.autograd.Function):
     """dense[k, (j,v,b), (i,u,a)] = sum_n weight_ij[u,v,n] * basis_ij[n,a,b,k] in one native
     launch; the gradient with respect to the weights is the same contraction against the
@@ -139,7 +144,12 @@ class _Combine(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):  # grad: [K, Cin, Cout]
-        return _Contract.apply(grad, ctx.module, _Tables(ctx.tables), True), None, None
+        tables = _Tables(ctx.tables)
+        # a node of its own costs 20 us of host time: only where something can see it
+        if (torch.is_grad_enabled() or _transforms_active()
+                or unpack_dual(grad).tangent is not None):
+            return _Contract.apply(grad, ctx.module, tables, True), None, None
+        return _Contract.forward(grad, ctx.module, tables, True), None, None
 
 
 def _synthesise(weight, module, tables, **pack):
