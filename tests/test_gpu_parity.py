@@ -2808,3 +2808,31 @@ def test_three_interpolate_channel_counts(c, shift, device):
                                                out.data_ptr(), _ext._stream(f)))
     p = [w[:, j:j + 1] * feats[idx[:, j]] for j in range(3)]
     assert np.array_equal(out.cpu().numpy(), (p[0] + p[1]) + p[2])
+
+
+def test_convolution_whose_output_gets_no_gradient(device, monkeypatch):
+    """A function behind the layer that returns no gradient for its features: the layer's
+    features and weights get zeros, as from a gradient of zeros, without its kernels."""
+    from ss_conv.convolution import Convolution
+    from ss_conv.sp_ops import ops
+    from ss_conv.sp_ops.tensor import SparseTensor
+
+    class Cut(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    monkeypatch.setattr(ops, "indice_conv_backward", None)
+    idx = torch.tensor([[0, 1, 2, 3], [0, 1, 2, 4], [1, 5, 5, 5]], dtype=torch.int32, device=device)
+    for dtype in (torch.float32, torch.float16):
+        for subm in (False, True):
+            conv = Convolution([(2, 0), (1, 1)], [(3, 0), (1, 1)], 3, padding=1, subm=subm).to(device)
+            feats = torch.randn(3, 5, device=device).to(dtype).requires_grad_(True)
+            y = conv(SparseTensor(feats, idx, [8] * 3, 2))
+            (Cut.apply(y.features).float().sum() + 0 * feats.float().sum()).backward()
+            for got, of in ((feats.grad, feats), (conv.kernel.weight.grad, conv.kernel.weight)):
+                assert got.dtype == of.dtype and got.shape == of.shape and not got.any()
