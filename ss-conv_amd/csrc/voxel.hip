@@ -459,9 +459,10 @@ constexpr int kGridNnAll = 1 << 30;  // counter value that means "redo every que
 // Nothing found is (inf, 0); a distance that is not a number is above it and never kept.
 // Kept lists then need no branches -- an insertion is three compare-and-exchange steps, the
 // three smallest of two sorted lists three minima and a sort -- where comparing distances
-// and rows by hand diverged in every step: the search is bound by its instructions (43 MB of
-// tables and results for 131 k points, 6 us of memory time; 62 -> 46 us there, 56 with the
-// first two shells together alone).
+// and rows by hand diverged in every step: the search is bound by its instructions (for
+// 131 k points in 8 grids of 128^3 it reads and writes 11 MB: table and prefix 2.1 each, queries
+// 2.1, results 4.7, 1.4 us at 8 TB/s; 62 -> 46 us there, 56 with the first two shells together
+// alone).
 typedef unsigned long long Cand;
 constexpr Cand kNoCand = 0x7F800000ull << 32;
 __device__ __forceinline__ Cand cand_of(float d, int k) {
@@ -536,7 +537,8 @@ __global__ void __launch_bounds__(256)
   }
   // The first round takes the query's own cell and the shell around it together: a cell holds
   // one voxel, so no query can have its three after the cell alone, and a round costs its
-  // exchange between the lanes (18 shuffles, nine insertions) however little it finds.
+  // exchange between the lanes (three times three 64-bit candidates shuffled and merged)
+  // however little it finds.
   for (int r = 1; r <= kGridNnMaxShell; ++r) {
     if (__all(settled)) break;  // (every query of the wave: the same decision in all lanes)
     Best3Cand cur = none;

@@ -1007,7 +1007,8 @@ def test_kernel_combine_matches_einsum(oracle, device):
 
 @pytest.mark.parametrize("rs_in,rs_out,size", [
     ([(1, 0)], [(1, 0)], 1),                             # one element, one basis function
-    ([(3, 0)], [(2, 0), (1, 1), (1, 2)], 3),             # blocks without a basis function
+    ([(3, 0)], [(2, 0), (1, 1), (1, 2)], 3),             # one or two functions to a block
+    ([(3, 0), (2, 1)], [(2, 0), (1, 3), (2, 1)], 1),     # four blocks without a basis function
     ([(1, 0), (2, 2)], [(2, 1), (1, 4)], 5),             # > 256 elements of a basis function
     ([(16, 0), (16, 1)], [(5, 0), (3, 1), (2, 3)], 3),
     ([(2, 3)], [(1, 4), (3, 3)], 7),                     # more than 8 basis functions
