@@ -55,7 +55,8 @@ class BatchNorm(nn.Module):
 
     def __setstate__(self, state):
         super().__setstate__(state)
-        if "n_scalar" not in self._layout_cpu:  # (modules saved whole before it was kept)
+        # (modules saved whole before the tables were kept, or that number with them)
+        if "n_scalar" not in self.__dict__.get("_layout_cpu", ()):
             self._layout_cpu = bnact.field_layout(self.Rs)
             self._layout_dev = {}
 

@@ -263,7 +263,7 @@ class SE3Kernel(torch.nn.Module):
     def __setstate__(self, state):
         super().__setstate__(state)
         # (modules saved whole before the gradient had tables of its own)
-        if self._tables is not None and len(self._tables) != 7:
+        if len(self.__dict__.get("_tables") or ()) != 7:
             self._tables = None
 
     def _apply(self, fn, *args, **kwargs):

@@ -495,3 +495,6 @@ def test_modules_saved_whole_before_their_tables_grew():
     again = pickle.loads(pickle.dumps(norm))
     assert again._layout_cpu["n_scalar"] == again.layout("cpu")["n_scalar"] == 2
     assert set(again.layout("cpu")) == set(bnact.field_layout(rs))
+    del ker._tables, norm._layout_cpu, norm._layout_dev  # files from before there were any
+    assert pickle.loads(pickle.dumps(ker))._tables is None
+    assert set(pickle.loads(pickle.dumps(norm)).layout("cpu")) == set(bnact.field_layout(rs))
