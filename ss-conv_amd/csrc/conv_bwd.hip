@@ -4,19 +4,22 @@
 // of every offset).  The input gradient needs no kernel of its own: it is the forward
 // convolution of dout with the pairs swapped and the filters transposed.
 //
-// Per offset this is a tall-skinny product [Cin x P_k] * [P_k x Cout] on fp32 MFMA.
-// A workgroup owns one offset, one 64 x 64 tile of (ci, co) and one contiguous range
-// of the offset's pairs; it gathers 64 pairs at a time into LDS, rows as they lie in
-// memory.  Which pair sits in which k slot of an MFMA does not matter for the sum, and
-// neither does which channel a lane stands for, as long as the result is stored
-// accordingly: lane l of channel block j stands for channel 4l + j, so one 16-byte LDS
-// read of a gathered row hands a lane its operands for all four channel blocks, and
-// two such reads (features, output gradient) feed 16 MFMAs.  Every wave keeps the
-// whole 64 x 64 tile (16 independent accumulators) over a quarter of the pairs; the
-// four waves' tiles are added in wave order at the end, and the ranges of pairs by a
-// second kernel in ascending order: the result does not depend on timing, no atomics.
+// Per offset this is a tall-skinny product [Cin x P_k] * [P_k x Cout].  A workgroup owns one
+// offset, one 64 x 64 tile of (ci, co) and one contiguous range of the offset's pairs.  Which
+// pair sits in which k slot of a matrix instruction does not matter for the sum, and neither
+// does which channel a lane stands for, as long as the result is stored accordingly: lane l of
+// channel block j stands for channel 4l + j, so one 16-byte read of a row hands a lane its
+// operands for all four channel blocks.  Every wave keeps the whole 64 x 64 tile (16
+// independent accumulators) over a quarter of the pairs; the four waves' tiles are added in
+// wave order at the end, and the ranges of pairs by a second kernel in ascending order: the
+// result does not depend on timing, no atomics.
+//
+// conv_bwd_filter_parts_kernel takes rows of whole quads of channels with 31-bit offsets;
+// conv_bwd_filter_kernel takes the rest: it gathers 64 pairs at a time into LDS, rows as they
+// lie in memory, and multiplies with float instructions.
 #include "ssc_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace ssc {
@@ -204,6 +207,265 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
   }
 }
 
+// The same tile of the same sums on the bfloat16 matrix instructions, sixteen times the rate of
+// the float ones: every element is cut into bfloat16 parts that add up to it (three for a
+// float, two for a half), and of the products of parts those are taken that a float sum still
+// sees -- six of nine for floats, the ones left out are below 2^-24 of the product; all four
+// for halves.
+//
+// No LDS in the loop: a wave takes 32 pairs at a time, lane (l16, g) reads four channels
+// (4 l16 .. + 3) of the rows of pairs 8 g .. 8 g + 7, and as the parts of two neighbouring
+// pairs' elements are packed into a word, the words of a channel are the operand of one
+// matrix step as it is wanted (eight pairs to a lane): the transposition costs nothing.
+//
+// What bounds it, 64 -> 128 channels, 1.54M pairs, floats: matrix instructions (96 of 16
+// cycles a wave and step) keep the matrix cores busy for a third of the time, 350 vector
+// instructions (7 for every two elements that are cut) and the gathers take about as long
+// each, and with the two waves a SIMD that 252 registers leave the three overlap in part only
+// (a wave waits for rows in 37 % of its time).  Finer interleaving of loads and matrix
+// instructions, or waiting for L1 only, gained less than 5 %.  Measured, both kernels with
+// their reduction, before -> now:
+//                                   float            half
+//    64 -> 128, 1.54M pairs    282 -> 197 us    274 -> 138 us
+//   128 -> 128, 0.78M pairs    278 -> 186       278 -> 140
+//    64 -> 64,  137k pairs      34 -> 22.5       34 -> 20
+//    32 -> 32,  44k pairs       19.3 -> 17       20 -> 15.7
+//    64 -> 152, stride 2, 52k   31 -> 27         31 -> 25
+//    64 -> 128, 5^3, 480k      100 -> 74        100 -> 54
+// Error of the gradient against 64 bits, relative, in the order of the rows above, floats:
+// 5.1e-7 -> 2.9e-7, 5.1e-7 -> 2.2e-7, 2.1e-7 -> 1.2e-7, 1.9e-7 -> 0.9e-7, 1.5e-7 -> 0.9e-7,
+// 2.8e-7 -> 1.2e-7.
+//
+// Infinities and NaN have no parts, and the parts of numbers below 2^-110 are cut off at
+// 2^-134: a workgroup that ends with a sum that is not finite, or is not zero and below
+// 2^-80, works its range out again with float instructions (lane (l16, g)'s row 8 g + j is
+// k slot g of step j).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef int int4v __attribute__((ext_vector_type(4)));
+constexpr int kBwStep = 32;                      // pairs of a wave's step
+constexpr unsigned kBwOutside = 0x7FFFF000u;     // byte offset beyond either matrix
+constexpr unsigned kBwColOutside = 0x80000000u;  // (added to any row's offset: outside as well)
+
+template <typename IO>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    conv_bwd_filter_parts_kernel(const IO *__restrict__ feats, int n_in, int cin,
+                                 const IO *__restrict__ dout, int n_out, int cout,
+                                 const int32_t *__restrict__ pairs, int64_t pair_stride,
+                                 const int32_t *__restrict__ pair_num, int plane_in, int n_split,
+                                 int n_co_tiles, int K, int n_tiles, float *__restrict__ partial) {
+  constexpr int P = sizeof(IO) == 4 ? 3 : 2;
+  constexpr unsigned kEB = sizeof(IO);
+  typedef decltype(buf_quad(__amdgpu_buffer_rsrc_t(), 0u, (const IO *)nullptr)) Quad;
+  __shared__ __align__(16) float tile[4 * kBwTile * kBwTile];
+  __shared__ int odd_s;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  // Consecutive workgroups land on different XCDs, one L2 each.  The pairs of an offset ascend
+  // in their output row, so the offsets' ranges of one number touch the same rows of the
+  // output gradient: the ranges, each with all offsets and tiles, go to the XCDs in runs.
+  const int total = gridDim.x, xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int item = xcd * (total >> 3) + min(xcd, total & 7) + slot;
+  const int s = item / (K * n_tiles), kt = item - s * (K * n_tiles);
+  const int k = kt / n_tiles, t_co = kt % n_tiles;
+  const int ci0 = (t_co / n_co_tiles) * kBwTile;
+  const int co0 = (t_co % n_co_tiles) * kBwTile;
+  const int n = pair_num[k];
+  int len = (n + n_split - 1) / n_split;
+  len = (len + 4 * kBwStep - 1) / (4 * kBwStep) * (4 * kBwStep);
+  const int p_begin = min(s * len, n), p_end = min(p_begin + len, n);
+  const int32_t *rows_in = pairs + ((int64_t)k * 2 + plane_in) * pair_stride;
+  const int32_t *rows_out = pairs + ((int64_t)k * 2 + (1 - plane_in)) * pair_stride;
+  const unsigned row_f = (unsigned)cin * kEB, row_d = (unsigned)cout * kEB;
+  // (pairs behind the range read as 0)
+  const __amdgpu_buffer_rsrc_t rs_i =
+      __builtin_amdgcn_make_buffer_rsrc((void *)rows_in, 0, p_end * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_o =
+      __builtin_amdgcn_make_buffer_rsrc((void *)rows_out, 0, p_end * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_f =
+      __builtin_amdgcn_make_buffer_rsrc((void *)feats, 0, (int)(n_in * row_f), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_d =
+      __builtin_amdgcn_make_buffer_rsrc((void *)dout, 0, (int)(n_out * row_d), 0x00020000);
+  const unsigned col_f = ci0 + 4 * l16 < cin ? (unsigned)(ci0 + 4 * l16) * kEB : kBwColOutside;
+  const unsigned col_d = co0 + 4 * l16 < cout ? (unsigned)(co0 + 4 * l16) * kEB : kBwColOutside;
+  if (tid == 0) odd_s = 0;
+
+  // acc[jm][jn]: D[ci0 + 4*(4g + r) + jm][co0 + 4*l16 + jn] in component r
+  float4v acc[4][4];
+  int idx_f[8], idx_d[8];
+  Quad qf[8], qd[8];
+  auto load_idx = [&](const __amdgpu_buffer_rsrc_t &rs, int p0, int (&idx)[8])
+      __attribute__((always_inline)) {
+    if (p0 + kBwStep > p_end) {  // (no load that lies partly behind the range)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        idx[j] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (p0 + 8 * g + j) * 4, 0, 0);
+      return;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int4v v = __builtin_bit_cast(
+          int4v, __builtin_amdgcn_raw_buffer_load_b128(rs, (p0 + 8 * g + 4 * h) * 4, 0, 0));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) idx[4 * h + j] = v[j];
+    }
+  };
+  // Byte offsets of a step's rows (row `rows` is behind the matrix' end: it reads as zeros).
+  auto offsets = [&](int p0, int rows, int (&idx)[8], unsigned row, unsigned col,
+                     unsigned (&off)[8]) __attribute__((always_inline)) {
+    if (p0 + kBwStep > p_end)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) idx[j] = p0 + 8 * g + j < p_end ? idx[j] : rows;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) off[j] = __umul24((unsigned)idx[j], row) + col;
+  };
+  // A step's rows, and after them the row numbers of the wave's next step: a wait for those
+  // is not a wait for loads of rows that are younger.
+  auto load_f = [&](int p0) __attribute__((always_inline)) {
+    unsigned off[8];
+    offsets(p0, n_in, idx_f, row_f, col_f, off);
+    load_idx(rs_i, p0 + 4 * kBwStep, idx_f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) qf[j] = buf_quad(rs_f, off[j], feats);
+  };
+  auto load_d = [&](int p0) __attribute__((always_inline)) {
+    unsigned off[8];
+    offsets(p0, n_out, idx_d, row_d, col_d, off);
+    load_idx(rs_o, p0 + 4 * kBwStep, idx_d);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) qd[j] = buf_quad(rs_d, off[j], dout);
+  };
+  // the waves take the range's steps in turn
+  const int p_wave = p_begin + wave * kBwStep;
+  auto run = [&](auto multiply) __attribute__((always_inline)) {
+#pragma unroll
+    for (int jm = 0; jm < 4; ++jm)
+#pragma unroll
+      for (int jn = 0; jn < 4; ++jn) acc[jm][jn] = float4v{0.f, 0.f, 0.f, 0.f};
+    if (p_wave < p_end) {
+      load_idx(rs_i, p_wave, idx_f);
+      load_idx(rs_o, p_wave, idx_d);
+      load_f(p_wave);
+      load_d(p_wave);
+    }
+    for (int p0 = p_wave; p0 < p_end; p0 += 4 * kBwStep) multiply(p0);
+  };
+  // (the pairs (-1, 0) and (0, -1) in registers: as literals they would be packed into one
+  // half of the operand, which the instruction reads twice)
+  uint32_t minus0 = 0x0000BF80u, minus1 = 0xBF800000u;
+  asm volatile("" : "+s"(minus0), "+s"(minus1));
+  const bf16x2 m0 = __builtin_bit_cast(bf16x2, minus0), m1 = __builtin_bit_cast(bf16x2, minus1);
+  // the operand of channel block c, part by part
+  auto cut = [&](const Quad (&q)[8], int c, int4v (&part)[P]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float u = widen4(q[2 * j])[c], v = widen4(q[2 * j + 1])[c];
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const bf16x2 b = __builtin_convertvector(float2v{u, v}, bf16x2);
+        part[p][j] = __builtin_bit_cast(int, b);
+        if (p + 1 < P) {
+          u = __builtin_amdgcn_fdot2_f32_bf16(b, m0, u, false);
+          v = __builtin_amdgcn_fdot2_f32_bf16(b, m1, v, false);
+        }
+      }
+    }
+  };
+  run([&](int p0) __attribute__((always_inline)) {
+    int4v pf[4][P];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) cut(qf, c, pf[c]);
+    load_f(p0 + 4 * kBwStep);  // (in flight during the multiplications)
+    // (a channel block of the gradient is cut among the multiplications of the one before; the
+    // barriers keep the compiler from cutting them all at once, for which there are no registers)
+    int4v pds[2][P];
+    cut(qd, 0, pds[0]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int jn = 0; jn < 4; ++jn) {
+      const int4v (&pd)[P] = pds[jn & 1];
+      if (jn < 3) cut(qd, jn + 1, pds[(jn + 1) & 1]);
+      if (jn == 2) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_d(p0 + 4 * kBwStep);
+      }
+      // A step's products are summed by themselves, the smallest first (of floats only those
+      // of parts a + b <= 2), and added to the sum of the steps before: one rounding at its
+      // size a step, not one an instruction.
+      float4v t[4];
+#pragma unroll
+      for (int jm = 0; jm < 4; ++jm) t[jm] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int a = P - 1; a >= 0; --a)
+#pragma unroll
+        for (int b = P - 1; b >= 0; --b) {
+          if (a + b > 2) continue;
+#pragma unroll
+          for (int jm = 0; jm < 4; ++jm)
+            t[jm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pf[jm][a]),
+                                                            __builtin_bit_cast(bf16x8, pd[b]), t[jm],
+                                                            0, 0, 0);
+        }
+#pragma unroll
+      for (int jm = 0; jm < 4; ++jm) acc[jm][jn] += t[jm];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  });
+  __syncthreads();  // (odd_s is cleared)
+  {
+    bool odd = false;
+#pragma unroll
+    for (int jm = 0; jm < 4; ++jm)
+#pragma unroll
+      for (int jn = 0; jn < 4; ++jn)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float m = fabsf(acc[jm][jn][r]);
+          odd = odd || !(m <= 3.402823466e38f) || (m < 8.271806125530277e-25f && m != 0.f);
+        }
+    if (odd) odd_s = 1;
+  }
+  __syncthreads();
+  if (odd_s != 0) {
+    run([&](int p0) __attribute__((always_inline)) {
+      float4v xf[8], xd[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        xf[j] = widen4(qf[j]);
+        xd[j] = widen4(qd[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int jm = 0; jm < 4; ++jm)
+#pragma unroll
+          for (int jn = 0; jn < 4; ++jn)
+            acc[jm][jn] = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[j][jm], xd[j][jn], acc[jm][jn], 0, 0, 0);
+      load_f(p0 + 4 * kBwStep);
+      load_d(p0 + 4 * kBwStep);
+    });
+  }
+  // The four waves' tiles in wave order, then the tile out (as above).
+#pragma unroll
+  for (int jm = 0; jm < 4; ++jm)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<float4v *>(tile + wave * kBwTile * kBwTile + (4 * (4 * g + r) + jm) * kBwTile + 4 * l16) =
+          float4v{acc[jm][0][r], acc[jm][1][r], acc[jm][2][r], acc[jm][3][r]};
+  __syncthreads();
+  float *dst = partial + ((int64_t)s * K + k) * cin * cout;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int ci = ci0 + 4 * (4 * wave + i) + g, co = co0 + 4 * l16;
+    const float4v *t = reinterpret_cast<const float4v *>(tile + (4 * (4 * wave + i) + g) * kBwTile + 4 * l16);
+    constexpr int kQ = kBwTile * kBwTile / 4;
+    const float4v v = ((t[0] + t[kQ]) + t[2 * kQ]) + t[3 * kQ];
+    if (ci < cin && co < cout) *reinterpret_cast<float4v *>(dst + (int64_t)ci * cout + co) = v;
+  }
+}
+
 // out[e] = partial[0][e] + partial[1][e] + ... in that order; out may have any strides.
 template <typename IO>
 __global__ void __launch_bounds__(256)
@@ -213,23 +475,48 @@ __global__ void __launch_bounds__(256)
   const int64_t per = (int64_t)K * cin * cout;
   if (e >= per) return;
   float v = partial[e];
+#pragma unroll 8
   for (int s = 1; s < n_split; ++s) v += partial[(int64_t)s * per + e];
-  const int co = (int)(e % cout);
-  const int64_t r = e / cout;
-  const int ci = (int)(r % cin);
-  const int k = (int)(r / cin);
+  int co, ci, k;
+  if (per <= 0xFFFFFFFFll) {
+    const unsigned r = (unsigned)e / (unsigned)cout;
+    co = (int)((unsigned)e - r * cout);
+    k = (int)(r / (unsigned)cin);
+    ci = (int)(r - (unsigned)k * cin);
+  } else {
+    const int64_t r = e / cout;
+    co = (int)(e % cout);
+    ci = (int)(r % cin);
+    k = (int)(r / cin);
+  }
   out[k * os_k + ci * os_ci + co * os_co] = (IO)v;
 }
 
 static int bwd_split(int K, int c_in, int c_out, int64_t pair_stride) {
-  // as many workgroups as the chip holds at once (4 per CU on 256 CUs) when the tiles
-  // alone are fewer, but ranges of at least 8 chunks
+  // four workgroups a CU (256 CUs) when the tiles alone are fewer, but ranges of at least 8 chunks
   const int64_t tiles = ceil_div(c_in, kBwTile) * ceil_div(c_out, kBwTile) * K;
   int64_t s = 1024 / tiles;
   const int64_t max_s = ceil_div(pair_stride > 0 ? pair_stride : 1, 8 * kBwChunk);
   if (s > max_s) s = max_s;
   if (s < 1) s = 1;
   return (int)s;
+}
+
+// Ranges of conv_bwd_filter_parts_kernel, at most bwd_split's: as many workgroups as the chip
+// holds at once (two a CU), twice as many where their ranges are still 2048 pairs long (they
+// end less unevenly: 128 -> 128 channels, 29k pairs an offset, 206 us with 4 ranges, 200 with
+// 9), and no range below 384 pairs, as a range costs a tile written and read: 64 -> 152 with
+// 1.9k pairs an offset 36 us with 12 ranges, 25 with 6; 64 -> 128 at 5^3 and 3.8k 84 us with 4
+// and 75 with 2; 32 -> 32 with 1.6k 18.9 us with 4 and 21.1 with 2.
+// An offset has no more pairs than either side has rows.
+static int bwd_parts_split(int K, int c_in, int c_out, int64_t pair_stride, int64_t n_in,
+                           int64_t n_out) {
+  const int64_t tiles = ceil_div(c_in, kBwTile) * ceil_div(c_out, kBwTile) * K;
+  const int64_t longest = std::min(pair_stride, std::min(n_in, n_out));
+  const int64_t once = std::max<int64_t>(1, (512 + tiles / 2) / tiles);
+  int64_t s = std::min(std::max(longest / 2048, once), 2 * once);
+  s = std::min(s, ceil_div(longest, 384));
+  return (int)std::min<int64_t>(s, bwd_split(K, c_in, c_out, pair_stride));
 }
 
 }  // namespace ssc
@@ -278,19 +565,31 @@ static int conv_bwd_filter(const IO *features, int64_t n_in, int32_t c_in, const
   const size_t need = ssc_conv_bwd_filter_workspace_bytes(K, c_in, c_out, pair_stride);
   SSC_CHECK(workspace_bytes >= need, SSC_EWORKSPACE,
             "conv backward workspace too small: %zu < %zu", workspace_bytes, need);
-  const int n_split = bwd_split(K, c_in, c_out, pair_stride);
   const int n_ci_tiles = (int)ceil_div(c_in, kBwTile), n_co_tiles = (int)ceil_div(c_out, kBwTile);
   SSC_CHECK((int64_t)n_ci_tiles * n_co_tiles <= 65535, SSC_ERUNTIME, "too many channel tiles");
   float *partial = static_cast<float *>(workspace);
   // features are gathered through the plane the forward pass gathered them through
   const int plane_in = inverse ? 1 : 0;
-  const dim3 grid((unsigned)n_split, (unsigned)K, (unsigned)(n_ci_tiles * n_co_tiles));
   const uint64_t feat_bytes = (uint64_t)n_in * c_in * sizeof(IO);
   const uint64_t dout_bytes = (uint64_t)n_out * c_out * sizeof(IO);
   // the largest byte offset must stay below the marker that stands for "outside"
   const bool buf = (c_in & 3) == 0 && (c_out & 3) == 0 && feat_bytes <= 0xFFFFF000u &&
                    dout_bytes <= 0xFFFFF000u;
-  if (buf)
+  // (row numbers and row sizes of 24 bits, offsets of 31: the index arithmetic of the kernel;
+  // within it that kernel is the faster one at every size measured, from 1.1 to 2 times)
+  const bool parts = (c_in & 3) == 0 && (c_out & 3) == 0 && feat_bytes <= kBwOutside &&
+                     dout_bytes <= kBwOutside && n_in < (1 << 24) && n_out < (1 << 24) &&
+                     (uint64_t)c_in * sizeof(IO) < (1u << 24) && (uint64_t)c_out * sizeof(IO) < (1u << 24) &&
+                     pair_stride < (1 << 28);
+  const int n_split = parts ? bwd_parts_split(K, c_in, c_out, pair_stride, n_in, n_out)
+                            : bwd_split(K, c_in, c_out, pair_stride);
+  const dim3 grid((unsigned)n_split, (unsigned)K, (unsigned)(n_ci_tiles * n_co_tiles));
+  if (parts)
+    hipLaunchKernelGGL(conv_bwd_filter_parts_kernel<IO>, dim3(grid.x * grid.y * grid.z), dim3(256), 0,
+                       s, features, (int)n_in, c_in, out_grad, (int)n_out, c_out,
+                       pairs, pair_stride, pair_num, plane_in, n_split, n_co_tiles, K,
+                       n_ci_tiles * n_co_tiles, partial);
+  else if (buf)
     hipLaunchKernelGGL((conv_bwd_filter_kernel<IO, true>), grid, dim3(256), 0, s, features, c_in,
                        (unsigned)feat_bytes, out_grad, c_out, (unsigned)dout_bytes, pairs,
                        pair_stride, pair_num, plane_in, n_split, n_co_tiles, partial);

@@ -2837,3 +2837,61 @@ def test_convolution_whose_output_gets_no_gradient(device, monkeypatch):
             (Cut.apply(y.features).float().sum() + 0 * feats.float().sum()).backward()
             for got, of in ((feats.grad, feats), (conv.kernel.weight.grad, conv.kernel.weight)):
                 assert got.dtype == of.dtype and got.shape == of.shape and not got.any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("cin,cout,inverse,what", [
+    (4, 4, 0, "plain"), (60, 64, 1, "plain"), (64, 68, 0, "plain"), (132, 128, 1, "plain"),
+    (68, 8, 0, "huge"), (8, 68, 0, "tiny"), (64, 64, 0, "not finite"), (5, 64, 0, "plain")])
+def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
+    """Offsets of pairs on both sides of a wave's and a workgroup's step, none at all and several
+    ranges; tiles that the channels fill in part; elements that have no bfloat16 parts (near the
+    largest float, below 2^-80, infinities and NaN).  Against 64 bits, element by element: a
+    float sum of m products is off by no more than m units of 2^-24 of the sum of their sizes,
+    8 more for the additions of waves and ranges; a half result is the rounded float one."""
+    from ss_conv import _ext
+    counts = [0, 1, 31, 32, 33, 127, 128, 129, 160, 1000, 5001]
+    K, stride, n_in, n_out = len(counts), max(counts) + 2, 5003, 5007
+    gen = torch.Generator().manual_seed(cin * 131 + cout)
+    f = torch.randn((n_in, cin), generator=gen)
+    d = torch.randn((n_out, cout), generator=gen)
+    pairs = torch.full((K, 2, stride), -1, dtype=torch.int32)
+    for k, m in enumerate(counts):
+        pairs[k, inverse, :m] = torch.randperm(n_in, generator=gen)[:m].int()
+        pairs[k, 1 - inverse, :m] = torch.arange(m, dtype=torch.int32) + 6
+    if what in ("huge", "tiny") and dtype == torch.float32:
+        f, d = (f * 2.0 ** 125, d * 2.0 ** -90) if what == "huge" else (f * 2.0 ** -50, d * 2.0 ** -45)
+    f, d = f.to(dtype), d.to(dtype)
+    if what == "huge" and dtype == torch.float32:
+        f[::7, ::3] = torch.finfo(torch.float32).max
+    if what == "not finite":
+        f[pairs[3, inverse, 5].long(), 7], d[20, 9] = float("inf"), float("nan")
+        f[pairs[8, inverse, 150].long(), 63] = float("-inf")
+    num = torch.tensor(counts, dtype=torch.int32, device=device)
+    p_dev, f_dev, d_dev = pairs.to(device), f.to(device), d.to(device)
+
+    def run(entry, a, b):
+        out = torch.empty((K, cin, cout), dtype=a.dtype, device=device)
+        need = _ext._lib.ssc_conv_bwd_filter_workspace_bytes(K, cin, cout, stride)
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        _ext._check(entry(a.data_ptr(), n_in, cin, b.data_ptr(), n_out, cout, p_dev.data_ptr(),
+                          stride, num.data_ptr(), K, inverse, out.data_ptr(), cin * cout, cout, 1,
+                          ws.data_ptr(), need, _ext._stream(a)))
+        return out.cpu()
+
+    if dtype == torch.float32:
+        got = run(_ext._lib.ssc_conv_bwd_filter_f32, f_dev, d_dev)
+    else:
+        half = run(_ext._lib.ssc_conv_bwd_filter_f16, f_dev, d_dev)
+        got = run(_ext._lib.ssc_conv_bwd_filter_f32, f_dev.float(), d_dev.float())
+        assert torch.equal(half.nan_to_num(7.0), got.half().nan_to_num(7.0))
+        assert torch.equal(half.isnan(), got.isnan())
+    for k, m in enumerate(counts):
+        a = f[pairs[k, inverse, :m].long()].double()
+        b = d[pairs[k, 1 - inverse, :m].long()].double()
+        ref, size = a.t() @ b, a.abs().t() @ b.abs()
+        finite = ref.isfinite()
+        assert torch.equal(got[k].isnan(), ref.isnan()), k
+        assert torch.equal(got[k][ref.isinf()].double(), ref[ref.isinf()]), k
+        off = (got[k].double() - ref).abs()
+        assert bool((off <= (m + 8) * 2.0 ** -24 * size)[finite].all()), (k, m)
