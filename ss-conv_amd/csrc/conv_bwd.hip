@@ -14,9 +14,9 @@
 // wave order at the end, and the ranges of pairs by a second kernel in ascending order: the
 // result does not depend on timing, no atomics.
 //
-// conv_bwd_filter_parts_kernel takes rows of whole quads of channels with 31-bit offsets;
-// conv_bwd_filter_kernel takes the rest: it gathers 64 pairs at a time into LDS, rows as they
-// lie in memory, and multiplies with float instructions.
+// conv_bwd_filter_parts_kernel takes output rows of four channels or more and matrices with
+// 31-bit offsets; conv_bwd_filter_kernel takes the rest: it gathers 64 pairs at a time into LDS,
+// rows as they lie in memory, and multiplies with float instructions.
 #include "ssc_common.h"
 
 #include <algorithm>
@@ -52,6 +52,19 @@ __device__ __forceinline__ int2v buf_quad(__amdgpu_buffer_rsrc_t r, unsigned off
                                           const _Float16 *) {
   return __builtin_bit_cast(int2v, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
 }
+
+// one channel, as loaded, and an element of a quad or of one channel as a float
+__device__ __forceinline__ float buf_one(__amdgpu_buffer_rsrc_t r, unsigned off, const float *) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
+}
+__device__ __forceinline__ _Float16 buf_one(__amdgpu_buffer_rsrc_t r, unsigned off,
+                                            const _Float16 *) {
+  return __builtin_bit_cast(_Float16, __builtin_amdgcn_raw_buffer_load_b16(r, (int)off, 0, 0));
+}
+__device__ __forceinline__ float element(const float4v &v, int c) { return v[c]; }
+__device__ __forceinline__ float element(const int2v &v, int c) { return widen4(v)[c]; }
+__device__ __forceinline__ float element(float v, int) { return v; }
+__device__ __forceinline__ float element(_Float16 v, int) { return (float)v; }
 
 // Four channels of row `row`, zero outside the matrix.
 template <typename IO>
@@ -226,13 +239,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
 // instructions, or waiting for L1 only, gained less than 5 %.  Measured, both kernels with
 // their reduction, before -> now:
 //                                   float            half
-//    64 -> 128, 1.54M pairs    282 -> 197 us    274 -> 138 us
-//   128 -> 128, 0.78M pairs    278 -> 186       278 -> 140
-//    64 -> 64,  137k pairs      34 -> 22.5       34 -> 20
-//    32 -> 32,  44k pairs       19.3 -> 17       20 -> 15.7
-//    64 -> 152, stride 2, 52k   31 -> 27         31 -> 25
-//    64 -> 128, 5^3, 480k      100 -> 74        100 -> 54
-// Error of the gradient against 64 bits, relative, in the order of the rows above, floats:
+//    64 -> 128, 1.54M pairs    282 -> 192 us    274 -> 135 us
+//   128 -> 128, 0.78M pairs    278 -> 183       278 -> 135
+//    64 -> 64,  137k pairs      34 -> 21         34 -> 19
+//    32 -> 32,  44k pairs       19.3 -> 15.7     20 -> 13.8
+//    64 -> 152, stride 2, 52k   31 -> 24         31 -> 21
+//    64 -> 128, 5^3, 480k      100 -> 72        100 -> 52
+//    30 -> 31,  205k            48 -> 20         66 -> 17
+//    64 -> 64,  10k             17 -> 11         18 -> 11
+//    32 -> 32,  stride 2, 5.5k  13.6 -> 10.8     13.7 -> 10.6
+// Rows need not be whole quads: a row's last quad is its last four channels.
+//
+// JM = 4 is that tile.  JM = 1 is for up to 16 input channels: a tile of 16 x 64 with one input
+// channel to a lane, a quarter of the matrix instructions and of the features' cutting, and
+// three waves a SIMD or more.  It is bound by the gathers of the output gradient and the wait
+// for them.
+//     3 -> 64,  415k pairs       67 -> 23 us      81 -> 21 us
+//    16 -> 64,  415k             57 -> 22 (39 with JM = 4)   59 -> 19 (33)
+//    14 -> 46,  205k             49 -> 15         64 -> 15
+// Error of the gradient against 64 bits, relative, of the first six rows above, floats:
 // 5.1e-7 -> 2.9e-7, 5.1e-7 -> 2.2e-7, 2.1e-7 -> 1.2e-7, 1.9e-7 -> 0.9e-7, 1.5e-7 -> 0.9e-7,
 // 2.8e-7 -> 1.2e-7.
 //
@@ -244,12 +269,13 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float float2v __attribute__((ext_vector_type(2)));
 typedef int int4v __attribute__((ext_vector_type(4)));
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kBwStep = 32;                      // pairs of a wave's step
 constexpr unsigned kBwOutside = 0x7FFFF000u;     // byte offset beyond either matrix
 constexpr unsigned kBwColOutside = 0x80000000u;  // (added to any row's offset: outside as well)
 
-template <typename IO>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <typename IO, int JM>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 4 ? 2 : 3)))
     conv_bwd_filter_parts_kernel(const IO *__restrict__ feats, int n_in, int cin,
                                  const IO *__restrict__ dout, int n_out, int cout,
                                  const int32_t *__restrict__ pairs, int64_t pair_stride,
@@ -257,8 +283,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                                  int n_co_tiles, int K, int n_tiles, float *__restrict__ partial) {
   constexpr int P = sizeof(IO) == 4 ? 3 : 2;
   constexpr unsigned kEB = sizeof(IO);
+  constexpr int kRows = 16 * JM;  // rows (ci) of the tile
   typedef decltype(buf_quad(__amdgpu_buffer_rsrc_t(), 0u, (const IO *)nullptr)) Quad;
-  __shared__ __align__(16) float tile[4 * kBwTile * kBwTile];
+  typedef std::conditional_t<JM == 4, Quad, IO> FeatQuad;
+  __shared__ __align__(16) float tile[4 * kRows * kBwTile];
   __shared__ int odd_s;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -270,7 +298,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int item = xcd * (total >> 3) + min(xcd, total & 7) + slot;
   const int s = item / (K * n_tiles), kt = item - s * (K * n_tiles);
   const int k = kt / n_tiles, t_co = kt % n_tiles;
-  const int ci0 = (t_co / n_co_tiles) * kBwTile;
+  const int ci0 = (t_co / n_co_tiles) * kRows;
   const int co0 = (t_co % n_co_tiles) * kBwTile;
   const int n = pair_num[k];
   int len = (n + n_split - 1) / n_split;
@@ -288,14 +316,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       __builtin_amdgcn_make_buffer_rsrc((void *)feats, 0, (int)(n_in * row_f), 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_d =
       __builtin_amdgcn_make_buffer_rsrc((void *)dout, 0, (int)(n_out * row_d), 0x00020000);
-  const unsigned col_f = ci0 + 4 * l16 < cin ? (unsigned)(ci0 + 4 * l16) * kEB : kBwColOutside;
-  const unsigned col_d = co0 + 4 * l16 < cout ? (unsigned)(co0 + 4 * l16) * kEB : kBwColOutside;
+  // The last quad of a row that ends within it is the row's last four channels: its first ones
+  // are worked out twice, to the same bits.
+  const auto quad = [](int c, int width) { return min(c, width - 4); };
+  const int ci = JM == 4 ? ci0 + 4 * l16 : ci0 + l16, co = co0 + 4 * l16;
+  const unsigned col_f =
+      ci < cin ? (unsigned)(JM == 4 ? quad(ci, cin) : ci) * kEB : kBwColOutside;
+  const unsigned col_d = co < cout ? (unsigned)quad(co, cout) * kEB : kBwColOutside;
   if (tid == 0) odd_s = 0;
 
-  // acc[jm][jn]: D[ci0 + 4*(4g + r) + jm][co0 + 4*l16 + jn] in component r
-  float4v acc[4][4];
+  // acc[jm][jn]: D[ci0 + JM*(4g + r) + jm][co0 + 4*l16 + jn] in component r
+  float4v acc[JM][4];
   int idx_f[8], idx_d[8];
-  Quad qf[8], qd[8];
+  FeatQuad qf[8];
+  Quad qd[8];
   auto load_idx = [&](const __amdgpu_buffer_rsrc_t &rs, int p0, int (&idx)[8])
       __attribute__((always_inline)) {
     if (p0 + kBwStep > p_end) {  // (no load that lies partly behind the range)
@@ -328,7 +362,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     offsets(p0, n_in, idx_f, row_f, col_f, off);
     load_idx(rs_i, p0 + 4 * kBwStep, idx_f);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) qf[j] = buf_quad(rs_f, off[j], feats);
+    for (int j = 0; j < 8; ++j) {
+      if constexpr (JM == 4)
+        qf[j] = buf_quad(rs_f, off[j], feats);
+      else
+        qf[j] = buf_one(rs_f, off[j], feats);
+    }
   };
   auto load_d = [&](int p0) __attribute__((always_inline)) {
     unsigned off[8];
@@ -341,7 +380,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int p_wave = p_begin + wave * kBwStep;
   auto run = [&](auto multiply) __attribute__((always_inline)) {
 #pragma unroll
-    for (int jm = 0; jm < 4; ++jm)
+    for (int jm = 0; jm < JM; ++jm)
 #pragma unroll
       for (int jn = 0; jn < 4; ++jn) acc[jm][jn] = float4v{0.f, 0.f, 0.f, 0.f};
     if (p_wave < p_end) {
@@ -358,10 +397,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   asm volatile("" : "+s"(minus0), "+s"(minus1));
   const bf16x2 m0 = __builtin_bit_cast(bf16x2, minus0), m1 = __builtin_bit_cast(bf16x2, minus1);
   // the operand of channel block c, part by part
-  auto cut = [&](const Quad (&q)[8], int c, int4v (&part)[P]) __attribute__((always_inline)) {
+  auto cut = [&](const auto (&q)[8], int c, int4v (&part)[P]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      float u = widen4(q[2 * j])[c], v = widen4(q[2 * j + 1])[c];
+      float u = element(q[2 * j], c), v = element(q[2 * j + 1], c);
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         const bf16x2 b = __builtin_convertvector(float2v{u, v}, bf16x2);
@@ -374,9 +413,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
   };
   run([&](int p0) __attribute__((always_inline)) {
-    int4v pf[4][P];
+    int4v pf[JM][P];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) cut(qf, c, pf[c]);
+    for (int c = 0; c < JM; ++c) cut(qf, c, pf[c]);
     load_f(p0 + 4 * kBwStep);  // (in flight during the multiplications)
     // (a channel block of the gradient is cut among the multiplications of the one before; the
     // barriers keep the compiler from cutting them all at once, for which there are no registers)
@@ -394,75 +433,85 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       // A step's products are summed by themselves, the smallest first (of floats only those
       // of parts a + b <= 2), and added to the sum of the steps before: one rounding at its
       // size a step, not one an instruction.
-      float4v t[4];
+      float4v t[JM];
 #pragma unroll
-      for (int jm = 0; jm < 4; ++jm) t[jm] = float4v{0.f, 0.f, 0.f, 0.f};
+      for (int jm = 0; jm < JM; ++jm) t[jm] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int a = P - 1; a >= 0; --a)
 #pragma unroll
         for (int b = P - 1; b >= 0; --b) {
           if (a + b > 2) continue;
 #pragma unroll
-          for (int jm = 0; jm < 4; ++jm)
+          for (int jm = 0; jm < JM; ++jm)
             t[jm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pf[jm][a]),
                                                             __builtin_bit_cast(bf16x8, pd[b]), t[jm],
                                                             0, 0, 0);
         }
 #pragma unroll
-      for (int jm = 0; jm < 4; ++jm) acc[jm][jn] += t[jm];
+      for (int jm = 0; jm < JM; ++jm) acc[jm][jn] += t[jm];
       __builtin_amdgcn_sched_barrier(0);
     }
   });
   __syncthreads();  // (odd_s is cleared)
   {
-    bool odd = false;
+    // (bits << 1) - 1 takes the sign away and zero to the top; 0 times what is not finite is NaN
+    uint32_t least = 0xFFFFFFFFu;
+    float nan = 0.f;
 #pragma unroll
-    for (int jm = 0; jm < 4; ++jm)
+    for (int jm = 0; jm < JM; ++jm)
 #pragma unroll
       for (int jn = 0; jn < 4; ++jn)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float m = fabsf(acc[jm][jn][r]);
-          odd = odd || !(m <= 3.402823466e38f) || (m < 8.271806125530277e-25f && m != 0.f);
+          const float v = acc[jm][jn][r];
+          least = min(least, (__builtin_bit_cast(uint32_t, v) << 1) - 1u);
+          nan = __builtin_fmaf(v, 0.f, nan);
         }
+    const bool odd = nan != 0.f || least < ((127u - 80u) << 24) - 1u;
     if (odd) odd_s = 1;
   }
   __syncthreads();
   if (odd_s != 0) {
     run([&](int p0) __attribute__((always_inline)) {
-      float4v xf[8], xd[8];
+      float xf[8][JM], xd[8][4];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        xf[j] = widen4(qf[j]);
-        xd[j] = widen4(qd[j]);
+#pragma unroll
+        for (int c = 0; c < JM; ++c) xf[j][c] = element(qf[j], c);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) xd[j][c] = element(qd[j], c);
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int jm = 0; jm < 4; ++jm)
+        for (int jm = 0; jm < JM; ++jm)
 #pragma unroll
           for (int jn = 0; jn < 4; ++jn)
-            acc[jm][jn] = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[j][jm], xd[j][jn], acc[jm][jn], 0, 0, 0);
+            acc[jm][jn] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(xf[j][jm], xd[j][jn], acc[jm][jn], 0, 0, 0);
       load_f(p0 + 4 * kBwStep);
       load_d(p0 + 4 * kBwStep);
     });
   }
-  // The four waves' tiles in wave order, then the tile out (as above).
+  // The four waves' tiles in wave order, then the tile out.
 #pragma unroll
-  for (int jm = 0; jm < 4; ++jm)
+  for (int jm = 0; jm < JM; ++jm)
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      *reinterpret_cast<float4v *>(tile + wave * kBwTile * kBwTile + (4 * (4 * g + r) + jm) * kBwTile + 4 * l16) =
+      *reinterpret_cast<float4v *>(tile + (wave * kRows + JM * (4 * g + r) + jm) * kBwTile + 4 * l16) =
           float4v{acc[jm][0][r], acc[jm][1][r], acc[jm][2][r], acc[jm][3][r]};
   __syncthreads();
   float *dst = partial + ((int64_t)s * K + k) * cin * cout;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int ci = ci0 + 4 * (4 * wave + i) + g, co = co0 + 4 * l16;
-    const float4v *t = reinterpret_cast<const float4v *>(tile + (4 * (4 * wave + i) + g) * kBwTile + 4 * l16);
-    constexpr int kQ = kBwTile * kBwTile / 4;
+  for (int i = 0; i < JM; ++i) {
+    const int row = JM == 4 ? 4 * (4 * wave + i) + g : 4 * wave + g;
+    const float4v *t = reinterpret_cast<const float4v *>(tile + row * kBwTile + 4 * l16);
+    constexpr int kQ = kRows * kBwTile / 4;
     const float4v v = ((t[0] + t[kQ]) + t[2 * kQ]) + t[3 * kQ];
-    if (ci < cin && co < cout) *reinterpret_cast<float4v *>(dst + (int64_t)ci * cout + co) = v;
+    const int c0 = JM == 4 ? ci0 + 4 * (4 * wave + i) : ci0 + row;
+    const int c = JM == 4 ? quad(c0, cin) + g : c0;
+    if (c0 < cin && co < cout)
+      *reinterpret_cast<float4u *>(dst + (int64_t)c * cout + quad(co, cout)) = v;
   }
 }
 
@@ -475,8 +524,14 @@ __global__ void __launch_bounds__(256)
   const int64_t per = (int64_t)K * cin * cout;
   if (e >= per) return;
   float v = partial[e];
-#pragma unroll 8
-  for (int s = 1; s < n_split; ++s) v += partial[(int64_t)s * per + e];
+  for (int s = 1; s < n_split; s += 8) {  // (eight loads in flight, also at the end)
+    float w[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = partial[(int64_t)min(s + i, n_split - 1) * per + e];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (s + i < n_split) v += w[i];
+  }
   int co, ci, k;
   if (per <= 0xFFFFFFFFll) {
     const unsigned r = (unsigned)e / (unsigned)cout;
@@ -576,20 +631,23 @@ static int conv_bwd_filter(const IO *features, int64_t n_in, int32_t c_in, const
   const bool buf = (c_in & 3) == 0 && (c_out & 3) == 0 && feat_bytes <= 0xFFFFF000u &&
                    dout_bytes <= 0xFFFFF000u;
   // (row numbers and row sizes of 24 bits, offsets of 31: the index arithmetic of the kernel;
-  // within it that kernel is the faster one at every size measured, from 1.1 to 2 times)
-  const bool parts = (c_in & 3) == 0 && (c_out & 3) == 0 && feat_bytes <= kBwOutside &&
+  // within it that kernel is the faster one at every size measured, from 1.1 to 3 times)
+  const bool parts = c_out >= 4 && feat_bytes <= kBwOutside &&
                      dout_bytes <= kBwOutside && n_in < (1 << 24) && n_out < (1 << 24) &&
                      (uint64_t)c_in * sizeof(IO) < (1u << 24) && (uint64_t)c_out * sizeof(IO) < (1u << 24) &&
                      pair_stride < (1 << 28);
   const int n_split = parts ? bwd_parts_split(K, c_in, c_out, pair_stride, n_in, n_out)
                             : bwd_split(K, c_in, c_out, pair_stride);
   const dim3 grid((unsigned)n_split, (unsigned)K, (unsigned)(n_ci_tiles * n_co_tiles));
-  if (parts)
-    hipLaunchKernelGGL(conv_bwd_filter_parts_kernel<IO>, dim3(grid.x * grid.y * grid.z), dim3(256), 0,
-                       s, features, (int)n_in, c_in, out_grad, (int)n_out, c_out,
-                       pairs, pair_stride, pair_num, plane_in, n_split, n_co_tiles, K,
-                       n_ci_tiles * n_co_tiles, partial);
-  else if (buf)
+  if (parts) {
+    // up to 16 channels: a tile of 16 rows, one to a lane, that takes a quarter of the instructions
+    const int n_tiles = (c_in <= 16 ? 1 : n_ci_tiles) * n_co_tiles;
+    hipLaunchKernelGGL((c_in <= 16 ? conv_bwd_filter_parts_kernel<IO, 1>
+                                   : conv_bwd_filter_parts_kernel<IO, 4>),
+                       dim3((unsigned)(n_split * K * n_tiles)), dim3(256), 0, s, features, (int)n_in,
+                       c_in, out_grad, (int)n_out, c_out, pairs, pair_stride, pair_num, plane_in,
+                       n_split, n_co_tiles, K, n_tiles, partial);
+  } else if (buf)
     hipLaunchKernelGGL((conv_bwd_filter_kernel<IO, true>), grid, dim3(256), 0, s, features, c_in,
                        (unsigned)feat_bytes, out_grad, c_out, (unsigned)dout_bytes, pairs,
                        pair_stride, pair_num, plane_in, n_split, n_co_tiles, partial);

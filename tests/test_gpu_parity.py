@@ -2842,7 +2842,9 @@ def test_convolution_whose_output_gets_no_gradient(device, monkeypatch):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("cin,cout,inverse,what", [
     (4, 4, 0, "plain"), (60, 64, 1, "plain"), (64, 68, 0, "plain"), (132, 128, 1, "plain"),
-    (68, 8, 0, "huge"), (8, 68, 0, "tiny"), (64, 64, 0, "not finite"), (5, 64, 0, "plain")])
+    (68, 8, 0, "huge"), (8, 68, 0, "tiny"), (64, 64, 0, "not finite"), (14, 66, 1, "not finite"),
+    (1, 4, 0, "plain"), (3, 64, 0, "plain"), (16, 5, 1, "plain"), (17, 64, 0, "plain"),
+    (31, 30, 1, "plain"), (65, 67, 0, "plain"), (5, 3, 0, "plain")])
 def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
     """Offsets of pairs on both sides of a wave's and a workgroup's step, none at all and several
     ranges; tiles that the channels fill in part; elements that have no bfloat16 parts (near the
@@ -2866,7 +2868,7 @@ def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
         f[::7, ::3] = torch.finfo(torch.float32).max
     if what == "not finite":
         f[pairs[3, inverse, 5].long(), 7], d[20, 9] = float("inf"), float("nan")
-        f[pairs[8, inverse, 150].long(), 63] = float("-inf")
+        f[pairs[8, inverse, 150].long(), -1] = float("-inf")
     num = torch.tensor(counts, dtype=torch.int32, device=device)
     p_dev, f_dev, d_dev = pairs.to(device), f.to(device), d.to(device)
 
