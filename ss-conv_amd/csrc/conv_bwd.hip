@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
 // instructions (7 for every two elements that are cut) and the gathers take about as long
 // each, and with the two waves a SIMD that 252 registers leave the three overlap in part only
 // (a wave waits for rows in 37 % of its time).  Finer interleaving of loads and matrix
-// instructions, or waiting for L1 only, gained less than 5 %.  Measured, both kernels with
+// instructions gained nothing, rows that all lie in L1 a tenth.  Measured, both kernels with
 // their reduction, before -> now:
 //                                   float            half
 //    64 -> 128, 1.54M pairs    282 -> 192 us    274 -> 135 us
@@ -262,9 +262,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
 // 2.8e-7 -> 1.2e-7.
 //
 // Infinities and NaN have no parts, and the parts of numbers below 2^-110 are cut off at
-// 2^-134: a workgroup that ends with a sum that is not finite, or is not zero and below
-// 2^-80, works its range out again with float instructions (lane (l16, g)'s row 8 g + j is
-// k slot g of step j).
+// 2^-134, which is within a float's rounding of a sum of 2^-80 as long as the other factor is
+// no more than 2^30: a workgroup that ends with a sum that is not finite, or is not zero and
+// below 2^-80, or that met an element above 2^30, works its range out again with float
+// instructions (lane (l16, g)'s row 8 g + j is k slot g of step j).
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float float2v __attribute__((ext_vector_type(2)));
@@ -346,14 +347,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
       for (int j = 0; j < 4; ++j) idx[4 * h + j] = v[j];
     }
   };
-  // Byte offsets of a step's rows (row `rows` is behind the matrix' end: it reads as zeros).
+  // Byte offsets of a step's rows.  Row `rows` is behind the matrix' end and reads as zeros, for
+  // pairs behind the range and row numbers below 0.
   auto offsets = [&](int p0, int rows, int (&idx)[8], unsigned row, unsigned col,
                      unsigned (&off)[8]) __attribute__((always_inline)) {
     if (p0 + kBwStep > p_end)
 #pragma unroll
       for (int j = 0; j < 8; ++j) idx[j] = p0 + 8 * g + j < p_end ? idx[j] : rows;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) off[j] = __umul24((unsigned)idx[j], row) + col;
+    for (int j = 0; j < 8; ++j)
+      off[j] = __umul24(min((unsigned)idx[j], (unsigned)rows), row) + col;
   };
   // A step's rows, and after them the row numbers of the wave's next step: a wait for those
   // is not a wait for loads of rows that are younger.
@@ -396,11 +399,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
   uint32_t minus0 = 0x0000BF80u, minus1 = 0xBF800000u;
   asm volatile("" : "+s"(minus0), "+s"(minus1));
   const bf16x2 m0 = __builtin_bit_cast(bf16x2, minus0), m1 = __builtin_bit_cast(bf16x2, minus1);
+  float largest = 0.f;
   // the operand of channel block c, part by part
   auto cut = [&](const auto (&q)[8], int c, int4v (&part)[P]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       float u = element(q[2 * j], c), v = element(q[2 * j + 1], c);
+      // (in this place: left to the compiler, the chain of maxima holds all elements at once)
+      if (P == 3) asm volatile("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(u), "v"(v));
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         const bf16x2 b = __builtin_convertvector(float2v{u, v}, bf16x2);
@@ -467,7 +473,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
           least = min(least, (__builtin_bit_cast(uint32_t, v) << 1) - 1u);
           nan = __builtin_fmaf(v, 0.f, nan);
         }
-    const bool odd = nan != 0.f || least < ((127u - 80u) << 24) - 1u;
+    const bool odd = nan != 0.f || largest > 1073741824.f || least < ((127u - 80u) << 24) - 1u;
     if (odd) odd_s = 1;
   }
   __syncthreads();

@@ -2842,13 +2842,13 @@ def test_convolution_whose_output_gets_no_gradient(device, monkeypatch):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("cin,cout,inverse,what", [
     (4, 4, 0, "plain"), (60, 64, 1, "plain"), (64, 68, 0, "plain"), (132, 128, 1, "plain"),
-    (68, 8, 0, "huge"), (8, 68, 0, "tiny"), (64, 64, 0, "not finite"), (14, 66, 1, "not finite"),
+    (68, 8, 0, "huge"), (8, 68, 0, "tiny"), (64, 64, 0, "far apart"), (64, 64, 0, "not finite"), (14, 66, 1, "not finite"),
     (1, 4, 0, "plain"), (3, 64, 0, "plain"), (16, 5, 1, "plain"), (17, 64, 0, "plain"),
     (31, 30, 1, "plain"), (65, 67, 0, "plain"), (5, 3, 0, "plain")])
 def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
     """Offsets of pairs on both sides of a wave's and a workgroup's step, none at all and several
     ranges; tiles that the channels fill in part; elements that have no bfloat16 parts (near the
-    largest float, below 2^-80, infinities and NaN).  Against 64 bits, element by element: a
+    largest float, below 2^-110, infinities and NaN).  Against 64 bits, element by element: a
     float sum of m products is off by no more than m units of 2^-24 of the sum of their sizes,
     8 more for the additions of waves and ranges; a half result is the rounded float one."""
     from ss_conv import _ext
@@ -2864,11 +2864,14 @@ def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
     if what in ("huge", "tiny") and dtype == torch.float32:
         f, d = (f * 2.0 ** 125, d * 2.0 ** -90) if what == "huge" else (f * 2.0 ** -50, d * 2.0 ** -45)
     f, d = f.to(dtype), d.to(dtype)
+    if what == "far apart" and dtype == torch.float32:
+        f, d = torch.where(f.abs() < 0.01, torch.full_like(f, 0.01), f) * 2.0 ** -118, d * 2.0 ** 100
     if what == "huge" and dtype == torch.float32:
         f[::7, ::3] = torch.finfo(torch.float32).max
     if what == "not finite":
         f[pairs[3, inverse, 5].long(), 7], d[20, 9] = float("inf"), float("nan")
         f[pairs[8, inverse, 150].long(), -1] = float("-inf")
+    pairs[9, :, 700] = -1  # (no pair: adds nothing)
     num = torch.tensor(counts, dtype=torch.int32, device=device)
     p_dev, f_dev, d_dev = pairs.to(device), f.to(device), d.to(device)
 
@@ -2889,8 +2892,8 @@ def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
         assert torch.equal(half.nan_to_num(7.0), got.half().nan_to_num(7.0))
         assert torch.equal(half.isnan(), got.isnan())
     for k, m in enumerate(counts):
-        a = f[pairs[k, inverse, :m].long()].double()
-        b = d[pairs[k, 1 - inverse, :m].long()].double()
+        pair = pairs[k, :, :m][:, pairs[k, 0, :m] >= 0].long()
+        a, b = f[pair[inverse]].double(), d[pair[1 - inverse]].double()
         ref, size = a.t() @ b, a.abs().t() @ b.abs()
         finite = ref.isfinite()
         assert torch.equal(got[k].isnan(), ref.isnan()), k
