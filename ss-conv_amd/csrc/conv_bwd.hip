@@ -239,8 +239,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
 // instructions gained nothing, rows that all lie in L1 a tenth.  Measured, both kernels with
 // their reduction, before -> now:
 //                                   float            half
-//    64 -> 128, 1.54M pairs    282 -> 192 us    274 -> 135 us
-//   128 -> 128, 0.78M pairs    278 -> 183       278 -> 135
+//    64 -> 128, 1.54M pairs    282 -> 195 us    274 -> 135 us
+//   128 -> 128, 0.78M pairs    278 -> 186       278 -> 137
 //    64 -> 64,  137k pairs      34 -> 21         34 -> 19
 //    32 -> 32,  44k pairs       19.3 -> 15.7     20 -> 13.8
 //    64 -> 152, stride 2, 52k   31 -> 24         31 -> 21
