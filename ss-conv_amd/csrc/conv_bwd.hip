@@ -318,7 +318,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
   const __amdgpu_buffer_rsrc_t rs_d =
       __builtin_amdgcn_make_buffer_rsrc((void *)dout, 0, (int)(n_out * row_d), 0x00020000);
   // The last quad of a row that ends within it is the row's last four channels: its first ones
-  // are worked out twice, to the same bits.
+  // are worked out twice, and stored by the quad that begins with them (or before them), which
+  // may be another workgroup's.
   const auto quad = [](int c, int width) { return min(c, width - 4); };
   const int ci = JM == 4 ? ci0 + 4 * l16 : ci0 + l16, co = co0 + 4 * l16;
   const unsigned col_f =
@@ -516,8 +517,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
     const float4v v = ((t[0] + t[kQ]) + t[2 * kQ]) + t[3 * kQ];
     const int c0 = JM == 4 ? ci0 + 4 * (4 * wave + i) : ci0 + row;
     const int c = JM == 4 ? quad(c0, cin) + g : c0;
-    if (c0 < cin && co < cout)
-      *reinterpret_cast<float4u *>(dst + (int64_t)c * cout + quad(co, cout)) = v;
+    if (c0 >= cin || co >= cout || c < c0) continue;  // (c < c0: a row of the quad before)
+    float *const to = dst + (int64_t)c * cout + quad(co, cout);
+    const int skip = co - quad(co, cout);  // columns of the quad before
+    if (skip == 0)
+      *reinterpret_cast<float4u *>(to) = v;
+    else
+#pragma unroll
+      for (int j = 1; j < 4; ++j)
+        if (j >= skip) to[j] = v[j];
   }
 }
 

@@ -2900,3 +2900,44 @@ def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
         assert torch.equal(got[k][ref.isinf()].double(), ref[ref.isinf()]), k
         off = (got[k].double() - ref).abs()
         assert bool((off <= (m + 8) * 2.0 ** -24 * size)[finite].all()), (k, m)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_filter_gradient_one_tile_to_an_element(dtype, device):
+    """65 x 67 channels: the last tiles' four channels reach back into the tile before them.  With
+    an infinity in channel 0 the first tiles work with float instructions and the last do not, so
+    the channels both have come out in different bits: those of the tile that the channel lies in
+    are stored, at every call.  They are the ones of a call with that tile alone."""
+    from ss_conv import _ext
+    K, m, n = 3, 4000, 4096
+    gen = torch.Generator().manual_seed(5)
+    f = torch.randn((n, 65), generator=gen).to(dtype)
+    d = torch.randn((n, 67), generator=gen).to(dtype)
+    pairs = torch.stack([torch.stack([torch.randperm(n, generator=gen)[:m], torch.arange(m)])
+                         for _ in range(K)]).int().to(device)
+    num = torch.full((K,), m, dtype=torch.int32, device=device)
+    entry = (_ext._lib.ssc_conv_bwd_filter_f32 if dtype == torch.float32
+             else _ext._lib.ssc_conv_bwd_filter_f16)
+
+    def run(a, b):
+        a, b = a.contiguous().to(device), b.contiguous().to(device)
+        cin, cout = a.shape[1], b.shape[1]
+        out = torch.full((K, cin, cout), 7.0, dtype=dtype, device=device)
+        need = _ext._lib.ssc_conv_bwd_filter_workspace_bytes(K, cin, cout, m)
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        _ext._check(entry(a.data_ptr(), n, cin, b.data_ptr(), n, cout, pairs.data_ptr(), m,
+                          num.data_ptr(), K, 0, out.data_ptr(), cin * cout, cout, 1,
+                          ws.data_ptr(), need, _ext._stream(a)))
+        return out.cpu().nan_to_num(7.0)
+
+    f_odd, d_odd = f.clone(), d.clone()
+    f_odd[:, 0], d_odd[:, 0] = float("inf"), float("inf")
+    for a, b in ((f_odd, d), (f, d_odd), (f_odd, d_odd), (f, d)):
+        got = run(a, b)
+        assert torch.equal(got, run(a, b))
+        assert torch.equal(got[:, :64, :64], run(a[:, :64], b[:, :64]))
+        last = run(a[:, 1:], b[:, :64])
+        assert torch.equal(got[:, 64:, :64], last[:, 63:])
+        assert torch.equal(got[:, :64, 64:], run(a[:, :64], b[:, 3:])[:, :, 61:])
+        if a is f_odd and b is d and dtype == torch.float32:  # (else nothing has been shown)
+            assert not torch.equal(got[:, 61:64, :64], last[:, 60:63])
