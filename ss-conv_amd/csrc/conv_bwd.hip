@@ -261,11 +261,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
 // 5.1e-7 -> 2.9e-7, 5.1e-7 -> 2.2e-7, 2.1e-7 -> 1.2e-7, 1.9e-7 -> 0.9e-7, 1.5e-7 -> 0.9e-7,
 // 2.8e-7 -> 1.2e-7.
 //
-// Infinities and NaN have no parts, and the parts of numbers below 2^-110 are cut off at
-// 2^-134, which is within a float's rounding of a sum of 2^-80 as long as the other factor is
-// no more than 2^30: a workgroup that ends with a sum that is not finite, or is not zero and
-// below 2^-80, or that met an element above 2^30, works its range out again with float
-// instructions (lane (l16, g)'s row 8 g + j is k slot g of step j).
+// What the parts cannot do is worked out with float instructions instead: a workgroup that meets
+// one of the following takes its range again (lane (l16, g)'s row 8 g + j is k slot g of step j).
+//  - Infinities, NaN, and floats that round to an infinity as bfloat16: a sum that is not finite.
+//  - Elements with bits below 2^-133, the last of a bfloat16: parts that do not add up.  What is
+//    left of an element for its third part is a bfloat16 then and only then if the lower half of
+//    its word is zero (conversion, dot product and matrix instruction keep subnormals), so one
+//    OR of two elements' words shows it.  Elements of 2^-110 and above, and zero, always pass.
+//  - Sums that are not zero and below 2^-95: six products of parts, each rounded at 2^-150, where
+//    the float instruction rounds one; of 2^26 pairs (a wave's most) they are off by 2^-121.4,
+//    which is 2^-26 of 2^-95.  A sum of zero has no product above the smallest subnormal, or its
+//    products cancel as they are.
+// Where every workgroup does so, 64 -> 128 channels take 360 us instead of 174.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float float2v __attribute__((ext_vector_type(2)));
@@ -276,7 +283,7 @@ constexpr unsigned kBwOutside = 0x7FFFF000u;     // byte offset beyond either ma
 constexpr unsigned kBwColOutside = 0x80000000u;  // (added to any row's offset: outside as well)
 
 template <typename IO, int JM>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 4 ? 2 : 3)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 4 ? 2 : 4)))
     conv_bwd_filter_parts_kernel(const IO *__restrict__ feats, int n_in, int cin,
                                  const IO *__restrict__ dout, int n_out, int cout,
                                  const int32_t *__restrict__ pairs, int64_t pair_stride,
@@ -400,16 +407,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
   uint32_t minus0 = 0x0000BF80u, minus1 = 0xBF800000u;
   asm volatile("" : "+s"(minus0), "+s"(minus1));
   const bf16x2 m0 = __builtin_bit_cast(bf16x2, minus0), m1 = __builtin_bit_cast(bf16x2, minus1);
-  float largest = 0.f;
-  // the operand of channel block c, part by part
-  auto cut = [&](const auto (&q)[8], int c, int4v (&part)[P]) __attribute__((always_inline)) {
+  uint32_t rest = 0;  // the words of which the third parts are made
+  // The operand of channel block c, part by part.  `hold` has the chain of ORs end with the block:
+  // left to the compiler, the features' holds all of them at once (53 registers spilled), and
+  // held at every element it waits for the dot products (184 us for 64 -> 128 channels instead
+  // of 174; 171 with the maximum that misses elements below 2^-134).
+  auto cut = [&](const auto (&q)[8], int c, int4v (&part)[P], bool hold)
+      __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       float u = element(q[2 * j], c), v = element(q[2 * j + 1], c);
-      // (in this place: left to the compiler, the chain of maxima holds all elements at once)
-      if (P == 3) asm volatile("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(u), "v"(v));
 #pragma unroll
       for (int p = 0; p < P; ++p) {
+        if (p == 2) {
+          rest |= __builtin_bit_cast(uint32_t, u) | __builtin_bit_cast(uint32_t, v);
+          if (hold && j == 3) asm volatile("" : "+v"(rest));
+        }
         const bf16x2 b = __builtin_convertvector(float2v{u, v}, bf16x2);
         part[p][j] = __builtin_bit_cast(int, b);
         if (p + 1 < P) {
@@ -422,17 +435,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
   run([&](int p0) __attribute__((always_inline)) {
     int4v pf[JM][P];
 #pragma unroll
-    for (int c = 0; c < JM; ++c) cut(qf, c, pf[c]);
+    for (int c = 0; c < JM; ++c) cut(qf, c, pf[c], true);
     load_f(p0 + 4 * kBwStep);  // (in flight during the multiplications)
     // (a channel block of the gradient is cut among the multiplications of the one before; the
     // barriers keep the compiler from cutting them all at once, for which there are no registers)
     int4v pds[2][P];
-    cut(qd, 0, pds[0]);
+    cut(qd, 0, pds[0], false);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int jn = 0; jn < 4; ++jn) {
       const int4v (&pd)[P] = pds[jn & 1];
-      if (jn < 3) cut(qd, jn + 1, pds[(jn + 1) & 1]);
+      if (jn < 3) cut(qd, jn + 1, pds[(jn + 1) & 1], false);
       if (jn == 2) {
         __builtin_amdgcn_sched_barrier(0);
         load_d(p0 + 4 * kBwStep);
@@ -474,7 +487,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
           least = min(least, (__builtin_bit_cast(uint32_t, v) << 1) - 1u);
           nan = __builtin_fmaf(v, 0.f, nan);
         }
-    const bool odd = nan != 0.f || largest > 1073741824.f || least < ((127u - 80u) << 24) - 1u;
+    const bool odd = nan != 0.f || (rest & 0xFFFFu) != 0 || least < ((127u - 95u) << 24) - 1u;
     if (odd) odd_s = 1;
   }
   __syncthreads();

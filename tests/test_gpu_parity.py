@@ -2843,14 +2843,19 @@ def test_convolution_whose_output_gets_no_gradient(device, monkeypatch):
 @pytest.mark.parametrize("cin,cout,inverse,what", [
     (4, 4, 0, "plain"), (60, 64, 1, "plain"), (64, 68, 0, "plain"), (132, 128, 1, "plain"),
     (68, 8, 0, "huge"), (8, 68, 0, "tiny"), (64, 64, 0, "far apart"), (64, 64, 0, "not finite"), (14, 66, 1, "not finite"),
+    (64, 64, 0, "least"), (16, 64, 1, "least"), (64, 64, 0, "small"), (16, 68, 0, "below"), (68, 64, 1, "below"),
+    (64, 64, 0, "one below"), (3, 64, 0, "one below"), (64, 64, 1, "cancel"), (16, 64, 0, "cancel"),
     (1, 4, 0, "plain"), (3, 64, 0, "plain"), (16, 5, 1, "plain"), (17, 64, 0, "plain"),
     (31, 30, 1, "plain"), (65, 67, 0, "plain"), (5, 3, 0, "plain")])
 def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
     """Offsets of pairs on both sides of a wave's and a workgroup's step, none at all and several
     ranges; tiles that the channels fill in part; elements that have no bfloat16 parts (near the
-    largest float, below 2^-110, infinities and NaN).  Against 64 bits, element by element: a
+    largest float, below 2^-110, infinities and NaN), all of them, those of one channel, and such
+    that the parts of a sum cancel but the elements do not; the least elements ("least") and sums
+    ("small") that are still worked out in parts.  Against 64 bits, element by element: a
     float sum of m products is off by no more than m units of 2^-24 of the sum of their sizes,
-    8 more for the additions of waves and ranges; a half result is the rounded float one."""
+    8 more for the additions of waves and ranges, and each of them by half the least subnormal
+    (2^-150) where it ends below 2^-126; a half result is the rounded float one."""
     from ss_conv import _ext
     counts = [0, 1, 31, 32, 33, 127, 128, 129, 160, 1000, 5001]
     K, stride, n_in, n_out = len(counts), max(counts) + 2, 5003, 5007
@@ -2866,6 +2871,22 @@ def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
     f, d = f.to(dtype), d.to(dtype)
     if what == "far apart" and dtype == torch.float32:
         f, d = torch.where(f.abs() < 0.01, torch.full_like(f, 0.01), f) * 2.0 ** -118, d * 2.0 ** 100
+    if what in ("least", "small") and dtype == torch.float32:
+        # full significands, one sign: every sum is at least its least product (2^-80, 2^-92)
+        low, of = (-109, 29) if what == "least" else (-46, -46)
+        f = (1 + torch.rand(f.shape, generator=gen)) * 2.0 ** torch.randint(low, low + 4, f.shape, generator=gen)
+        d = (1 + torch.rand(d.shape, generator=gen)) * 2.0 ** of
+    if what == "below" and dtype == torch.float32:
+        f, d = f * 2.0 ** -138, d * 2.0 ** 20
+    if what == "one below" and dtype == torch.float32:
+        f[:, 2], d = f[:, 2] * 2.0 ** -138, d * 2.0 ** 20
+    if what == "cancel" and dtype == torch.float32:
+        # +-(1 + 2^-16) 2^-125 in turn, the one a subnormal's size larger that the parts leave out
+        f = torch.full_like(f, (1 + 2.0 ** -16) * 2.0 ** -125)
+        f[1::2] = -f[1::2] - 2.0 ** -136
+        d = torch.full_like(d, 2.0 ** 20)
+        for k, m in enumerate(counts):
+            pairs[k, inverse, :m] = torch.arange(m, dtype=torch.int32)
     if what == "huge" and dtype == torch.float32:
         f[::7, ::3] = torch.finfo(torch.float32).max
     if what == "not finite":
@@ -2899,7 +2920,7 @@ def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
         assert torch.equal(got[k].isnan(), ref.isnan()), k
         assert torch.equal(got[k][ref.isinf()].double(), ref[ref.isinf()]), k
         off = (got[k].double() - ref).abs()
-        assert bool((off <= (m + 8) * 2.0 ** -24 * size)[finite].all()), (k, m)
+        assert bool((off <= (m + 8) * (2.0 ** -24 * size + 2.0 ** -150))[finite].all()), (k, m)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
