@@ -2962,3 +2962,47 @@ def test_filter_gradient_one_tile_to_an_element(dtype, device):
         assert torch.equal(got[:, :64, 64:], run(a[:, :64], b[:, 3:])[:, :, 61:])
         if a is f_odd and b is d and dtype == torch.float32:  # (else nothing has been shown)
             assert not torch.equal(got[:, 61:64, :64], last[:, 60:63])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("rows,cin,cout", [
+    ((1 << 24) - 1, 4, 8), (1 << 24, 4, 8), ((1 << 24) - 1, 5, 6), (1 << 24, 5, 6), (1 << 24, 17, 3),
+    ((1 << 23) - 16, 64, 72), (1 << 23, 64, 72), ((1 << 24) + 1, 64, 68)])
+def test_filter_gradient_large_matrices(rows, cin, cout, dtype, device):
+    """Row numbers of 24 bits and byte offsets of 31 are the bfloat16-part kernel's: both sides of
+    these limits, quads and odd widths of the kernels beyond them, offsets above 4 GiB.  The pairs
+    are few, the first and the last rows and one that is no pair among them; the bound is that of
+    test_filter_gradient_edges.  Either matrix is the large one."""
+    from ss_conv import _ext
+    K, m, small = 3, 700, 900
+    gen = torch.Generator().manual_seed(cin)
+    at = torch.randint(0, rows, (K, m), generator=gen)
+    at[:, 0], at[:, -1], at[:, 1] = 0, rows - 1, rows - 2
+    at = at.sort(dim=1).values
+    to = torch.stack([torch.randperm(small, generator=gen)[:m] for _ in range(K)])
+    entry = (_ext._lib.ssc_conv_bwd_filter_f32 if dtype == torch.float32
+             else _ext._lib.ssc_conv_bwd_filter_f16)
+    for large_in in (True, False):
+        width = cin if large_in else cout
+        large = torch.zeros((rows, width), dtype=dtype, device=device)
+        large[at.flatten().to(device)] = torch.randn((K * m, width), generator=gen).to(dtype).to(device)
+        other = torch.randn((small, cout if large_in else cin), generator=gen).to(dtype).to(device)
+        f, d = (large, other) if large_in else (other, large)
+        pairs = torch.stack([at, to] if large_in else [to, at], dim=1).int()
+        pairs[1, :, 300] = -1
+        p_dev = pairs.to(device)
+        num = torch.full((K,), m, dtype=torch.int32, device=device)
+        out = torch.full((K, cin, cout), 7.0, dtype=dtype, device=device)
+        need = _ext._lib.ssc_conv_bwd_filter_workspace_bytes(K, cin, cout, m)
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        _ext._check(entry(f.data_ptr(), f.shape[0], cin, d.data_ptr(), d.shape[0], cout,
+                          p_dev.data_ptr(), m, num.data_ptr(), K, 0, out.data_ptr(), cin * cout,
+                          cout, 1, ws.data_ptr(), need, _ext._stream(f)))
+        for k in range(K):
+            pair = pairs[k][:, pairs[k, 0] >= 0].long().to(device)
+            a, b = f[pair[0]].cpu().double(), d[pair[1]].cpu().double()
+            ref, size = a.t() @ b, a.abs().t() @ b.abs()
+            bound = (m + 8) * 2.0 ** -24 * size
+            if dtype == torch.float16:
+                bound = bound + 2.0 ** -11 * (ref.abs() + bound) + 2.0 ** -25
+            assert bool(((out[k].cpu().double() - ref).abs() <= bound).all()), k
