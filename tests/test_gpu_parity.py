@@ -2843,7 +2843,8 @@ def test_convolution_whose_output_gets_no_gradient(device, monkeypatch):
 @pytest.mark.parametrize("cin,cout,inverse,what", [
     (4, 4, 0, "plain"), (60, 64, 1, "plain"), (64, 68, 0, "plain"), (132, 128, 1, "plain"),
     (68, 8, 0, "huge"), (8, 68, 0, "tiny"), (64, 64, 0, "far apart"), (64, 64, 0, "not finite"), (14, 66, 1, "not finite"),
-    (64, 64, 0, "least"), (16, 64, 1, "least"), (64, 64, 0, "small"), (16, 68, 0, "below"), (68, 64, 1, "below"),
+    (64, 64, 0, "least"), (16, 64, 1, "least"), (64, 64, 0, "small"), (64, 68, 1, "large"),
+    (16, 64, 0, "large"), (16, 68, 0, "below"), (68, 64, 1, "below"),
     (64, 64, 0, "one below"), (3, 64, 0, "one below"), (64, 64, 1, "cancel"), (16, 64, 0, "cancel"),
     (1, 4, 0, "plain"), (3, 64, 0, "plain"), (16, 5, 1, "plain"), (17, 64, 0, "plain"),
     (31, 30, 1, "plain"), (65, 67, 0, "plain"), (5, 3, 0, "plain")])
@@ -2852,8 +2853,8 @@ def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
     ranges; tiles that the channels fill in part; elements that have no bfloat16 parts (near the
     largest float, below 2^-110, infinities and NaN), all of them, those of one channel, and such
     that the parts of a sum cancel but the elements do not; the least elements ("least") and sums
-    ("small") that are still worked out in parts.  Against 64 bits, element by element: a
-    float sum of m products is off by no more than m units of 2^-24 of the sum of their sizes,
+    ("small") that are still worked out in parts, and large elements that are.  Against 64 bits,
+    element by element: a float sum of m products is off by no more than m units of 2^-24 of the sum of their sizes,
     8 more for the additions of waves and ranges, and each of them by half the least subnormal
     (2^-150) where it ends below 2^-126; a half result is the rounded float one."""
     from ss_conv import _ext
@@ -2876,6 +2877,8 @@ def test_filter_gradient_edges(cin, cout, inverse, what, dtype, device):
         low, of = (-109, 29) if what == "least" else (-46, -46)
         f = (1 + torch.rand(f.shape, generator=gen)) * 2.0 ** torch.randint(low, low + 4, f.shape, generator=gen)
         d = (1 + torch.rand(d.shape, generator=gen)) * 2.0 ** of
+    if what == "large" and dtype == torch.float32:
+        f, d = f * 2.0 ** 100, d * 2.0 ** 15
     if what == "below" and dtype == torch.float32:
         f, d = f * 2.0 ** -138, d * 2.0 ** 20
     if what == "one below" and dtype == torch.float32:
