@@ -237,26 +237,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
 // each, and with the two waves a SIMD that 252 registers leave the three overlap in part only
 // (a wave waits for rows in 37 % of its time).  Finer interleaving of loads and matrix
 // instructions gained nothing, rows that all lie in L1 a tenth.  Measured, both kernels with
-// their reduction, before -> now:
+// their reduction, on pairs drawn at random, conv_bwd_filter_kernel -> this one:
 //                                   float            half
-//    64 -> 128, 1.54M pairs    282 -> 195 us    274 -> 135 us
-//   128 -> 128, 0.78M pairs    278 -> 186       278 -> 137
-//    64 -> 64,  137k pairs      34 -> 21         34 -> 19
-//    32 -> 32,  44k pairs       19.3 -> 15.7     20 -> 13.8
-//    64 -> 152, stride 2, 52k   31 -> 24         31 -> 21
-//    64 -> 128, 5^3, 480k      100 -> 72        100 -> 52
-//    30 -> 31,  205k            48 -> 20         66 -> 17
-//    64 -> 64,  10k             17 -> 11         18 -> 11
-//    32 -> 32,  stride 2, 5.5k  13.6 -> 10.8     13.7 -> 10.6
+//    64 -> 128, 1.54M pairs    272 -> 175 us    270 -> 118 us
+//   128 -> 128, 0.78M pairs    260 -> 163       272 -> 121
+//    64 -> 64,  137k pairs      31 -> 21         32 -> 18
+//    32 -> 32,  44k pairs       19 -> 13         20 -> 11
+//    64 -> 152, stride 2, 52k   31 -> 21         31 -> 18
+//    64 -> 128, 5^3, 480k       89 -> 56         94 -> 45
+//    30 -> 31,  205k            46 -> 20         54 -> 18
+//    64 -> 64,  10k             17 -> 11         18 -> 10
+//    32 -> 32,  stride 2, 5.5k  13 -> 9.3        14 -> 8.7
 // Rows need not be whole quads: a row's last quad is its last four channels.
 //
 // JM = 4 is that tile.  JM = 1 is for up to 16 input channels: a tile of 16 x 64 with one input
 // channel to a lane, a quarter of the matrix instructions and of the features' cutting, and
-// three waves a SIMD or more.  It is bound by the gathers of the output gradient and the wait
-// for them.
-//     3 -> 64,  415k pairs       67 -> 23 us      81 -> 21 us
-//    16 -> 64,  415k             57 -> 22 (39 with JM = 4)   59 -> 19 (33)
-//    14 -> 46,  205k             49 -> 15         64 -> 15
+// four waves a SIMD.  It is bound by the gathers of the output gradient and the wait for them.
+//     3 -> 64,  415k pairs       65 -> 22 us      75 -> 20 us
+//    16 -> 64,  415k             56 -> 21 (39 with JM = 4)   56 -> 18 (33)
+//    14 -> 46,  205k             48 -> 13         54 -> 12
 // Error of the gradient against 64 bits, relative, of the first six rows above, floats:
 // 5.1e-7 -> 2.9e-7, 5.1e-7 -> 2.2e-7, 2.1e-7 -> 1.2e-7, 1.9e-7 -> 0.9e-7, 1.5e-7 -> 0.9e-7,
 // 2.8e-7 -> 1.2e-7.
@@ -272,7 +271,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
 //    the float instruction rounds one; of 2^26 pairs (a wave's most) they are off by 2^-121.4,
 //    which is 2^-26 of 2^-95.  A sum of zero has no product above the smallest subnormal, or its
 //    products cancel as they are.
-// Where every workgroup does so, 64 -> 128 channels take 360 us instead of 174.
+// Where every workgroup does so, 64 -> 128 channels take 360 us instead of 174 (260 in
+// conv_bwd_filter_kernel), 64 -> 64 with 137k pairs 38 instead of 21 (31), 16 -> 64 35 instead of
+// 21 (55).
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float float2v __attribute__((ext_vector_type(2)));
@@ -341,7 +342,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JM == 
   Quad qd[8];
   auto load_idx = [&](const __amdgpu_buffer_rsrc_t &rs, int p0, int (&idx)[8])
       __attribute__((always_inline)) {
-    if (p0 + kBwStep > p_end) {  // (no load that lies partly behind the range)
+    if (p0 + kBwStep > p_end) {  // (a word at a time: those behind the range read as 0)
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         idx[j] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (p0 + 8 * g + j) * 4, 0, 0);
@@ -587,7 +588,8 @@ static int bwd_split(int K, int c_in, int c_out, int64_t pair_stride) {
 // Ranges of conv_bwd_filter_parts_kernel, at most bwd_split's: as many workgroups as the chip
 // holds at once (two a CU), twice as many where their ranges are still 2048 pairs long (they
 // end less unevenly: 128 -> 128 channels, 29k pairs an offset, 206 us with 4 ranges, 200 with
-// 9), and no range below 384 pairs, as a range costs a tile written and read: 64 -> 152 with
+// 9), and one to about 384 pairs of the longest possible offset, as a range costs a tile written
+// and read (385 pairs make two ranges; shorter offsets have shorter ones): 64 -> 152 with
 // 1.9k pairs an offset 36 us with 12 ranges, 25 with 6; 64 -> 128 at 5^3 and 3.8k 84 us with 4
 // and 75 with 2; 32 -> 32 with 1.6k 18.9 us with 4 and 21.1 with 2.
 // An offset has no more pairs than either side has rows.
@@ -658,7 +660,7 @@ static int conv_bwd_filter(const IO *features, int64_t n_in, int32_t c_in, const
   const bool buf = (c_in & 3) == 0 && (c_out & 3) == 0 && feat_bytes <= 0xFFFFF000u &&
                    dout_bytes <= 0xFFFFF000u;
   // (row numbers and row sizes of 24 bits, offsets of 31: the index arithmetic of the kernel;
-  // within it that kernel is the faster one at every size measured, from 1.1 to 3 times)
+  // within it that kernel is the faster one at every size measured, from 1.4 to 4.4 times)
   const bool parts = c_out >= 4 && feat_bytes <= kBwOutside &&
                      dout_bytes <= kBwOutside && n_in < (1 << 24) && n_out < (1 << 24) &&
                      (uint64_t)c_in * sizeof(IO) < (1u << 24) && (uint64_t)c_out * sizeof(IO) < (1u << 24) &&
