@@ -206,6 +206,11 @@ int ssc_rulebook_conv_finish(const ssc_geometry *g, int64_t n_in, int32_t *n_out
  * Every row of out[n_out,Cout] is written (zeros where no pair lands).
  * ---------------------------------------------------------------------- */
 #define SSC_CONV_PAIRS_CANONICAL 2
+/* The rulebook is of a regular (not submanifold, not transposed) convolution of unit stride: may
+ * be added to `kernel_volume` of ssc_conv_fwd_*, ssc_conv_plan_build and ssc_conv_run_*, and to
+ * `elem_bytes` of ssc_rulebook_conv_begin / _finish.  It tells how many pairs to expect, which
+ * decides what form the kernel takes, and is the same in all calls on one plan. */
+#define SSC_CONV_UNIT_STRIDE 0x10000
 
 size_t ssc_conv_workspace_bytes(int64_t n_out, int32_t kernel_volume, int32_t c_in,
                                 int32_t c_out, int64_t pair_stride);
@@ -407,7 +412,10 @@ int ssc_profile_conv(int32_t enable);
  * 512  the schedule filled by a launch of its own for every plan: plans with one range to a
  *      workgroup and a single work split otherwise have it filled range by range by the
  *      launch that counts the ranges' row blocks.  Results are bit-identical (only where in
- *      its buffers a range's part of the schedule lies differs). */
+ *      its buffers a range's part of the schedule lies differs).
+ *   1024  no bfloat16-parts form (float layers of whole chunks of 64 input channels whose
+ *      offsets have pairs enough in a tile); 2048, 4096  that form with blocks of 64 or of 32
+ *      pairs wherever it can be.  Results agree to 1e-6. */
 int ssc_conv_tuning(int32_t flags);
 /* Tell the library that the caller queues index work (ssc_rulebook_*, ssc_conv_plan_build) on
  * a stream of its own, where it runs while a convolution on another stream holds every CU

@@ -11,6 +11,10 @@
 // cost MFMA work, and because each wave owns a fixed set of columns and walks the
 // offsets in ascending order the result is bit-reproducible without atomics.
 //
+// Where an offset has pairs enough in a tile (parts_block) the multiplication runs on the bfloat16
+// matrix instructions instead, every element cut into three parts that add up to it, over
+// blocks of 32 or 64 pairs: the parts form of conv_kernel.h.
+//
 // Host side of a call: pack the filters into MFMA fragment order; check that the
 // pairs are sorted (re-order them if not); split the output rows over the
 // workgroups by work and cut the ranges into tiles; build the row-block schedule;
@@ -19,6 +23,8 @@
 #include "conv_kernel.h"
 #include "conv_pack.h"
 #include "ssc_common.h"
+
+#include <algorithm>
 
 namespace ssc {
 static_assert(kPackKC == kKC, "conv_pack.h packs half filters in chunks of kKC channels");
@@ -173,8 +179,8 @@ __global__ void __launch_bounds__(256)
 // The search starts from the cell of the tile's first row in grid_segs[], the same
 // segments for a regular grid of `granule` rows (grid_segments_kernel).
 // Also spill[t*K + k] = how far the last row block of tile t-1 may reach into tile t:
-// the first pair at or after segs[t*K + k], at most 15 further, whose row is >=
-// spill_end[t].
+// the first pair at or after segs[t*K + k], at most blk - 1 further, whose row is >=
+// spill_end[t] (blk: pairs of an offset to a block, 16 or 32).
 __global__ void __launch_bounds__(256)
     tile_segments_kernel(const int32_t *__restrict__ flag, const int32_t *__restrict__ pairs,
                          const int32_t *__restrict__ sorted, int64_t pair_stride, int plane_s,
@@ -182,8 +188,8 @@ __global__ void __launch_bounds__(256)
                          const int32_t *__restrict__ n_tiles_dev,
                          const int32_t *__restrict__ tile_row0, int64_t n_out,
                          const int32_t *__restrict__ grid_segs, int granule,
-                         const int32_t *__restrict__ spill_end, int32_t *__restrict__ segs,
-                         int32_t *__restrict__ spill) {
+                         const int32_t *__restrict__ spill_end, int blk,
+                         int32_t *__restrict__ segs, int32_t *__restrict__ spill) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t n_tiles = n_tiles_dev[0];
   if (idx >= (n_tiles + 1) * K) return;
@@ -204,10 +210,13 @@ __global__ void __launch_bounds__(256)
   }
   segs[idx] = lo;
   const int bound = spill_end[t];
-  int cnt = 0;
-#pragma unroll
-  for (int j = 0; j < 15; ++j) cnt += (lo + j < n && s[lo + j] < bound) ? 1 : 0;  // rows ascend
-  spill[idx] = lo + cnt;
+  int end = lo + blk - 1 < n ? lo + blk - 1 : n, first = lo;
+  while (first < end) {  // rows ascend
+    const int mid = (first + end) >> 1;
+    if (s[mid] < bound) first = mid + 1;
+    else end = mid;
+  }
+  spill[idx] = first;
 }
 
 // segs[c*K + k] = first pair of offset k whose scatter row is >= c*granule, for the
@@ -275,19 +284,24 @@ constexpr int kSpillRows = 160;
 // (the five-group form, whose window is 376 rows: 200 -> 200 channels with 125 offsets takes
 // 14.3 ms with 160, 13.9 with 192 or 224, 14.7 with 128)
 constexpr int kSpillRowsFive = 192;
+// (the parts form, whose window is 488 rows with blocks of 32 pairs and 400 with blocks of 64)
+constexpr int kSpillRowsParts = 192;
 
 // cost of a tile beyond its pairs, in pair slots: padding per offset, and about a stage's
 // worth of time for writing it out (measured: 2 K + 128 and 3 K + 64 are as good on the
 // 27-offset benchmark layers; with 125 offsets 4 K + 64 is 4 % faster than 2 K + 128, and
 // more than that slower again)
-__device__ __forceinline__ int64_t split_tile_cost(int K) { return (int64_t)K * 4 + 64; }
+// (blocks of 32 and 64 pairs pad as much more)
+__host__ __device__ __forceinline__ int64_t split_tile_cost(int K, int blk) {
+  return (int64_t)K * (blk / 4) + 64;
+}
 
 // Work in rows below cell b of the fine grid (scaled by T to stay in integers).
 __device__ __forceinline__ int64_t split_work(int64_t pairs_below, int64_t b, int64_t n_out,
-                                              int T, int K, int granule) {
+                                              int T, int K, int granule, int blk) {
   int64_t r = b * granule;
   if (r > n_out) r = n_out;
-  return pairs_below * T + r * split_tile_cost(K);
+  return pairs_below * T + r * split_tile_cost(K, blk);
 }
 
 // One thread per cell boundary b = 0..nb of the fine grid: the ranges whose first row
@@ -295,7 +309,8 @@ __device__ __forceinline__ int64_t split_work(int64_t pairs_below, int64_t b, in
 // (work(b-1), work(b)].  range_row0[w], w = 0..n_wg.
 __global__ void __launch_bounds__(256)
     split_bounds_kernel(const int32_t *__restrict__ fine_segs, int K, int64_t nb, int64_t n_out,
-                        int T, int n_wg, int granule, int32_t *__restrict__ range_row0) {
+                        int T, int n_wg, int granule, int blk,
+                        int32_t *__restrict__ range_row0) {
   int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b > nb) return;
   int64_t below = 0, below_prev = 0, all = 0;
@@ -304,15 +319,15 @@ __global__ void __launch_bounds__(256)
     if (b > 0) below_prev += fine_segs[(b - 1) * K + k];
     all += fine_segs[nb * K + k];
   }
-  const int64_t total = split_work(all, nb, n_out, T, K, granule);
+  const int64_t total = split_work(all, nb, n_out, T, K, granule, blk);
   // ranges w with ceil(total * w / n_wg) <= work, i.e. w <= work * n_wg / total
   auto reached = [&](int64_t work) -> int64_t {
     if (total <= 0) return n_wg + 1;
     int64_t c = work * n_wg / total + 1;
     return c > n_wg + 1 ? n_wg + 1 : c;
   };
-  const int64_t w0 = b > 0 ? reached(split_work(below_prev, b - 1, n_out, T, K, granule)) : 0;
-  const int64_t w1 = reached(split_work(below, b, n_out, T, K, granule));
+  const int64_t w0 = b > 0 ? reached(split_work(below_prev, b - 1, n_out, T, K, granule, blk)) : 0;
+  const int64_t w1 = reached(split_work(below, b, n_out, T, K, granule, blk));
   int64_t r = b * granule;
   if (r > n_out) r = n_out;
   for (int64_t w = w0; w < w1; ++w)
@@ -332,7 +347,7 @@ __global__ void __launch_bounds__(256)
 // there.  row_old: range_row0 of the first split; row_new: that of the second.
 __global__ void __launch_bounds__(256)
     split_rebalance_kernel(const int32_t *__restrict__ fine_segs, int K, int64_t nb,
-                           int64_t n_out, int T, int n_wg, int granule,
+                           int64_t n_out, int T, int n_wg, int granule, int blk,
                            const int32_t *__restrict__ row_old,
                            const int32_t *__restrict__ range_grp, int32_t *__restrict__ row_new) {
   __shared__ int row_s[kMaxRanges + 1];
@@ -342,7 +357,7 @@ __global__ void __launch_bounds__(256)
   auto work_below = [&](int64_t cell) -> double {
     int64_t below = 0;
     for (int k = 0; k < K; ++k) below += fine_segs[cell * K + k];
-    return (double)split_work(below, cell, n_out, T, K, granule);
+    return (double)split_work(below, cell, n_out, T, K, granule, blk);
   };
   for (int w = threadIdx.x; w <= n_wg; w += blockDim.x) {  // n_wg ranges, <= kMaxRanges
     int r = row_old[w];
@@ -559,7 +574,7 @@ __global__ void __launch_bounds__(256)
                               int64_t pair_stride, int plane_s,
                               const int32_t *__restrict__ pair_num, int K,
                               const int32_t *__restrict__ range_row0, int n_rng, int T,
-                              int window, int n_out, int32_t *__restrict__ wg_tile, int32_t *__restrict__ tile_row0,
+                              int window, int n_out, int blk, int32_t *__restrict__ wg_tile, int32_t *__restrict__ tile_row0,
                               int32_t *__restrict__ n_tiles_dev, int32_t *__restrict__ spill_end,
                               int32_t *__restrict__ tile_slot0, int32_t *__restrict__ segs,
                               int32_t *__restrict__ spill) {
@@ -571,7 +586,7 @@ __global__ void __launch_bounds__(256)
   const int k = blockIdx.y;
   const int64_t j0 = (int64_t)blockIdx.x * CHUNK;
   const int32_t *s = pairs + ((int64_t)k * 2 + plane_s) * pair_stride;
-  constexpr int kPer = LDSROWS ? (CHUNK + 15 + 255) / 256 : 1;
+  constexpr int kPer = LDSROWS ? (CHUNK + 63 + 255) / 256 : 1;
   int held[kPer];
   if constexpr (LDSROWS) {
 #pragma unroll
@@ -634,9 +649,9 @@ __global__ void __launch_bounds__(256)
       }
     }
   }
-  // the block's run of the offset's pairs: their rows (and those of the 15 pairs behind
+  // the block's run of the offset's pairs: their rows (and those of the 63 pairs behind
   // them, for the spill) in LDS
-  __shared__ int rows[LDSROWS ? CHUNK + 16 : 1];
+  __shared__ int rows[LDSROWS ? CHUNK + 64 : 1];
   if (n == 0) {  // no pair: every tile's segment is empty
     if (blockIdx.x == 0)
       for (int t = threadIdx.x; t <= n_tiles; t += 256) {
@@ -653,7 +668,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
       const int i = threadIdx.x + 256 * u;
-      if (i < CHUNK + 15) rows[i] = j0 + i < n ? held[u] : 0x7FFFFFFF;
+      if (i < CHUNK + 63) rows[i] = j0 + i < n ? held[u] : 0x7FFFFFFF;
     }
     __syncthreads();
     // the tiles whose first row lies in (row of the pair before the run, row of its last pair]
@@ -667,9 +682,12 @@ __global__ void __launch_bounds__(256)
         if (rows[mid] < tl.row0) lo = mid + 1;
         else hi = mid;
       }
-      int beyond = 0;
-#pragma unroll
-      for (int q = 0; q < 15; ++q) beyond += rows[lo + q] < tl.spill ? 1 : 0;  // rows ascend
+      int beyond = 0, most = blk - 1;
+      while (beyond < most) {  // rows ascend
+        const int mid = (beyond + most) >> 1;
+        if (rows[lo + mid] < tl.spill) beyond = mid + 1;
+        else most = mid;
+      }
       segs[(int64_t)t * K + k] = (int32_t)(j0 + lo);
       spill[(int64_t)t * K + k] = (int32_t)(j0 + lo + beyond);
     }
@@ -693,8 +711,12 @@ __global__ void __launch_bounds__(256)
         lo += f * step;
         len = (f + 1) * step < len ? step : len - f * step;
       }
-      const bool in_spill = sub < 15 && row_at(lo + sub) < tl.spill;
-      const int beyond = __popc((unsigned)(__ballot(in_spill) >> shift) & 0xFFFFu);
+      const bool in_spill = sub < blk - 1 && row_at(lo + sub) < tl.spill;
+      int beyond = __popc((unsigned)(__ballot(in_spill) >> shift) & 0xFFFFu);
+      for (int q = 16; q < blk; q += 16) {
+        const bool more = sub + q < blk - 1 && row_at(lo + q + sub) < tl.spill;
+        beyond += __popc((unsigned)(__ballot(more) >> shift) & 0xFFFFu);
+      }
       if (sub == 0) {
         segs[(int64_t)t * K + k] = (int32_t)(j0 + lo);
         spill[(int64_t)t * K + k] = (int32_t)(j0 + lo + beyond);
@@ -753,7 +775,7 @@ struct SchedFill {
   const int32_t *tile_row0, *tile_slot0;
   int T;
   uint32_t in_scale, in_pad;
-  int out_scale, k_scale;
+  int out_scale, k_scale, blk;
   int32_t *sched_in, *sched_out, *grp_meta;
 };
 
@@ -795,7 +817,7 @@ __device__ __forceinline__ void sched_fill_item(const SchedFill &f, int64_t t, i
   // rows a tile touches span less than T, so one conditional subtraction does it
   const int slot_off = first ? first[9] - first[8] : tile_slot0[t] - tile_row0[t];
   // four row blocks at a time: their loads are issued together
-  const int n16 = (n + 15) & ~15;
+  const int n16 = (n + f.blk - 1) & -f.blk;  // (a block's row blocks beyond its pairs: padding)
   for (int p0 = lane; p0 < n16; p0 += 64, mb += 4) {
     int gi[4], so[4];
 #pragma unroll
@@ -869,7 +891,7 @@ __device__ __forceinline__ void range_sched_steps(
         if (t < t1) {
           int e = s;
           if (q[u] > s) {
-            e = s + ((q[u] - s + 15) & ~15);
+            e = s + ((q[u] - s + fill.blk - 1) & -fill.blk);
             if (e > lim[u]) e = lim[u];
           }
           sf[item(t, k)] = s;
@@ -886,7 +908,7 @@ __device__ __forceinline__ void range_sched_steps(
     int run = 0;
     for (int k0 = 0; k0 < K; k0 += 64) {
       const int k = k0 + lane;
-      const int nb = k < K ? (sc[item(t, k)] + 15) >> 4 : 0;
+      const int nb = k < K ? ((sc[item(t, k)] + fill.blk - 1) & -fill.blk) >> 4 : 0;
       int incl = nb;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) {
@@ -898,8 +920,10 @@ __device__ __forceinline__ void range_sched_steps(
     }
     if (lane == 0) {
       tn[tile(t)] = run;
-      const int groups = (run + 3) >> 2;
-      tl[tile(t)] = groups > 0 ? groups : 1;  // a tile without pairs gets an empty group
+      // (blocks of 64 pairs: an even number; a tile without pairs gets empty groups)
+      const int gs = fill.blk == 64 ? 2 : 1;
+      const int groups = ((run + 3) >> 2) + gs - 1 & -gs;
+      tl[tile(t)] = groups > 0 ? groups : gs;
     }
   }
   __threadfence_block();
@@ -1078,7 +1102,7 @@ __global__ void __launch_bounds__(256)
                       const int32_t *__restrict__ n_tiles_dev,
                       const int32_t *__restrict__ tile_row0,
                       const int32_t *__restrict__ tile_slot0, int T, uint32_t in_scale,
-                      uint32_t in_pad, int out_scale, int k_scale,
+                      uint32_t in_pad, int out_scale, int k_scale, int blk,
                       int32_t *__restrict__ sched_in, int32_t *__restrict__ sched_out,
                       int32_t *__restrict__ grp_meta) {
   // groups before every range (n_wg <= 256 of them): exclusive prefix of range_grp, which
@@ -1124,25 +1148,26 @@ __global__ void __launch_bounds__(256)
   const int64_t g1 = (t + 1 < n_tiles && tile_rng[t + 1] == rng) ? rg0 + tile_loc[t + 1]
                                                                 : rg0 + range_grp[rng];
   SchedFill f = {pairs, sorted, flag, pair_stride, plane_g, tile_row0, tile_slot0, T, in_scale,
-                 in_pad, out_scale, k_scale, sched_in, sched_out, grp_meta};
+                 in_pad, out_scale, k_scale, blk, sched_in, sched_out, grp_meta};
   sched_fill_item(f, t, k, lane, g0, g1, share_first[t * K + k], share_cnt[t * K + k],
                   kofs[t * K + k], tile_nmb[t]);
 }
 
 
-static size_t conv_lds_bytes(int T, int acc_cols) {
-  return ((size_t)(T + 1) * (acc_cols + 4) + 2 * (size_t)kStage * kAStride) * 4;
+static size_t conv_lds_bytes(int T, int acc_cols, int blk) {
+  const size_t staged = blk > 16 ? parts_staged_bytes(blk) : 2 * (size_t)kStage * kAStride * 4;
+  return (size_t)(T + 1) * (acc_cols + 4) * 4 + staged;
 }
 
 constexpr size_t kLdsLeft = 4096 + 256;
-static int pick_tile(int acc_cols, bool leave_room) {
+static int pick_tile(int acc_cols, int blk, bool leave_room) {
   // One workgroup per CU: (almost) all of the 160 KB of LDS goes to the accumulators.
   // (kLdsLeft bytes stay free: the kernels of the index work -- rulebooks and plans of other
   // layers, queued on a stream of their own -- are built to fit there, beside this kernel's
   // workgroups)
   // (... unless the kernel will run for long: the index work of a neighbouring layer is
   // small change next to it, and the rows of the window are worth more)
-  size_t budget = 160 * 1024 - conv_lds_bytes(0, acc_cols) - (leave_room ? kLdsLeft : 512);
+  size_t budget = 160 * 1024 - conv_lds_bytes(0, acc_cols, blk) - (leave_room ? kLdsLeft : 512);
   int t = (int)(budget / ((size_t)(acc_cols + 4) * 4));
   t = t / 8 * 8;
   if (t < kMinTile) t = kMinTile;
@@ -1177,7 +1202,19 @@ static bool g_conv_fuse_fill = true;  // range_sched_kernel<true> instead of sch
 static thread_local bool g_index_beside_conv = false;  // (a setting of the calling host thread)
 static bool g_conv_rebalance = true;  // long kernels: a second work split from the first one's counts
 static bool g_conv_round8 = false;    // ranges per column block: a multiple of 8 only
+static int g_conv_parts_blk = 0;      // ... with blocks of 32 or 64 pairs wherever it can be
+static bool g_conv_parts = true;      // the bfloat16-parts form
 static bool g_conv_small = true;      // layers of at most 8 input channels: conv_small_kernel
+
+// groups: pairs/64 plus, per (tile, offset), up to one partial block (of blk pairs), plus one
+// partial (or empty) group per tile, or two, plus the groups the kernel's prefetches may
+// touch beyond the end of the schedule
+static int64_t plan_groups(int64_t n_tiles, int64_t n_out, int K, int64_t pair_stride, int blk) {
+  const int64_t max_pairs_k = pair_stride < n_out ? pair_stride : n_out;
+  const int64_t per = blk / 16;
+  return ((int64_t)K * (max_pairs_k / 16 + per) + n_tiles * K * per) / 4 + (blk == 64 ? 3 : 2) * n_tiles +
+         4 + 16;
+}
 
 // The sizes that follow from the number of workgroups per column block.
 // `sizing`: the plan is only being sized (the number of input rows, and with it the number
@@ -1192,15 +1229,46 @@ static void plan_split(ConvPlan &p, int n_wg, int n_rng, int64_t n_out, int K,
   p.granule = sizing || n_out / n_rng < 2048 ? kSplitGranuleSmall : kSplitGranule;
   p.n_fine = ceil_div(n_out > 0 ? n_out : 1, p.granule);
   p.words_per_k = ceil_div(n_out > 0 ? n_out : 1, 32);
-  // groups: pairs/64 plus, per (tile, offset), up to one partial block, plus one
-  // partial (or empty) group per tile, plus the groups the kernel's prefetches may
-  // touch beyond the end of the schedule
-  int64_t max_pairs_k = pair_stride < n_out ? pair_stride : n_out;
-  p.grp_cap = ((int64_t)K * (max_pairs_k / 16 + 1) + p.n_tiles * K) / 4 + 2 * p.n_tiles + 4 + 16;
+  p.grp_cap = plan_groups(p.n_tiles, n_out, K, pair_stride, p.blk);
 }
 
+// Pairs of an offset to a block of the parts form for a convolution of n_out rows over n_wg
+// workgroups and tiles of tile32 / tile64 rows, 0: the float form.  What decides is how many pairs
+// an offset has in a tile (each offset's last block of a tile is padded), which the rows and the
+// kind of the rulebook tell: a convolution of unit stride pairs nearly every input row with
+// an output row under every offset, a strided one an eighth of them (stride 2).  Microseconds of
+// the kernel, float form / blocks of 32 / of 64, 3^3 offsets:
+//    pairs of an offset in a tile                                     channels
+//     11  (unit, gradient)  22 / 30 / 46       28  (unit)  290 / 338 / 561    64 -> 128
+//     24  (stride 2)        45 / 36 / 47       38  (unit)  158 / 155 / 228    64 -> 304
+//     28  (stride 2)       152 / 120 / 219     55  (unit)  419 / 312 / 452   128 -> 256
+//     35  (stride 2)       239 / 183 / 206     57  (unit)   46 /  39 /  43    64 -> 64
+//     57  (every row)       39 /  31 /  28     88  (stride 2) 1396 / 1057 / 943   128 -> 304
+//    110  (unit)          6880 / 5600 / 4520  216  (every row) 287 / 215 / 189   128 -> 64
+// Of a strided layer an output row has the offsets of its parity only, so that the pairs of a
+// tile bunch; where every row has every offset the blocks but the last one are full.
+constexpr int kPartsMost32 = 10, kPartsMost64 = 4;
+static int parts_block(int64_t n_in, int64_t n_out, int64_t pair_stride, bool unit, int n_wg,
+                       int tile32, int tile64) {
+  const bool inverse = pair_stride == n_out && n_in != n_out;
+  const int64_t rb_in = pair_stride, rb_out = inverse ? n_in : n_out;
+  if (n_out > kPartsMost32 * rb_in) return 0;  // (what buffers are sized for; no rule below comes near)
+  if (rb_out > 4 * rb_in) unit = true;  // (a stride of 2 makes 3.4 rows of one at most)
+  const double fill = std::min(1.0, (unit ? 1.0 : 0.125) * (double)rb_in / (double)n_out);
+  const double rows = (double)n_out / n_wg;
+  const double in32 = fill * std::min(rows, (double)tile32), in64 = fill * std::min(rows, (double)tile64);
+  if (fill >= 0.8 && rows < tile64) {
+    const int64_t whole = (int64_t)in64 + 1;
+    if (whole >= 32 && ceil_div(whole, 64) * 64 * 5 <= ceil_div(whole, 32) * 32 * 6) return 64;
+  } else if (in64 >= 72.0 && n_out <= kPartsMost64 * rb_in) {
+    return 64;
+  }
+  return in32 >= (unit ? 34.0 : 20.0) ? 32 : 0;
+}
+
+// unit: the rulebook is of a convolution of unit stride (SSC_CONV_UNIT_STRIDE).
 static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_out,
-                          int64_t pair_stride, int elem_bytes = 4) {
+                          int64_t pair_stride, int elem_bytes = 4, bool unit = false) {
   ConvPlan p;
   p.ncb = (int)ceil_div(c_out, 16);
   p.nch = (int)ceil_div(c_in, kKC);
@@ -1220,16 +1288,33 @@ static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_ou
   // the five-group form: a lone last group goes along with the last full block (the
   // kernel needs four chunks for it, one for each wave's turn at the fifth group's sums)
   p.five = g_conv_five && elem_bytes == 4 && p.ncb % p.ncw == 1 && p.ncb > p.ncw && p.nch >= 4;
-  p.acc_cols = p.five ? 16 * p.ncw + 16 : 16 * p.ncw;
   // the gather can be a range-checked buffer load when rows are multiples of four
   // channels and byte offsets into the features (plus the padding marker) fit 32 bits
   p.gather = 0;
   if ((c_in & 3) == 0 && (uint64_t)n_in * c_in * elem_bytes <= (uint64_t)kGatherPad)
     p.gather = (c_in % kKC) == 0 ? 1 : 2;
+  // the parts form
+  p.parts_packed = elem_bytes == 4 && p.ns == 16 && c_in > 32 &&
+                   (uint64_t)K * p.ncb * p.nch * (4096 + kPartFragBytes) < ((uint64_t)1 << 32);
+  const bool parts_can = g_conv_parts && p.parts_packed;
+  p.blk = 16;
+  if (parts_can && n_in > 0 && p.gather != 0) {
+    const int cols = (int)ceil_div(p.ncb, p.ncw);
+    const int blk = g_conv_parts_blk > 0
+                        ? g_conv_parts_blk
+                        : parts_block(n_in, n_out, pair_stride, unit,
+                                      std::min(256, std::max(1, device_cu_count() / cols)),
+                                      pick_tile(64, 32, true) - kSpillRowsParts,
+                                      pick_tile(64, 64, true) - kSpillRowsParts);
+    if (blk > 0) p.blk = blk;
+  }
+  p.parts = p.blk > 16;
+  if (p.parts) p.five = false;
+  p.acc_cols = p.five ? 16 * p.ncw + 16 : 16 * p.ncw;
   // (wider layers: the launches of one column block each cost more than the lone group
   // in a block of its own does -- 128 -> 256 channels at stride 2 takes 0.255 ms as four
   // launches against 0.185 ms as one, 200 -> 200 with 125 offsets 17.6 against 16.8 ms)
-  p.has_tail = !p.five && g_conv_tail && elem_bytes == 4 && p.ncb % p.ncw == 1 && p.ncb / p.ncw <= 2;
+  p.has_tail = !p.parts && !p.five && g_conv_tail && elem_bytes == 4 && p.ncb % p.ncw == 1 && p.ncb / p.ncw <= 2;
   const bool serial = p.has_tail || p.five;
   const int blocks = serial ? p.ncb / p.ncw : (int)ceil_div(p.ncb, p.ncw);
   p.n_colblk = serial ? 1 : blocks;
@@ -1261,8 +1346,8 @@ static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_ou
   // they are; layers whose pairs the estimate overstates -- a strided layer with more
   // outputs than inputs -- are short kernels and gain.)
   const bool long_kernel = n_in > 0 && est_stages >= kRebalanceStages;
-  p.T = pick_tile(p.acc_cols, !long_kernel);
-  p.tile_rows = p.T - (p.five ? kSpillRowsFive : kSpillRows);
+  p.T = pick_tile(p.acc_cols, p.blk, !long_kernel);
+  p.tile_rows = p.T - (p.parts ? kSpillRowsParts : p.five ? kSpillRowsFive : kSpillRows);
   // Two ranges to a workgroup, paired by what they came to (range_assign_kernel): one more
   // small launch and one more range end per workgroup, whose last row blocks cannot be
   // filled from a next tile (K / 8 groups), against the 5-10 % by which single ranges
@@ -1272,7 +1357,20 @@ static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_ou
                     (g_conv_pair_always || n_in <= 0 ||
                      (!p.rebalance && est_groups >= kPairGroups && est_groups >= (int64_t)K / 2));
   plan_split(p, n_wg, pair ? 2 * n_wg : n_wg, n_out, K, pair_stride, n_in <= 0);
-  p.lds_bytes = conv_lds_bytes(p.T, p.acc_cols);
+  // (sizing calls: room for the parts form as well, which parts_block takes only where the
+  // outputs are at most so many times the inputs)
+  if (parts_can && n_in <= 0) {
+    for (int blk = 32; blk <= 64; blk *= 2) {
+      const int64_t most = g_conv_parts_blk > 0
+                               ? n_out
+                               : std::min(n_out, (int64_t)(blk == 32 ? kPartsMost32 : kPartsMost64) * pair_stride);
+      const int tile = pick_tile(64, blk, true) - kSpillRowsParts;
+      const int64_t tiles = ceil_div(most > 0 ? most : 1, tile) + p.n_rng;
+      p.n_tiles = std::max(p.n_tiles, tiles);
+      p.grp_cap = std::max(p.grp_cap, plan_groups(tiles, most, K, pair_stride, blk));
+    }
+  }
+  p.lds_bytes = conv_lds_bytes(p.T, p.acc_cols, p.blk);
   p.small = g_conv_small && conv_small_applies(K, c_in, c_out, elem_bytes);
   if (p.small) p.rebalance = false;
   p.kvol = K;
@@ -1281,9 +1379,10 @@ static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_ou
 }
 
 
-// 4 KiB per fragment for either element type (half fragments use the first half).
+// 4 KiB per fragment for either element type (half fragments use the first half), and the
+// fragments in parts for layers that may take that form (room for them whatever the type).
 static size_t conv_packed_bytes(const ConvPlan &p, int K) {
-  return align_up((size_t)K * p.ncb * p.nch * 4096);
+  return align_up((size_t)K * p.ncb * p.nch * (4096 + (p.parts_packed ? kPartFragBytes : 0)));
 }
 
 static size_t conv_plan_walk(void *base, const ConvPlan &p, ConvWs *w) {
@@ -1429,6 +1528,18 @@ static int launch_all(const ConvPlan &p, const ConvWs &w, const IO *features, in
       SSC_CHECK(false, SSC_ERUNTIME, "the five-group form is built for float rows");
     }
   }
+  if constexpr (kFloat && GATHER != 0 && NS == 16) {
+    if (p.blk == 64)
+      return with_epi ? launch_conv_f32<GATHER, 16, true, 5>(p, w, features, n_in, c_in, K, out,
+                                                             c_out, 0, -1, epi, s)
+                      : launch_conv_f32<GATHER, 16, false, 5>(p, w, features, n_in, c_in, K, out,
+                                                              c_out, 0, -1, epi, s);
+    if (p.parts)
+      return with_epi ? launch_conv_f32<GATHER, 16, true, 4>(p, w, features, n_in, c_in, K, out,
+                                                             c_out, 0, -1, epi, s)
+                      : launch_conv_f32<GATHER, 16, false, 4>(p, w, features, n_in, c_in, K, out,
+                                                              c_out, 0, -1, epi, s);
+  }
   for (int l = 0; l < p.n_launch; ++l) {
     const int col_base = l * p.n_colblk * 16 * p.ncw;
     int rc;
@@ -1503,6 +1614,8 @@ int ssc_conv_tuning(int32_t flags) {
   g_conv_pair_always = (flags & 128) != 0;
   g_conv_small = (flags & 256) == 0;
   g_conv_fuse_fill = (flags & 512) == 0;
+  g_conv_parts = (flags & 1024) == 0;
+  g_conv_parts_blk = (flags & 2048) ? 64 : (flags & 4096) ? 32 : 0;
   return SSC_OK;
 }
 
@@ -1562,7 +1675,7 @@ static int conv_plan_build(const ConvPlan &p, const ConvWs &w, const int32_t *pa
                           w.tile_slot0, p.T,
                           p.gather ? (uint32_t)c_in * (uint32_t)elem_bytes : 1u,
                           p.gather ? kGatherPad : 0xFFFFFFFFu, (p.acc_cols + 4) * 4,
-                          p.ncb * p.nch * frag_bytes, w.sched_in, w.sched_out, w.grp_meta};
+                          p.ncb * p.nch * frag_bytes, p.blk, w.sched_in, w.sched_out, w.grp_meta};
   // One range to a workgroup and a single work split: the launch that counts a range's row
   // blocks goes on to fill its schedule (no sched_fill_kernel).
   // (not for index work queued beside a running convolution: there two small kernels that
@@ -1588,14 +1701,14 @@ static int conv_plan_build(const ConvPlan &p, const ConvWs &w, const int32_t *pa
     hipLaunchKernelGGL(segments_kernel, dim3((unsigned)ceil_div(pair_stride, kSegChunk), (unsigned)K), dim3(256),
                        2 * ((size_t)p.n_rng + 1) * sizeof(int), s,
                        w.flag, pairs, pair_stride, plane_s, pair_num, K, w.range_row0, p.n_rng,
-                       p.tile_rows, p.T, (int)n_out, w.wg_tile, w.tile_row0, w.n_tiles_dev,
+                       p.tile_rows, p.T, (int)n_out, p.blk, w.wg_tile, w.tile_row0, w.n_tiles_dev,
                        w.spill_end, w.tile_slot0, w.segs, w.spill);
     SSC_LAUNCH_CHECK("pair_tile_segments");
     if ((rc = range_sched()) != SSC_OK) return rc;
     if (fuse_fill) return SSC_OK;
   }
   const int64_t packed_n = pack ? (int64_t)K * p.ncb * p.nch * 1024 : 0;
-  PackArgs pk = {nullptr, 0, 0, 0, 0, 0, 0, 0, 0, nullptr, 16};
+  PackArgs pk = {nullptr, 0, 0, 0, 0, 0, 0, 0, 0, nullptr, 16, 0};
   if (pack) pk = *pack;
   if (!in_order && !seeded) {  // otherwise the filters are packed beside the first kernel of the split
     if (pack) {
@@ -1650,7 +1763,7 @@ static int conv_plan_build(const ConvPlan &p, const ConvWs &w, const int32_t *pa
                        p.n_fine, p.granule, w.fine_segs, pk);
     hipLaunchKernelGGL(split_bounds_kernel, dim3((unsigned)ceil_div(p.n_fine + 1, 256)), dim3(256),
                        0, s, w.fine_segs, K, p.n_fine, n_out, p.tile_rows, p.n_rng, p.granule,
-                       w.range_row0);
+                       p.blk, w.range_row0);
   }
   // the ranges' tiles, their segments, shares and row-block counts
   const int64_t nseg = (p.n_tiles + 1) * K;
@@ -1661,8 +1774,8 @@ static int conv_plan_build(const ConvPlan &p, const ConvWs &w, const int32_t *pa
     SSC_LAUNCH_CHECK("split");
     hipLaunchKernelGGL(tile_segments_kernel, dim3((unsigned)ceil_div(nseg, 256)), dim3(256), 0, s,
                        w.flag, pairs, w.sorted, pair_stride, plane_s, pair_num, K, w.n_tiles_dev,
-                       w.tile_row0, n_out, w.fine_segs, p.granule, w.spill_end, w.segs,
-                       w.spill);
+                       w.tile_row0, n_out, w.fine_segs, p.granule, w.spill_end, p.blk,
+                       w.segs, w.spill);
     SSC_LAUNCH_CHECK("tile_segments");
     return range_sched();
   };
@@ -1672,7 +1785,7 @@ static int conv_plan_build(const ConvPlan &p, const ConvWs &w, const int32_t *pa
   if (p.rebalance) {  // long kernels: once more, from the groups the ranges came to
     hipLaunchKernelGGL(split_rebalance_kernel, dim3((unsigned)ceil_div(p.n_fine + 1, 256)),
                        dim3(256), 0, s, w.fine_segs, K, p.n_fine, n_out, p.tile_rows, p.n_rng,
-                       p.granule, w.range_row0, w.range_grp, w.range_row1);
+                       p.granule, p.blk, w.range_row0, w.range_grp, w.range_row1);
     SSC_LAUNCH_CHECK("split_rebalance");
     rc = tiles_of(w.range_row1);
     if (rc != SSC_OK) return rc;
@@ -1691,7 +1804,7 @@ static int conv_plan_build(const ConvPlan &p, const ConvWs &w, const int32_t *pa
                      w.tile_slot0, p.T,
                      p.gather ? (uint32_t)c_in * (uint32_t)elem_bytes : 1u,
                      p.gather ? kGatherPad : 0xFFFFFFFFu, (p.acc_cols + 4) * 4,
-                     p.ncb * p.nch * frag_bytes, w.sched_in, w.sched_out, w.grp_meta);
+                     p.ncb * p.nch * frag_bytes, p.blk, w.sched_in, w.sched_out, w.grp_meta);
   SSC_LAUNCH_CHECK("schedule");
   return SSC_OK;
 }
@@ -1758,6 +1871,12 @@ static int conv_check_sizes(int K, int c_in, int c_out, int64_t n_in, int64_t n_
   return SSC_OK;
 }
 
+// SSC_CONV_UNIT_STRIDE rides on the kernel volume (or on the element size).
+static int strip_unit(int v, bool *unit) {
+  *unit = v > 0 && (v & SSC_CONV_UNIT_STRIDE) != 0;
+  return *unit ? v & ~SSC_CONV_UNIT_STRIDE : v;
+}
+
 // The forward convolution for features, filters and output of element type IO.
 template <typename IO>
 static int conv_fwd(const IO *features, int64_t n_in, int32_t c_in, const IO *filters,
@@ -1765,7 +1884,8 @@ static int conv_fwd(const IO *features, int64_t n_in, int32_t c_in, const IO *fi
                     const int32_t *pairs, int64_t pair_stride, const int32_t *pair_num,
                     int32_t kernel_volume, int32_t inverse, int32_t subm, IO *out, int64_t n_out,
                     void *workspace, size_t workspace_bytes, ssc_stream_t stream) {
-  const int K = kernel_volume;
+  bool unit;
+  const int K = strip_unit(kernel_volume, &unit);
   int rc = conv_check_sizes(K, c_in, c_out, n_in, n_out, pair_stride);
   if (rc != SSC_OK) return rc;
   if (n_out == 0) return SSC_OK;
@@ -1778,10 +1898,10 @@ static int conv_fwd(const IO *features, int64_t n_in, int32_t c_in, const IO *fi
   SSC_CHECK(workspace_bytes >= need, SSC_EWORKSPACE, "conv workspace too small: %zu < %zu",
             workspace_bytes, need);
 
-  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, (int)sizeof(IO));
+  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, (int)sizeof(IO), unit);
   ConvWs w;
   conv_ws_walk(workspace, p, K, pair_stride, &w);
-  const PackArgs pack = {filters, fs_k, fs_ci, fs_co, K, c_in, c_out, p.ncb, p.nch, w.packed, p.ns};
+  const PackArgs pack = {filters, fs_k, fs_ci, fs_co, K, c_in, c_out, p.ncb, p.nch, w.packed, p.ns, p.parts_packed};
   const bool in_order = (subm & SSC_CONV_PAIRS_CANONICAL) != 0;
   rc = conv_plan_build<IO>(p, w, pairs, pair_stride, pair_num, K, inverse, in_order, c_in, n_out,
                            (int)sizeof(IO), &pack, s);
@@ -1799,7 +1919,7 @@ static int conv_pack(const IO *filters, int64_t fs_k, int64_t fs_ci, int64_t fs_
   SSC_CHECK(packed_bytes >= conv_packed_bytes(p, K), SSC_EWORKSPACE,
             "buffer of the packed filters too small: %zu < %zu", packed_bytes,
             conv_packed_bytes(p, K));
-  const PackArgs pack = {filters, fs_k, fs_ci, fs_co, K, c_in, c_out, p.ncb, p.nch, packed, p.ns};
+  const PackArgs pack = {filters, fs_k, fs_ci, fs_co, K, c_in, c_out, p.ncb, p.nch, packed, p.ns, p.parts_packed};
   const int64_t packed_n = (int64_t)K * p.ncb * p.nch * 1024;
   hipLaunchKernelGGL(pack_filters_kernel<IO>, dim3((unsigned)ceil_div(packed_n, 256)), dim3(256), 0,
                      s, pack, (int32_t *)nullptr);
@@ -1810,14 +1930,16 @@ static int conv_pack(const IO *filters, int64_t fs_k, int64_t fs_ci, int64_t fs_
 template <typename IO>
 static int conv_planned(const IO *features, int64_t n_in, int32_t c_in, const void *packed,
                         size_t packed_bytes, const void *plan, size_t plan_bytes, int64_t pair_stride,
-                        int32_t K, int32_t c_out, IO *out, int64_t n_out, hipStream_t s) {
+                        int32_t kernel_volume, int32_t c_out, IO *out, int64_t n_out, hipStream_t s) {
+  bool unit;
+  const int K = strip_unit(kernel_volume, &unit);
   int rc = conv_check_sizes(K, c_in, c_out, n_in, n_out, pair_stride);
   if (rc != SSC_OK) return rc;
   if (n_out == 0) return SSC_OK;
   SSC_CHECK(out != nullptr, SSC_EINVAL, "out is NULL");
   if (pair_stride == 0 || n_in == 0) return fill_zero(out, n_out * c_out, s);
   SSC_CHECK(features && packed && plan, SSC_EINVAL, "NULL pointer argument");
-  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, (int)sizeof(IO));
+  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, (int)sizeof(IO), unit);
   SSC_CHECK(packed_bytes >= conv_packed_bytes(p, K), SSC_EWORKSPACE,
             "buffer of the packed filters too small");
   SSC_CHECK(plan_bytes >= conv_plan_walk(nullptr, p, nullptr), SSC_EWORKSPACE,
@@ -1832,9 +1954,11 @@ static int conv_planned(const IO *features, int64_t n_in, int32_t c_in, const vo
 template <typename IO>
 static int conv_planned_epilogue(const IO *features, int64_t n_in, int32_t c_in,
                                  const void *packed, size_t packed_bytes, const void *plan,
-                                 size_t plan_bytes, int64_t pair_stride, int32_t K, int32_t c_cols,
-                                 const ssc_conv_epilogue *e, IO *out, int64_t n_out,
-                                 hipStream_t s) {
+                                 size_t plan_bytes, int64_t pair_stride, int32_t kernel_volume,
+                                 int32_t c_cols, const ssc_conv_epilogue *e, IO *out,
+                                 int64_t n_out, hipStream_t s) {
+  bool unit;
+  const int K = strip_unit(kernel_volume, &unit);
   int rc = conv_check_sizes(K, c_in, c_cols, n_in, n_out, pair_stride);
   if (rc != SSC_OK) return rc;
   SSC_CHECK(e != nullptr, SSC_EINVAL, "epilogue is NULL");
@@ -1850,7 +1974,7 @@ static int conv_planned_epilogue(const IO *features, int64_t n_in, int32_t c_in,
   SSC_CHECK(e->shift && e->scale && e->add && e->pre_bias && e->mode && e->gate && e->dest &&
                 e->gate_run,
             SSC_EINVAL, "NULL table in the epilogue");
-  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_cols, pair_stride, (int)sizeof(IO));
+  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_cols, pair_stride, (int)sizeof(IO), unit);
   SSC_CHECK(packed_bytes >= conv_packed_bytes(p, K), SSC_EWORKSPACE,
             "buffer of the packed filters too small");
   SSC_CHECK(plan_bytes >= conv_plan_walk(nullptr, p, nullptr), SSC_EWORKSPACE,
@@ -1954,13 +2078,14 @@ int ssc_conv_plan_build(const int32_t *pairs, int64_t pair_stride, const int32_t
                         int64_t n_out, int32_t c_in, int32_t c_out, int32_t elem_bytes, void *plan,
                         size_t plan_bytes, void *scratch, size_t scratch_bytes,
                         ssc_stream_t stream) {
-  const int K = kernel_volume;
+  bool unit;
+  const int K = strip_unit(kernel_volume, &unit);
   int rc = conv_check_sizes(K, c_in, c_out, n_in, n_out, pair_stride);
   if (rc != SSC_OK) return rc;
   SSC_CHECK(elem_bytes == 4 || elem_bytes == 2, SSC_EINVAL, "elem_bytes must be 4 or 2");
   if (n_out == 0 || pair_stride == 0 || n_in == 0) return SSC_OK;  // nothing to schedule
   SSC_CHECK(pairs && pair_num && plan && scratch, SSC_EINVAL, "NULL pointer argument");
-  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, elem_bytes);
+  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, elem_bytes, unit);
   SSC_CHECK(plan_bytes >= conv_plan_walk(nullptr, p, nullptr), SSC_EWORKSPACE,
             "plan buffer too small");
   SSC_CHECK(scratch_bytes >= conv_scratch_walk(nullptr, p, K, pair_stride, nullptr),
@@ -1986,7 +2111,7 @@ static int combine_job_of(const float *weight, const float *basis, const int32_t
   const ConvPlan p = make_plan(0, 1, K, c_in, c_out, 0, 4);
   SSC_CHECK(packed_bytes >= conv_packed_bytes(p, K), SSC_EWORKSPACE,
             "buffer of the packed filters too small");
-  job->pk = PackArgs{nullptr, 0, 0, 0, K, c_in, c_out, p.ncb, p.nch, packed, p.ns};
+  job->pk = PackArgs{nullptr, 0, 0, 0, K, c_in, c_out, p.ncb, p.nch, packed, p.ns, p.parts_packed};
   job->weight = weight;
   job->basis = basis;
   job->chan_out = chan_out;
@@ -2017,6 +2142,8 @@ int ssc_rulebook_conv_begin(const int32_t *indices, int64_t n_in, const ssc_geom
   g_pending_layer = PendingLayer();
   SSC_CHECK(g != nullptr, SSC_EINVAL, "geometry is NULL");
   SSC_CHECK(c_in >= 1 && c_out >= 1, SSC_EINVAL, "channel counts must be positive");
+  bool unit;
+  elem_bytes = strip_unit(elem_bytes, &unit);
   SSC_CHECK(elem_bytes == 4 || elem_bytes == 2, SSC_EINVAL, "elem_bytes must be 4 or 2");
   CombineJob job = {};
   if (filters != nullptr) {
@@ -2038,9 +2165,11 @@ int ssc_rulebook_conv_begin(const int32_t *indices, int64_t n_in, const ssc_geom
     for (int a = 0; a < 3; ++a) strided = strided || g->stride[a] != 1 || g->dilation[a] != 1;
     ConvWs w = {};
     const size_t head = conv_scratch_head(scratch, &w);
-    const ConvPlan more = make_plan(n_in, n_in + 1, (int)K, c_in, c_out, n_in, elem_bytes);
+    // (the form depends on the number of outputs as well, and with it the number of ranges of
+    // layers with a lone last column group: the guess is a scattered cloud's)
+    const ConvPlan more = make_plan(n_in, 10 * n_in + 1, (int)K, c_in, c_out, n_in, elem_bytes, unit);
     const ConvPlan fewer =
-        make_plan(n_in, n_in > 1 ? n_in - 1 : 1, (int)K, c_in, c_out, n_in, elem_bytes);
+        make_plan(n_in, n_in > 1 ? n_in - 1 : 1, (int)K, c_in, c_out, n_in, elem_bytes, unit);
     const bool more_ok = !more.rebalance && !more.small;
     const bool fewer_ok = strided && n_in > 1 && !fewer.rebalance && !fewer.small &&
                           !(more_ok && fewer.n_rng == more.n_rng &&
@@ -2049,7 +2178,7 @@ int ssc_rulebook_conv_begin(const int32_t *indices, int64_t n_in, const ssc_geom
       const ConvPlan &first = more_ok ? more : fewer;
       rq.n_rng = first.n_rng;
       rq.tile_rows = first.tile_rows;
-      rq.tile_cost = (long long)K * 4 + 64;  // split_tile_cost
+      rq.tile_cost = split_tile_cost((int)K, first.blk);
       rq.range_row0 = w.range_row0;
       if (more_ok && fewer_ok) {
         rq.n_rng_alt = fewer.n_rng;
@@ -2081,6 +2210,8 @@ int ssc_rulebook_conv_finish(const ssc_geometry *g, int64_t n_in, int32_t *n_out
   g_pending_layer = PendingLayer();
   int rc = ssc_rulebook_finish(g, n_in, n_out_host, in_order_host);
   if (rc != SSC_OK) return rc;
+  bool unit;
+  elem_bytes = strip_unit(elem_bytes, &unit);
   const int64_t n_out = *n_out_host;
   int K = 1;
   for (int a = 0; a < 3; ++a) K *= g->ksize[a];
@@ -2089,7 +2220,7 @@ int ssc_rulebook_conv_finish(const ssc_geometry *g, int64_t n_in, int32_t *n_out
   SSC_CHECK(elem_bytes == 4 || elem_bytes == 2, SSC_EINVAL, "elem_bytes must be 4 or 2");
   if (n_out == 0 || n_in == 0) return SSC_OK;  // nothing to schedule
   SSC_CHECK(pairs && pair_num && plan && scratch, SSC_EINVAL, "NULL pointer argument");
-  const ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, n_in, elem_bytes);
+  const ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, n_in, elem_bytes, unit);
   SSC_CHECK(plan_bytes >= conv_plan_walk(nullptr, p, nullptr), SSC_EWORKSPACE,
             "plan buffer too small");
   SSC_CHECK(scratch_bytes >= conv_scratch_walk(nullptr, p, K, n_in, nullptr), SSC_EWORKSPACE,

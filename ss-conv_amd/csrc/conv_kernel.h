@@ -1,11 +1,13 @@
 // The convolution kernel (conv_fwd_kernel), what a launch of it needs to know of a plan,
-// and the launch itself.  Eight translation units instantiate it: conv.hip the plain form
+// and the launch itself.  Ten translation units instantiate it: conv.hip the plain form
 // (float and half rows), conv_epi.hip the one with the epilogue, conv_tail.hip and
 // conv_tail_epi.hip the one-column-group form without and with it, conv_five.hip and
 // conv_five_epi.hip the five-group form, conv_wide.hip and conv_wide_epi.hip the plain
-// kernel over plans of the five-group form -- compiled side by side, the parts of the
-// instances take a third of the time.
+// kernel over plans of the five-group form, conv_parts.hip and conv_parts_epi.hip the
+// bfloat16-parts form -- compiled side by side, the parts of the instances take a third of
+// the time.
 #pragma once
+#include "conv_pack.h"
 #include "ssc_common.h"
 
 #include <type_traits>
@@ -181,9 +183,74 @@ struct ConvEpilogue {
   int act_s, act_g, c_dest;
 };
 
+// ---- bfloat16 parts ---------------------------------------------------------------------
+// An element of a float matrix as three bfloat16 parts that add up to it: the element rounded,
+// what is left rounded, and the rest.  The matrix cores multiply bfloat16 sixteen times as fast
+// as floats; of the nine products of parts six are taken (the ones left out are below 2^-24 of
+// the product).
+// What the parts cannot do (PartsCheck::odd) and what then happens: see the parts form below.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+struct PartsCheck {
+  float nan;       // NaN once a sum was not finite (0 times it is NaN)
+  uint32_t least;  // smallest magnitude of a sum that is not zero: (bits << 1) - 1
+  uint32_t rest;   // OR of the words of which third parts were made
+  __device__ __forceinline__ void sum(float v) {
+    least = min(least, (__builtin_bit_cast(uint32_t, v) << 1) - 1u);
+    nan = __builtin_fmaf(v, 0.f, nan);
+  }
+  __device__ __forceinline__ bool odd() const {
+    return nan != 0.f || (rest & 0xFFFFu) != 0 || least < ((127u - 95u) << 24) - 1u;
+  }
+};
+// Two elements' parts, each pair of parts packed into a word.  (What a part leaves by the dot
+// product of a bfloat16 pair: it holds the matrix cores up for its time, which shift, mask and
+// subtraction do not -- 48 matrix instructions of a wave beside 112 others of another one: 812
+// cycles alone, 1392 with dot products, 900 with subtractions -- but those are twice as many, and
+// the kernel is 2 % slower with them.)
+struct PartsCut {
+  bf16x2 m0, m1;  // (-1, 0) and (0, -1)
+  __device__ __forceinline__ PartsCut() {
+    // (in registers: as literals they would be packed into one half of the operand, which the
+    // instruction reads twice)
+    uint32_t minus0 = 0x0000BF80u, minus1 = 0xBF800000u;
+    asm volatile("" : "+s"(minus0), "+s"(minus1));
+    m0 = __builtin_bit_cast(bf16x2, minus0);
+    m1 = __builtin_bit_cast(bf16x2, minus1);
+  }
+  __device__ __forceinline__ void two(float u, float v, int &hi, int &mid, int &lo,
+                                      uint32_t &rest) const {
+    const bf16x2 a = __builtin_convertvector(float2v{u, v}, bf16x2);
+    hi = __builtin_bit_cast(int, a);
+    u = __builtin_amdgcn_fdot2_f32_bf16(a, m0, u, false);
+    v = __builtin_amdgcn_fdot2_f32_bf16(a, m1, v, false);
+    const bf16x2 b = __builtin_convertvector(float2v{u, v}, bf16x2);
+    mid = __builtin_bit_cast(int, b);
+    u = __builtin_amdgcn_fdot2_f32_bf16(b, m0, u, false);
+    v = __builtin_amdgcn_fdot2_f32_bf16(b, m1, v, false);
+    rest |= __builtin_bit_cast(uint32_t, u) | __builtin_bit_cast(uint32_t, v);
+    lo = __builtin_bit_cast(int, __builtin_convertvector(float2v{u, v}, bf16x2));
+  }
+};
+// Staged rows in LDS: two stages of 2 blk pairs x 32 channels x 3 parts (blk: pairs to a block).
+inline size_t parts_staged_bytes(int blk) { return 2 * (size_t)(2 * blk) * 192 + 16; }
+// Position in the schedule of the parts form: group and chunk of 64 channels.  The last group
+// repeats: what is fetched ahead of a workgroup's end is its last group again.
+struct PartsPos {
+  int g, cc;
+  __device__ __forceinline__ void advance(int gs, int nch, int g_last) {  // gs: groups to a stage
+    ++cc;
+    if (cc == nch) {
+      cc = 0;
+      g = g < g_last ? g + gs : g_last;
+    }
+  }
+};
+
 // FORM: 0 the kernel as described above; 1 the one-column-group form; 2 the five-group form
 // (see the consumers); 3 the plain kernel on a plan of the five-group form, whose accumulator
-// rows are 16 columns wider (the launches of such a plan that have no fifth group).
+// rows are 16 columns wider (the launches of such a plan that have no fifth group); 4 and 5 the
+// bfloat16-parts form, over blocks of 32 and of 64 pairs.
 template <typename IO, int GATHER, int NCW, int NS, bool EPI, int FORM>
 __global__ void __launch_bounds__((NCW + 4) * 64)
     __attribute__((amdgpu_waves_per_eu((NCW + 4) / 4, (NCW + 4) / 4)))
@@ -194,7 +261,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
                     const int32_t *__restrict__ wg_grp,
                     int nch, int ncb, IO *__restrict__ out, int cout, int T, int cols_per_xcd,
                     int col_base, int xcol, ConvEpilogue epi) {
-  constexpr bool TAIL = FORM == 1, FIVE = FORM == 2, WIDE = FORM == 3;
+  constexpr bool TAIL = FORM == 1, FIVE = FORM == 2, WIDE = FORM == 3,
+                 PARTS = FORM == 4 || FORM == 5;
   constexpr int kCN = 16 * NCW;   // output columns per workgroup
   constexpr int kEB = Io<IO>::kBytes;
   constexpr bool kHalf = kEB == 2;
@@ -208,6 +276,10 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
   // accumulator row stride in floats (the five-group form: 16 more columns)
   constexpr int kAS = kCN + (FIVE || WIDE ? 16 : 0) + 4;
   constexpr int NT = (NCW + 4) * 64;
+  // threads that write a tile out (the parts form over blocks of 64 with the epilogue: the
+  // consumers only, the producers have no registers for it)
+  constexpr bool kProducersFlush = !(EPI && FORM == 5);
+  constexpr int NTF = kProducersFlush ? NT : NCW * 64;
   constexpr int NP = 256;  // producer threads
   constexpr int NE = kStage * 16 / NP;
   extern __shared__ __align__(16) float lds[];
@@ -259,6 +331,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
   const int nstages = (g_end - g_begin) * nch;  // stages of this workgroup
   const int col0 = col_base + cblk * kCN;
   static_assert(FORM == 0 || (NCW == 4 && !kHalf), "the other forms are built for float");
+  static_assert(!PARTS || (NS == 16 && GATHER != 0), "the parts form: whole chunks, buffer loads");
+  PartsCheck check = {0.f, 0xFFFFFFFFu, 0u};  // (the parts form: what its sums and elements showed)
 
   {
     float4v z = {0.f, 0.f, 0.f, 0.f};
@@ -283,7 +357,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
   };
   // bcol0: first output column of the block of 64 the columns belong to; ncols: how many of
   // the block's columns the workgroup has (64, or the 16 of a fifth group)
-  auto epi_consts = [&](int bcol0, int ncols) -> EpiConsts {
+  auto epi_consts = [&](int bcol0, int ncols, int tid) -> EpiConsts {
     EpiConsts e;
     e.gca = 0.f;
     e.gcb = 0.f;
@@ -322,19 +396,26 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
     }
     return e;
   };
-  EpiConsts ec = {}, ecx = {};  // of the workgroup's block of 64 columns; of a fifth group
-  if constexpr (EPI) {
-    ec = epi_consts(col0, kCN);
-    if constexpr (FIVE) ecx = epi_consts(xcol, 16);
+  // of the workgroup's block of 64 columns; of a fifth group
+  // (the parts form has no registers to keep them in: it loads them as a tile is written out)
+  EpiConsts ec = {}, ecx = {};
+  if constexpr (EPI && !PARTS) {
+    ec = epi_consts(col0, kCN, tid);
+    if constexpr (FIVE) ecx = epi_consts(xcol, 16, tid);
   }
   const int e_c_dest = epi.c_dest, e_act_s = epi.act_s, e_act_g = epi.act_g;
   auto flush_tile = [&](int row0, int rows, int slot0) __attribute__((always_inline)) {
+    if (!kProducersFlush && producer) return;
+    int tid = threadIdx.x;
+    // (the parts form: or what follows from it alone is worked out ahead of the loop, kept in
+    // scratch memory, and its loads stand between those of the rows)
+    if constexpr (PARTS) asm volatile("" : "+v"(tid));
     if constexpr (FIVE && !EPI) {
       // the fifth column group (accumulator columns kCN .. kCN + 15): four threads a row
       if (xcol >= 0) {
         const float4v z = {0.f, 0.f, 0.f, 0.f};
         const int c4 = (tid & 3) * 4;
-        for (int r = tid >> 2; r < rows; r += NT / 4) {
+        for (int r = tid >> 2; r < rows; r += NTF / 4) {
           int sl = slot0 + r;
           if (sl >= T) sl -= T;
           float4v *ap = reinterpret_cast<float4v *>(acc + sl * kAS + kCN + c4);
@@ -356,7 +437,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
       // 16 columns a wave owns: add them up in the first 16, clear the others, and write
       // the tile out as any other.
       const float4v z = {0.f, 0.f, 0.f, 0.f};
-      for (int r = tid >> 2; r < rows; r += NT / 4) {
+      for (int r = tid >> 2; r < rows; r += NTF / 4) {
         int sl = slot0 + r;
         if (sl >= T) sl -= T;
         float4v *ap = reinterpret_cast<float4v *>(acc + sl * kAS + (tid & 3) * 4);
@@ -383,7 +464,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
         constexpr bool FAST = decltype(fast_tag)::value;
         constexpr bool XG = decltype(x_tag)::value;
         constexpr int U = 2;
-        constexpr int RS = NT / (kCN / 4);
+        constexpr int RS = NTF / (kCN / 4);
         const int r_t = tid / (kCN / 4), c_t = (tid % (kCN / 4)) * 4;
         const bool own = !XG || c_t < 16;  // the thread has columns
         constexpr int kCol0 = XG ? kCN : 0;
@@ -413,6 +494,10 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
           float *a0 = acc + sl0 * kAS + kCol0, *a1 = acc + sl1 * kAS + kCol0;
           if (e.gcl >= 0) {
             const float x0 = a0[e.gcl], x1 = two ? a1[e.gcl] : 0.f;
+            if constexpr (PARTS) {
+              check.sum(x0);
+              check.sum(x1);
+            }
             a0[e.gcl] = gate_act(x0);
             if (two) a1[e.gcl] = gate_act(x1);
           }
@@ -422,6 +507,15 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
           if (two) {
             if (own) v1 = *reinterpret_cast<float4v *>(a1 + c_t);
             g1 = float4v{a1[e.mg[0] >> 4], a1[e.mg[1] >> 4], a1[e.mg[2] >> 4], a1[e.mg[3] >> 4]};
+          }
+          if constexpr (PARTS) {
+            // (a gate's column holds its activated value by now: its sum was looked at above)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const bool stored = (e.mg[i] & 15) != 3;
+              check.sum(stored ? v0[i] : 0.f);
+              check.sum(stored ? v1[i] : 0.f);
+            }
           }
           __builtin_amdgcn_sched_barrier(0);  // the clears stay behind every read above
           if (own) *reinterpret_cast<float4v *>(a0 + c_t) = z;
@@ -456,6 +550,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
           gp += U * gstep;
         }
       };
+      if constexpr (PARTS) ec = epi_consts(col0, kCN, tid);
       const bool fast = (e_act_s == SSC_ACT_NONE || e_act_s == SSC_ACT_RELU) &&
                         (e_act_g == SSC_ACT_NONE || e_act_g == SSC_ACT_SIGMOID);
       if constexpr (FIVE) {
@@ -473,14 +568,14 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
       return;
     }
     if ((cout & 3) == 0) {
-      // A thread keeps its 4 columns and walks down the rows, NT / (kCN / 4) rows per
+      // A thread keeps its 4 columns and walks down the rows, NTF / (kCN / 4) rows per
       // step: addresses advance by constants, so a step is little more than its LDS
       // read, LDS clear and store, and four reads are in flight before the first store
       // (one at a time, every step would pay the full LDS latency while the matrix
       // cores idle).
       const float4v z = {0.f, 0.f, 0.f, 0.f};
       constexpr int U = 4;
-      constexpr int RS = NT / (kCN / 4);  // rows per step
+      constexpr int RS = NTF / (kCN / 4);  // rows per step
       const int r_t = tid / (kCN / 4), c_t = (tid % (kCN / 4)) * 4;
       const bool col_ok = col0 + c_t < cout;
       IO *gp = out + (int64_t)(row0 + r_t) * cout + col0 + c_t;
@@ -495,6 +590,10 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
             float4v *ap = reinterpret_cast<float4v *>(acc + sl * kAS + c_t);
             v[u] = *ap;
             *ap = z;
+            if constexpr (PARTS) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) check.sum(v[u][i]);
+            }
           }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -505,10 +604,11 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
         gp += U * gstep;
       }
     } else {
-      for (int e = tid; e < rows * kCN; e += NT) {
+      for (int e = tid; e < rows * kCN; e += NTF) {
         int r = e / kCN, c = e % kCN;
         int sl = slot0 + r;
         if (sl >= T) sl -= T;
+        if constexpr (PARTS) check.sum(acc[sl * kAS + c]);
         if (col0 + c < cout)
           __builtin_nontemporal_store((IO)acc[sl * kAS + c], out + (int64_t)(row0 + r) * cout + col0 + c);
         acc[sl * kAS + c] = 0.f;
@@ -526,6 +626,423 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
     rows = r < 0 ? -r : r;
     return r > 0 && pos.cc == nch - 1;
   };
+
+  // ---------------------------------------------------------------- the bfloat16-parts form
+  // The plan's blocks are kBP = 16 NB pairs of one offset (NB row blocks, 2 or 4).  A stage is two
+  // blocks x 32 input channels, one matrix step of v_mfma_f32_16x16x32_bf16; two stages are a
+  // chunk.  Consumer wave (r, c) multiplies block r with the 32 columns c of the workgroup's
+  // 64: a weight fragment serves 16 NB rows, a staged row 32 columns.  Producers cut the gathered
+  // rows into parts on their way into LDS, the filters come in parts (conv_pack.h).
+  // A stage's barrier stands before its last row block: by then the consumers hold that in
+  // registers and the next stage is in LDS; its first row block is read during the last one's
+  // products.
+  // The products of a chunk are summed by themselves and then added to those of the chunks
+  // before (one rounding at the sum's size a chunk, not twelve); a group's stay in registers.
+  // Waves (0, c) and (1, c) have the same columns and may have the same output rows: (0, c) adds
+  // its products of a group to the accumulators during the first stage of the next group and
+  // (1, c) during the second, or one after the other when the tile ends: every sum in the
+  // order of the schedule.
+  //
+  // What the parts cannot do is worked out again with float instructions: a workgroup that has
+  // met one of the following walks its groups a second time (see the end of the form).
+  //  - Infinities, NaN, and floats that round to an infinity as bfloat16: a sum not finite.
+  //  - Elements with bits below 2^-133, the last of a bfloat16: of a row, what is left for the
+  //    third part is a bfloat16 then and only then if the lower half of its word is zero; of
+  //    the filters, a NaN stands in their place.
+  //  - Sums that are not zero and below 2^-95: six products of parts, each rounded at 2^-150.
+  //
+  // What bounds it (128 -> 64 channels, 216 stages of 48 matrix instructions a wave, 185 us): a
+  // stage is 788 cycles of matrix instructions and takes about 1800; LDS (48 reads of a KiB at 4-8
+  // cycles, 48 writes of 512 bytes at 8) and the vector memory path (40 KiB at 64 bytes a cycle)
+  // are busy 600-700 cycles each, the producers' cutting 450, which share the SIMDs with the
+  // products; none of them alone sets the pace.  Blocks of 64 halve the fragment loads of a product
+  // and the barriers, and pad more; four row blocks leave registers for two stages of fragments.
+  // Microseconds, float form -> blocks of 32 / of 64, and the error against 64 bits:
+  //   128 -> 64,  1.54M pairs, every row   287 ->  210 /  185    2.0e-7 -> 1.5e-7
+  //   128 -> 304, 1.69M pairs, stride 2   1396 -> 1063 /  934    1.8e-7 -> 1.3e-7
+  //   256 -> 608, 0.51M pairs, stride 2   1710 -> 1216 / 1095    2.1e-7 -> 1.4e-7
+  //   512 -> 608, 1.03M pairs             6880 -> 5513 / 4465    2.6e-7 -> 1.6e-7
+  //   608 -> 512, 1.03M pairs, every row  6580 -> 4720 / 4277    3.3e-7 -> 1.8e-7
+  //   304 -> 128, 1.69M pairs, stride 2   1523 -> 1235 / 1312    1.7e-7 -> 1.2e-7
+  //    64 -> 128, 1.54M pairs, 1 in 10     290 ->  328 /  500    (stays with the float form)
+  // With the sums of all chunks in one chain the error of the wide ones is 2.7e-7 to 4.1e-7.
+  if constexpr (PARTS) {
+    constexpr int NB = FORM == 5 ? 4 : 2;
+    constexpr int GS = NB / 2;                  // groups of the schedule to a stage
+    constexpr int kStageB = 2 * NB * 3 * 1024;  // bytes of a staged stage
+    const int g_last = g_end - GS;
+    const int n_ck = (g_end - g_begin) / GS * nch;  // chunks of this workgroup
+    char *const abytes = reinterpret_cast<char *>(abuf);
+    int *const odd_s = reinterpret_cast<int *>(abytes + 2 * kStageB);
+    const __amdgpu_buffer_rsrc_t rs_feat =
+        __builtin_amdgcn_make_buffer_rsrc((void *)features, 0, (int)feat_bytes, kRsrcFlags);
+    const __amdgpu_buffer_rsrc_t rs_w =
+        __builtin_amdgcn_make_buffer_rsrc((void *)packed, 0, (int)packed_bytes, kRsrcFlags);
+    const __amdgpu_buffer_rsrc_t rs_in =
+        __builtin_amdgcn_make_buffer_rsrc((void *)sched_in, 0, (int)sched_bytes, kRsrcFlags);
+    const __amdgpu_buffer_rsrc_t rs_out =
+        __builtin_amdgcn_make_buffer_rsrc((void *)sched_out, 0, (int)sched_bytes, kRsrcFlags);
+    if (n_ck == 0) return;  // (the whole workgroup)
+    if (tid == 0) odd_s[0] = 0;
+    // A staged row block is, part by part, a KiB in the order of the consumers' lanes: lane
+    // (l16, g) has the 16 bytes at 256 g + 16 (l16 ^ swizzle(g)), which neither their reads
+    // nor the producers' writes meet banks twice with (reads 4-7 cycles a KiB, where rows of
+    // 192 + 16 bytes take 8; writes 8 cycles for 512 bytes either way).
+    auto swizzle = [](int g) -> int { return (0x84C0 >> (4 * g)) & 15; };  // 0, 12, 4, 8
+    if (producer) {
+      const PartsCut cut;
+      const int pt = tid - NCW * 64;
+      const int row = pt >> 3;   // this thread's pairs: row, row + 32, ...
+      const int piece = pt & 7;  // its four channels of a stage
+      const bool beyond[2] = {(nch - 1) * 64 + piece * 4 >= cin, (nch - 1) * 64 + 32 + piece * 4 >= cin};
+      // lane group g of an operand has channels 4 g .. + 3 and 16 + 4 g .. + 3 of a stage, as
+      // in the packed filters
+      char *const st_base = abytes + (row >> 4) * 3072 + (piece & 3) * 256 +
+                            (((row & 15) ^ swizzle(piece & 3)) * 16) + (piece >> 2) * 8;
+      // rows[s % RD]: the rows of stage s, RD stages (RC chunks) in flight; idx[c % 4]: the
+      // gather offsets of chunk c, four chunks further (loads return in order: a wait for
+      // offsets is one for the rows that were asked for before them)
+      constexpr int RD = 16 / NB, RC = RD / 2;
+      int idx[4][NB];
+      float4v rows[RD][NB];
+      auto load_idx = [&](const PartsPos &pos, int (&ix)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) ix[j] = buf_load1(rs_in, row * 4 + j * 128, pos.g * 256);
+      };
+      auto load_rows = [&](const PartsPos &pos, int ks, const int (&ix)[NB], float4v (&v)[NB])
+          __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          int off = ix[j];
+          if constexpr (GATHER == 2) off = (pos.cc == nch - 1 && beyond[ks]) ? (int)kGatherPad : off;
+          v[j] = buf_load4(rs_feat, off + piece * 16, pos.cc * 256 + ks * 128);
+        }
+      };
+      auto store_rows = [&](int buf, const float4v (&v)[NB]) __attribute__((always_inline)) {
+        int2v p[NB][3];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          int h, m, l;
+          cut.two(v[j].x, v[j].y, h, m, l, check.rest);
+          p[j][0].x = h;
+          p[j][1].x = m;
+          p[j][2].x = l;
+          cut.two(v[j].z, v[j].w, h, m, l, check.rest);
+          p[j][0].y = h;
+          p[j][1].y = m;
+          p[j][2].y = l;
+        }
+        char *dst = st_base + buf * kStageB;
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+            *reinterpret_cast<int2v *>(dst + j * 2 * 3072 + i * 1024) = p[j][i];
+      };
+      PartsPos p_rows = {g_begin, 0}, p_idx = {g_begin, 0}, p_cur = {g_begin, 0};
+      {
+        // stage 0 goes to LDS, the rows of stages 1 .. RD stay in flight, and the offsets of
+        // chunks RC .. RC + 3; loads in the order in which the loop waits for them
+        int ix[RC][NB];
+#pragma unroll
+        for (int c = 0; c < RC; ++c) {
+          load_idx(p_idx, ix[c]);
+          p_idx.advance(GS, nch, g_last);
+        }
+#pragma unroll
+        for (int c = RC; c < RC + 4; ++c) {
+          load_idx(p_idx, idx[c & 3]);
+          p_idx.advance(GS, nch, g_last);
+        }
+        float4v r0[NB];
+        load_rows(p_rows, 0, ix[0], r0);
+#pragma unroll
+        for (int s = 1; s < RD; ++s) {
+          if ((s & 1) == 0) p_rows.advance(GS, nch, g_last);
+          load_rows(p_rows, s & 1, ix[s >> 1], rows[s]);
+        }
+        p_rows.advance(GS, nch, g_last);
+        load_rows(p_rows, 0, idx[RC & 3], rows[0]);
+        store_rows(0, r0);
+      }
+      // (tile rows of the chunk's group, negative unless it ends with the group: read a chunk ahead)
+      int tile_rows = grp_meta[(int64_t)(g_begin + GS - 1) * 8 + 5];
+      asm volatile("" : "+s"(tile_rows));  // (here: a load still out would be waited for in the loop)
+      __syncthreads();  // stage 0 is there
+      // Chunk c, stages s and s + 1: the rows of s + 1 and s + 2 are staged, those of s + 1 + RD
+      // (chunk c + RC) and s + 2 + RD and the offsets of chunk c + RC + 4 are asked for.
+      auto chunk = [&](auto phase) __attribute__((always_inline)) {
+        constexpr int ph = decltype(phase)::value;  // == c % 4
+        constexpr int r1 = (2 * ph + 1) % RD, r2 = (2 * ph + 2) % RD, i1 = (ph + RC) & 3,
+                      i2 = (ph + RC + 1) & 3;
+        const int g_cur = p_cur.g, n_rows = tile_rows;
+        const bool last = n_rows > 0 && p_cur.cc == nch - 1;
+        p_cur.advance(GS, nch, g_last);
+        tile_rows = grp_meta[(int64_t)(p_cur.g + GS - 1) * 8 + 5];
+        store_rows(1, rows[r1]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_rows(p_rows, 1, idx[i1], rows[r1]);
+        p_rows.advance(GS, nch, g_last);
+        load_idx(p_idx, idx[i1]);
+        p_idx.advance(GS, nch, g_last);
+        __syncthreads();
+        store_rows(0, rows[r2]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_rows(p_rows, 0, idx[i2], rows[r2]);
+        __syncthreads();
+        if (last) {
+          __syncthreads();
+          __syncthreads();
+          const int32_t *m = grp_meta + (int64_t)g_cur * 8;
+          flush_tile(m[4], n_rows, m[6]);
+          __syncthreads();
+        }
+      };
+      int c = 0;
+      for (; c + 4 <= n_ck; c += 4) {
+        chunk(std::integral_constant<int, 0>());
+        chunk(std::integral_constant<int, 1>());
+        chunk(std::integral_constant<int, 2>());
+        chunk(std::integral_constant<int, 3>());
+      }
+      if (c < n_ck) chunk(std::integral_constant<int, 0>());
+      if (c + 1 < n_ck) chunk(std::integral_constant<int, 1>());
+      if (c + 2 < n_ck) chunk(std::integral_constant<int, 2>());
+    } else {
+      // stages whose filters are in registers, and how far ahead they are asked for (a stage of
+      // four row blocks lasts twice as long and leaves fewer registers)
+      constexpr int WR = NB == 2 ? 4 : 2, AHEAD = WR - 1;
+      const int g = lane >> 4, l16 = lane & 15;
+      const int wr = wave >> 1, wc = wave & 1;
+      const int parts_at = (int)(packed_bytes / (4096u + kPartFragBytes) * 4096u);
+      const int cb0 = min(col0 / 16 + 2 * wc, ncb - 1), cb1 = min(col0 / 16 + 2 * wc + 1, ncb - 1);
+      const int w_base[2] = {parts_at + cb0 * nch * kPartFragBytes,
+                             parts_at + cb1 * nch * kPartFragBytes};
+      const char *const a_base = abytes + wr * NB * 3072 + g * 256 + (l16 ^ swizzle(g)) * 16;
+      typedef __attribute__((address_space(3))) float4v lds_float4v;
+      const int acc_base = (int)(size_t)(__attribute__((address_space(3))) char *)acc;
+      auto lds_load4 = [](int addr) -> float4v { return *(lds_float4v *)(size_t)addr; };
+      auto lds_store4 = [](int addr, const float4v &v) { *(lds_float4v *)(size_t)addr = v; };
+      const int acc_lane = acc_base + (wc * 32 + g * 4) * 4;  // (and 64 bytes on: the second group)
+      // rings; the loop is unrolled over two chunks (four stages):
+      //   w[s % WR]    filters of stage s [column group][part]
+      //   a[b & 1]     rows of row block b [part], read from LDS one block ahead
+      //   orow[c & 1]  accumulator rows of this lane's pairs in the group of chunk c
+      int4v w[WR][2][3], a[2][3];
+      int orow[2][NB];
+      // sums [row block][column group]: of this chunk; of the group's chunks before or, during a
+      // group's first chunk, of the group before; accumulators as they were read
+      float4v t[NB][2], sum[NB][2], x[2][2];
+      bool pending = false;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          t[b][i] = sum[b][i] = x[b & 1][i] = float4v{0.f, 0.f, 0.f, 0.f};
+      auto kof_of = [&](const PartsPos &pos) -> int {
+        return grp_meta[(int64_t)pos.g * 8 + (NB == 2 ? 2 * wr : 8 * wr)];
+      };
+      // byte offset of a chunk's filters but for the column group's part (packed as floats an
+      // offset's filters are k_scale bytes, in parts 3/2 of that)
+      auto soff_of = [](int kof, int cc) -> int { return (int)((unsigned)kof / 2u * 3u) + cc * kPartFragBytes; };
+      auto load_w = [&](int soff, int ks, int i, int p) __attribute__((always_inline)) -> int4v {
+        return __builtin_bit_cast(
+            int4v, buf_load4(rs_w, lane * 16 + ks * 3072 + p * 1024, soff + w_base[i]));
+      };
+      auto load_orow = [&](const PartsPos &pos, int (&o)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          o[b] = buf_load1(rs_out, l16 * 4 + (wr * NB + b) * 64, pos.g * 256);
+      };
+      auto read_a = [&](int buf, int b, int part) __attribute__((always_inline)) -> int4v {
+        return *reinterpret_cast<const int4v *>(a_base + buf * kStageB + b * 3072 + part * 1024);
+      };
+      PartsPos p_cur = {g_begin, 0}, p_next = {g_begin, 0}, p_f = {g_begin, 0};
+      p_next.advance(GS, nch, g_last);
+      int soff = soff_of(kof_of(p_f), 0);  // filters of the chunk that are asked for next
+      p_f.advance(GS, nch, g_last);
+#pragma unroll
+      for (int st = 0; st < AHEAD; ++st)  // in the loop's order: stage by stage, part by part
+#pragma unroll
+        for (int p = 2; p >= 0; --p)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            if (st == 2 && p == 2 && i == 0) {
+              soff = soff_of(kof_of(p_f), p_f.cc);
+              p_f.advance(GS, nch, g_last);
+            }
+            w[st][i][p] = load_w(soff, st & 1, i, p);
+          }
+      load_orow(p_cur, orow[0]);
+      int kof = kof_of(p_f);  // of the chunk behind soff's
+      int tile_rows = grp_meta[(int64_t)(g_begin + GS - 1) * 8 + 5];  // (as in the producers)
+      asm volatile("" : "+s"(tile_rows), "+s"(kof));
+      __syncthreads();
+#pragma unroll
+      for (int p = 0; p < 3; ++p) a[0][p] = read_a(0, 0, p);
+      // two row blocks of the group before: h = 0 or 1
+      auto commit_read = [&](const int (&o)[NB], int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) x[b][i] = lds_load4(o[2 * h + b] + acc_lane + i * 64);
+      };
+      auto commit_write = [&](const int (&o)[NB], int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            lds_store4(o[2 * h + b] + acc_lane + i * 64, x[b][i] + sum[2 * h + b][i]);
+      };
+      // the products of parts, the smallest first
+      constexpr int kWp[6] = {2, 0, 1, 1, 0, 0}, kAp[6] = {0, 2, 1, 0, 1, 0};
+      // One chunk.  Everything a stage needs besides its products lies between them, and the
+      // branches in it are short: what they hold shares no registers with loads in flight.
+      auto chunk = [&](auto phase) __attribute__((always_inline)) {
+        constexpr int cp = decltype(phase)::value;  // == c % 2
+        const int g_cur = p_cur.g, n_rows = tile_rows;
+        const bool grp_first = p_cur.cc == 0, grp_last = p_cur.cc == nch - 1;
+        const bool commit = pending && grp_first;
+        // (a first chunk's products take the place of the sums: a factor and no branch)
+        const float keep = grp_first ? 0.f : 1.f;
+        auto add_up = [&](int b, int i) __attribute__((always_inline)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[b][i][e] = __builtin_fmaf(sum[b][i][e], keep, t[b][i][e]);
+        };
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          const int cur = (2 * cp + ks) % WR, nxt = (2 * cp + ks + AHEAD) % WR;
+          const bool turn = commit && wr == ks;
+#pragma unroll
+          for (int b = 0; b < NB; ++b) {
+            if (b == NB - 1) __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int p = 0; p < 6; ++p) {
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+                t[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    __builtin_bit_cast(bf16x8, w[cur][i][kWp[p]]),
+                    __builtin_bit_cast(bf16x8, a[b & 1][kAp[p]]),
+                    ks == 0 && p == 0 ? float4v{0.f, 0.f, 0.f, 0.f} : t[b][i], 0, 0, 0);
+              if (p < 3) {  // the next row block's rows
+                constexpr int kRead[3] = {0, 2, 1};
+                a[(b + 1) & 1][kRead[p]] =
+                    b < NB - 1 ? read_a(ks, b + 1, kRead[p]) : read_a(ks ^ 1, 0, kRead[p]);
+              }
+              if (b == 0 && p >= 1 && p < 4) {  // the filters of stage s + AHEAD
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                  w[nxt][i][3 - p] = load_w(soff, (ks + AHEAD) & 1, i, 3 - p);
+              }
+              if (b < NB / 2 && p == 0 && turn) commit_read(orow[cp ^ 1], b);
+              if (b < NB / 2 && p == 4 && turn) commit_write(orow[cp ^ 1], b);
+              if (ks == 1 && b > 0 && (p == 2 || p == 3)) add_up(b - 1, p - 2);
+              if (ks == 1 && b == NB - 1 && p == 4) load_orow(p_next, orow[cp ^ 1]);
+              if (ks == 0 && b == NB - 2 && p == 3) {
+                // from here on the next chunk's filters are asked for, or its successor's (stage
+                // s + AHEAD); the next chunk's tile.  (Scalar loads: behind the row block's last
+                // wait for LDS data, which they would turn into a wait for everything.)
+                soff = soff_of(kof, p_f.cc);
+                p_f.advance(GS, nch, g_last);
+                kof = kof_of(p_f);
+                tile_rows = grp_meta[(int64_t)(p_next.g + GS - 1) * 8 + 5];
+              }
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) add_up(NB - 1, i);
+        p_cur.advance(GS, nch, g_last);
+        p_next.advance(GS, nch, g_last);
+        if (commit) pending = false;
+        if (grp_last) pending = true;
+        if (grp_last && n_rows > 0) {
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            if (wr == r) {
+#pragma unroll
+              for (int h = 0; h < NB / 2; ++h) {
+                commit_read(orow[cp], h);
+                commit_write(orow[cp], h);
+              }
+            }
+            __syncthreads();
+          }
+          pending = false;
+          const int32_t *m = grp_meta + (int64_t)g_cur * 8;
+          flush_tile(m[4], n_rows, m[6]);
+          // (nothing of these is wanted behind a tile: no registers for them while it is written)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) sum[b][i] = x[b & 1][i] = float4v{0.f, 0.f, 0.f, 0.f};
+          __syncthreads();
+        }
+      };
+      int c = 0;
+      for (; c + 2 <= n_ck; c += 2) {
+        chunk(std::integral_constant<int, 0>());
+        chunk(std::integral_constant<int, 1>());
+      }
+      if (c < n_ck) chunk(std::integral_constant<int, 0>());
+    }
+    // (all waves are behind the last tile's last barrier: every range ends with a tile's end)
+    if (check.odd()) odd_s[0] = 1;
+    __syncthreads();
+    if (odd_s[0] == 0) return;
+    // The workgroup's tiles again, on float instructions: consumer wave w has columns 16 w .. of
+    // the 64 and walks the row blocks in order, operands straight from memory.  Rare, and slower
+    // than the float form.
+    {
+      const int g = lane >> 4, l16 = lane & 15;
+      const int w_base = min(col0 / 16 + (producer ? 0 : wave), ncb - 1) * nch * 4096;
+      float *const acc_lane = acc + (producer ? 0 : wave) * 16 + g * 4;
+      for (int gi = g_begin; gi < g_end; ++gi) {
+        if (!producer) {
+          float4v d[4];
+          int in_off[4], out_off[4], kof[4];
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            d[b] = float4v{0.f, 0.f, 0.f, 0.f};
+            in_off[b] = sched_in[(int64_t)gi * 64 + b * 16 + l16];
+            out_off[b] = sched_out[(int64_t)gi * 64 + b * 16 + l16];
+            kof[b] = grp_meta[(int64_t)gi * 8 + b];
+          }
+          for (int cc = 0; cc < nch; ++cc)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+              float4v av[4], wv[4];
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                int off = in_off[b];
+                if (GATHER == 2 && cc * 64 + q * 16 + g * 4 >= cin) off = (int)kGatherPad;
+                av[q] = buf_load4(rs_feat, off + q * 64 + g * 16, cc * 256);
+                wv[q] = buf_load4(rs_w, lane * 16 + q * 1024, kof[b] + w_base + cc * 4096);
+              }
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                  d[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q][j], av[q][j], d[b], 0, 0, 0);
+            }
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            float4v *to = reinterpret_cast<float4v *>(reinterpret_cast<char *>(acc_lane) + out_off[b]);
+            *to += d[b];
+          }
+        }
+        const int32_t *m = grp_meta + (int64_t)gi * 8;
+        if (m[5] > 0) {
+          __syncthreads();
+          flush_tile(m[4], m[5], m[6]);
+          __syncthreads();
+        }
+      }
+    }
+    return;
+  }
 
   if (producer) {
     // ------------------------------------------------------------------ producer
@@ -1177,6 +1694,10 @@ struct ConvPlan {
   // a layer of a handful of input channels: no schedule, no matrix kernel -- the plan is a
   // table of every output row's input rows and the rows are computed by conv_small_kernel
   bool small;
+  // the bfloat16-parts form
+  bool parts;
+  bool parts_packed;  // the packed filters have the parts behind the floats
+  int blk;  // pairs of an offset to a block: 16, in the parts form 32 or 64
   int kvol;           // kernel volume and number of output rows the plan was made for
   int64_t out_rows;
 };
@@ -1227,7 +1748,8 @@ inline int launch_conv(const ConvPlan &p, const ConvWs &w, const IO *features, i
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     attr_set = true;
   }
-  const uint64_t packed_bytes = (uint64_t)K * p.ncb * p.nch * Io<IO>::kFragBytes;
+  const uint64_t packed_bytes = (uint64_t)K * p.ncb * p.nch *
+                                (FORM >= 4 ? Io<IO>::kFragBytes + kPartFragBytes : Io<IO>::kFragBytes);
   const uint64_t sched_bytes = (uint64_t)p.grp_cap * 256;
   SSC_CHECK(packed_bytes < ((uint64_t)1 << 32) && sched_bytes < ((uint64_t)1 << 32), SSC_ERUNTIME,
             "convolution too large for 32-bit buffer offsets (filters %llu B, schedule %llu B)",
@@ -1245,11 +1767,13 @@ inline int launch_conv(const ConvPlan &p, const ConvWs &w, const IO *features, i
   // (4 MiB per XCD) and the grid divides that way (256 -> 256 channels, 7 MiB: 2.44 ->
   // 2.24 ms on the 64^3 benchmark geometry; 128 -> 256 at stride 2, 3.5 MiB, is 5 % slower
   // that way and stays with the row-major mapping)
-  const bool by_column = packed_bytes > ((uint64_t)4 << 20) && p.n_colblk > 1 &&
+  const uint64_t walked_bytes = (uint64_t)K * p.ncb * p.nch *
+                                (FORM >= 4 ? kPartFragBytes : Io<IO>::kFragBytes);
+  const bool by_column = walked_bytes > ((uint64_t)4 << 20) && p.n_colblk > 1 &&
                          8 % p.n_colblk == 0 && (p.n_wg * p.n_colblk) % 8 == 0 &&
                          g_conv_by_column;
   // (-1: a grid that is no multiple of 8 wide takes the kernel's mapping for any grid)
-  const bool big = packed_bytes > ((uint64_t)4 << 20) && p.n_colblk > 1 && g_conv_by_column;
+  const bool big = walked_bytes > ((uint64_t)4 << 20) && p.n_colblk > 1 && g_conv_by_column;
   const int cols_per_xcd = by_column ? 8 / p.n_colblk
                            : ((p.n_wg & 7) != 0 && p.n_wg * p.n_colblk >= 16) ? (big ? -2 : -1) : 0;
   hipLaunchKernelGGL((conv_fwd_kernel<IO, GATHER, NCW, NS, EPI, FORM>), grid, dim3((NCW + 4) * 64), p.lds_bytes, s, features, c_in,

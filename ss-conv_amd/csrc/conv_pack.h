@@ -17,7 +17,35 @@ struct PackArgs {
   int K, cin, cout, ncb, nch;
   void *packed_out;
   int ns;  // MFMA steps per chunk (float filters; half filters always use whole chunks)
+  int parts;  // float filters: packed in parts as well (see pack_parts_element)
 };
+
+// Float filters in whole chunks of 64 channels are packed a second time, behind the first, as
+// the bfloat16 parts that the parts form of conv_fwd_kernel multiplies: per (offset, column
+// group, chunk), two steps of 32 channels x three parts x 64 lanes x 8 channels.  Lane group g
+// of step s has the channels 32 s + 4 g .. + 3 and 32 s + 16 + 4 g .. + 3 of the chunk, the ones it
+// has in the float fragments 2 s and 2 s + 1.
+constexpr int kPartFragBytes = 2 * 3 * 1024;
+// Element idx of the packed filters, value v.  An element that is not the sum of its parts (bits
+// below 2^-133; floats that round to an infinity) gets a NaN for its first part: every sum it
+// is in is refused and worked out again with the float fragments (infinities and NaN do so by
+// themselves).
+__device__ __forceinline__ void pack_parts_element(const PackArgs &a, int64_t idx, float v) {
+  const int64_t frag = idx >> 10;
+  const int f = (int)(idx & 1023), q = f >> 8, lane = (f >> 2) & 63, j = f & 3;
+  __bf16 *dst = reinterpret_cast<__bf16 *>(static_cast<char *>(a.packed_out) +
+                                           (int64_t)a.K * a.ncb * a.nch * 4096 + frag * kPartFragBytes) +
+                ((q >> 1) * 3 * 64 + lane) * 8 + (q & 1) * 4 + j;
+  __bf16 hi = (__bf16)v;
+  float left = v - (float)hi;
+  const __bf16 mid = (__bf16)left;
+  left -= (float)mid;
+  const __bf16 lo = (__bf16)left;
+  if ((float)lo != left) hi = (__bf16)__builtin_nanf("");
+  dst[0] = hi;
+  dst[64 * 8] = mid;
+  dst[2 * 64 * 8] = lo;
+}
 
 // Offset k, input channel ci and output channel co of element idx of the packed filters
 // (ci >= cin or co >= cout: a padding element).
@@ -61,6 +89,9 @@ __device__ __forceinline__ void pack_filter_element(const PackArgs &a, int64_t i
   IO v = (IO)0.f;
   if (ci < a.cin && co < a.cout) v = w[k * a.fs_k + ci * a.fs_ci + co * a.fs_co];
   static_cast<IO *>(a.packed_out)[idx] = v;
+  if constexpr (sizeof(IO) == 4) {
+    if (a.parts) pack_parts_element(a, idx, v);
+  }
 }
 
 
@@ -87,6 +118,7 @@ __device__ __forceinline__ void combine_pack_element(const CombineJob &j, int64_
     j.dense[((int64_t)k * j.pk.cin + ci) * j.pk.cout + co] = v;
   }
   static_cast<float *>(j.pk.packed_out)[idx] = v;
+  if (j.pk.parts) pack_parts_element(j.pk, idx, v);
 }
 int launch_combine_pack(const CombineJob &job, hipStream_t s);
 
