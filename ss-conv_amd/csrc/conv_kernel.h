@@ -19,7 +19,7 @@ typedef int int4v __attribute__((ext_vector_type(4)));
 
 constexpr int kKC = 64;       // input channels per chunk = 16 MFMA steps of 4
 constexpr int kStage = 64;    // pairs staged per barrier = 4 row blocks of 16
-constexpr int kAStride = 68;  // floats per staged row (64 + 4: 16-byte aligned, bank spread)
+constexpr int kAStride = 64;  // floats per staged row (its 16-byte pieces permuted: staged_piece)
 constexpr int kMinTile = 64;
 
 // ---- the convolution --------------------------------------------------------------------
@@ -62,7 +62,7 @@ constexpr int kMinTile = 64;
 // so every output element sees its offsets added in ascending k: reproducible,
 // no atomics.
 //
-// Dynamic LDS: acc[T+1][16*NCW+4] | abuf[2][64][68]
+// Dynamic LDS: acc[T+1][16*NCW+4] | abuf[2][64][64]
 constexpr int kRowsAhead = 4;  // stages whose gathered rows are in flight in registers
 constexpr int kIdxAhead = 2;   // further stages whose gather offsets are in flight
 constexpr unsigned kGatherPad = 0xFFFFF000u;  // byte offset that gathers zeros (beyond any feature buffer)
@@ -115,7 +115,7 @@ template <> struct Io<float> {
 };
 template <> struct Io<_Float16> {
   static constexpr int kBytes = 2;
-  static constexpr int kRowBytes = 144;  // 128 + 16: 16-byte aligned, bank spread as for float
+  static constexpr int kRowBytes = 128;
   static constexpr int kFragBytes = 2048;
   typedef int2v Raw;
   static __device__ __forceinline__ Raw zero() { return Raw{0, 0}; }
@@ -138,6 +138,14 @@ template <> struct Io<_Float16> {
     __builtin_nontemporal_store(__builtin_bit_cast(int2v, h), reinterpret_cast<int2v *>(p));
   }
 };
+
+// Where 16-byte piece `piece` of a staged row (16 of a float one, 8 of a half one) lies in it, row:
+// its number in its row block.  A read of one piece by the 16 rows of a block, and by four lane
+// groups of four neighbouring pieces, then meets no bank twice: 4.1 cycles a KiB where rows with
+// 16 bytes of padding take 8.4 (the float form 64 -> 128 channels, 1.54M pairs: 289 -> 281 us).
+template <bool HALF> __device__ __forceinline__ int staged_piece(int piece, int row) {
+  return (HALF ? piece ^ (row >> 1) : piece ^ row) * 16;
+}
 
 // Position of a stage in the schedule: group index and channel chunk.  Advanced
 // with scalar arithmetic only.
@@ -1104,8 +1112,14 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
     };
     // where this thread's piece goes in a staged row: its own 16 bytes, or, for a piece of
     // the partly used quarter, element (piece - 4 kQFull) of each lane group's 16 bytes
-    char *const st_base = reinterpret_cast<char *>(abuf) + (pt >> 4) * kRowB +
-                          (spread ? (16 * kQFull + (piece - 4 * kQFull)) * kEB : piece * 4 * kEB);
+    const int r16 = pt >> 4;  // the rows' number in their row blocks
+    char *const st_base = reinterpret_cast<char *>(abuf) + r16 * kRowB +
+                          (spread  ? (piece - 4 * kQFull) * kEB
+                           : kHalf ? staged_piece<true>(piece >> 1, r16) + (piece & 1) * 8
+                                   : staged_piece<false>(piece, r16));
+    int spread_at[4];  // pieces of the four lane groups in the partly used quarter
+#pragma unroll
+    for (int i = 0; i < 4; ++i) spread_at[i] = staged_piece<false>((4 * kQFull + i) & 15, r16);
     auto store_rows = [&](int parity, const Held (&r)[NE]) {
 #pragma unroll
       for (int j = 0; j < NE; ++j) {
@@ -1113,10 +1127,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
         if constexpr (!kHalf && kQRem != 0) {
           if (spread) {
             const float4v v = __builtin_bit_cast(float4v, r[j]);
-            reinterpret_cast<float *>(dst)[0] = v.x;
-            reinterpret_cast<float *>(dst)[4] = v.y;
-            reinterpret_cast<float *>(dst)[8] = v.z;
-            reinterpret_cast<float *>(dst)[12] = v.w;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) *reinterpret_cast<float *>(dst + spread_at[i]) = v[i];
             continue;
           }
         }
@@ -1208,7 +1220,12 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
     const int w_voff = lane * 16;  // this lane's 16 bytes of a KiB of fragments
     constexpr int kWStep = 1024;   // from one 16-byte piece to the next
     const int w_soff0 = cb * nch * kFragB;  // fragments of this wave's column block
-    const char *const a_base = reinterpret_cast<const char *>(abuf) + l16 * kRowB + g * 16;
+    // this lane's 16 bytes of quarter q of its row in a row block
+    const char *a_base[NF];
+#pragma unroll
+    for (int q = 0; q < NF; ++q)
+      a_base[q] = reinterpret_cast<const char *>(abuf) + l16 * kRowB +
+                  staged_piece<kHalf>(4 * q + g, l16);
     // The accumulators are addressed with 32-bit LDS byte addresses (acc_lane includes
     // the base of acc): no pointer arithmetic left for the vector ALU.
     typedef __attribute__((address_space(3))) float4v lds_float4v;
@@ -1321,7 +1338,6 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
       //                loaded four stages ahead, into the slot the stage before just used
       int kof[4];
       int4v tl[4];
-      const char *const ab_wave = a_base + wave * 16 * kRowB;
       auto load_kof = [&](const StagePos &pos) -> int {
         return buf_load1(rs_meta, wave * 4, pos.g * 32);
       };
@@ -1362,10 +1378,10 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
           kof[nx] = load_kof(p_k);
           p_k.advance(nch);
         }
-        const char *ab = ab_wave + (ph & 1) * kStage * kRowB;
         Frag a[NF];
 #pragma unroll
-        for (int q = 0; q < NF; ++q) a[q] = *reinterpret_cast<const Frag *>(ab + q * 64);
+        for (int q = 0; q < NF; ++q)
+          a[q] = *reinterpret_cast<const Frag *>(a_base[q] + (wave * 16 + (ph & 1) * kStage) * kRowB);
         const bool commit = p_cur.cc == nch - 1;  // the group's last chunk
         const int addr = commit ? orow[ph] + acc_lane : dummy_addr;
         const float4v accr = lds_load4(addr);
@@ -1423,7 +1439,6 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
     int aprev = dummy_x;
     bool x_pending = false;
     constexpr bool x_on = FIVE;  // (a launch of the form has a fifth group: xcol >= 0)
-    const char *const abx = a_base + wave * 16 * kRowB;
     const int w_soffx = (x_on ? xcol / 16 : 0) * nch * kFragB;
     auto load_kofx = [&](const StagePos &pos) -> int {
       return buf_load1(rs_meta, wave * 4, pos.g * 32);
@@ -1459,7 +1474,6 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
     auto run_stage = [&](auto parity, bool last_cur, const StagePos &cur, const StagePos &next,
                          const StagePos &after, TileEnd &end_next) {
       constexpr int par = decltype(parity)::value;
-      const char *ab = a_base + par * kStage * kRowB;
       const int base_cur = w_soff0 + cur.cc * kFragB;
       const int base_next = w_soff0 + next.cc * kFragB;
       // Staged rows in registers: of this block and the next.  Half: of all four blocks, read
@@ -1469,7 +1483,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
       constexpr int kARing = kHalf ? 4 : 2;
       Frag a[kARing][NF];
       auto load_a = [&](int m, int q, Frag (&av)[NF]) {
-        av[q] = *reinterpret_cast<const Frag *>(ab + m * 16 * kRowB + q * 64);
+        av[q] = *reinterpret_cast<const Frag *>(a_base[q] + (par * kStage + m * 16) * kRowB);
       };
 #pragma unroll
       for (int m = 0; m < (kHalf ? 4 : 1); ++m)
@@ -1539,7 +1553,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
 #pragma unroll
             for (int qq = 0; qq < NF; ++qq)
               if (i == kGapA[qq])
-                a[0][qq] = *reinterpret_cast<const Frag *>(abx + par * kStage * kRowB + qq * 64);
+                a[0][qq] = *reinterpret_cast<const Frag *>(a_base[qq] +
+                                                           (par * kStage + wave * 16) * kRowB);
           }
           // this stage's record was last used by block 0: refill it for the stage
           // after the next
