@@ -948,7 +948,7 @@ def indice_conv_half(features, filters, indice_pairs, indice_num, num_act_out, i
 
 
 def _indice_conv_backward(dtype, name, features, filters, out_bp, indice_pairs, indice_num,
-                          inverse, subm):
+                          inverse, subm, want):
     _need_gpu(features, filters, out_bp, indice_pairs)
     if features.dtype != dtype or filters.dtype != dtype or out_bp.dtype != dtype:
         raise RuntimeError("%s needs %s tensors" % (name, dtype))
@@ -965,9 +965,12 @@ def _indice_conv_backward(dtype, name, features, filters, out_bp, indice_pairs, 
     dev = features.device
     s = _stream(features)
     # input gradient: the forward kernel on out_bp, pairs swapped, filters transposed
-    input_bp = _conv_any(out_bp, owner, filters, (fs_k, fs_co, fs_ci), indice_pairs, pairs, num, K,
-                         c_out, c_in, n_in, not inverse, subm)
-    # filter gradient
+    input_bp = filters_bp = None
+    if want[0]:
+        input_bp = _conv_any(out_bp, owner, filters, (fs_k, fs_co, fs_ci), indice_pairs, pairs, num,
+                             K, c_out, c_in, n_in, not inverse, subm)
+    if not want[1]:
+        return [input_bp, filters_bp]
     filters_bp = torch.empty(tuple(filters.shape), dtype=dtype, device=dev)
     ws2 = _workspace(_lib.ssc_conv_bwd_filter_workspace_bytes(K, c_in, c_out, pairs.size(2)), dev)
     _check(_ENTRIES[dtype][3](_ptr(features), n_in, c_in, _ptr(out_bp), n_out, c_out, _ptr(pairs),
@@ -976,18 +979,20 @@ def _indice_conv_backward(dtype, name, features, filters, out_bp, indice_pairs, 
     return [input_bp, filters_bp]
 
 
-def indice_conv_backward_fp32(features, filters, out_bp, indice_pairs, indice_num, inverse, subm):
+def indice_conv_backward_fp32(features, filters, out_bp, indice_pairs, indice_num, inverse, subm,
+                              want=(True, True)):
     """src/conv/indice_conv.h:344-426 (bound at src/ss_conv_ops_api.cpp:22): returns
-    [input_bp like features, filters_bp shaped like filters]."""
+    [input_bp like features, filters_bp shaped like filters], None for what is not wanted."""
     return _indice_conv_backward(torch.float32, "indice_conv_backward_fp32", features, filters,
-                                 out_bp, indice_pairs, indice_num, inverse, subm)
+                                 out_bp, indice_pairs, indice_num, inverse, subm, want)
 
 
-def indice_conv_backward_half(features, filters, out_bp, indice_pairs, indice_num, inverse, subm):
+def indice_conv_backward_half(features, filters, out_bp, indice_pairs, indice_num, inverse, subm,
+                              want=(True, True)):
     """indiceConvBackward<at::Half> (src/ss_conv_ops.cu:79-83, bound at
     src/ss_conv_ops_api.cpp:24): half-precision tensors, fp32 arithmetic."""
     return _indice_conv_backward(torch.float16, "indice_conv_backward_half", features, filters,
-                                 out_bp, indice_pairs, indice_num, inverse, subm)
+                                 out_bp, indice_pairs, indice_num, inverse, subm, want)
 
 
 _POOL_ENTRIES = {

@@ -30,7 +30,7 @@ class _ConvBase(Function):
             indice_pairs._ssc_meta = ctx.ssc_meta
         input_bp, filters_bp = ops.indice_conv_backward(
             features, filters, grad_output.contiguous(), indice_pairs, indice_pair_num,
-            cls.inverse, cls.subm)
+            cls.inverse, cls.subm, ctx.needs_input_grad[:2])
         return input_bp, filters_bp, None, None, None
 
 
@@ -104,7 +104,7 @@ class SparseConvRulebookFunction(Function):
             indice_pairs._ssc_meta = ctx.ssc_meta
         input_bp, filters_bp = ops.indice_conv_backward(
             features, filters, grad_output.contiguous(), indice_pairs, indice_pair_num, False,
-            ctx.subm)
+            ctx.subm, ctx.needs_input_grad[:2])
         return (input_bp, filters_bp) + (None,) * 9
 
 

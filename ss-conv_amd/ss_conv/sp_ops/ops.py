@@ -73,14 +73,14 @@ def indice_conv_forward(features, filters, indice_pairs, indice_pair_num, num_ac
 
 
 def indice_conv_backward(features, filters, out_bp, indice_pairs, indice_pair_num, inverse=False,
-                         subm=False):
-    """[input_bp, filters_bp] (reference: sp_ops/ops.py:116-150)."""
+                         subm=False, want=(True, True)):
+    """[input_bp, filters_bp] (reference: sp_ops/ops.py:116-150), None for what is not wanted."""
     if filters.dtype == torch.float32:
         return _ext.indice_conv_backward_fp32(features, filters, out_bp, indice_pairs,
-                                              indice_pair_num, int(inverse), int(subm))
+                                              indice_pair_num, int(inverse), int(subm), want)
     if filters.dtype == torch.half:
         return _ext.indice_conv_backward_half(features, filters, out_bp, indice_pairs,
-                                              indice_pair_num, int(inverse), int(subm))
+                                              indice_pair_num, int(inverse), int(subm), want)
     raise NotImplementedError("convolution is built for float32 and half filters")
 
 

@@ -157,3 +157,22 @@ def test_parts_with_epilogue(blk, odd, device):
         finally:
             _ext._lib.ssc_conv_tuning(1)
     assert rel_l2(got[0], got[1]) < 2e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_gradients_nobody_asks_for(dtype, device):
+    """A convolution whose input, or whose filters, need no gradient: the other one's bits do not
+    change and nothing is returned in its place."""
+    from ss_conv.sp_ops.functional import SparseConvFunction
+    n_in, o_idx, pairs, num = _rulebook(700, 12, 3, 1, 7, device)
+    x = torch.randn(n_in, 64, device=device).to(dtype)
+    w = (torch.randn(3, 3, 3, 64, 72, device=device) / 40).to(dtype)
+    dy = torch.randn(o_idx.shape[0], 72, device=device).to(dtype)
+    got = {}
+    for want in ((True, True), (True, False), (False, True)):
+        a, b = [t.clone().requires_grad_(need) for t, need in zip((x, w), want)]
+        SparseConvFunction.apply(a, b, pairs, num, o_idx.shape[0]).backward(dy)
+        got[want] = a.grad, b.grad
+    assert got[True, False][1] is None and got[False, True][0] is None
+    assert torch.equal(got[True, False][0], got[True, True][0])
+    assert torch.equal(got[False, True][1], got[True, True][1])
