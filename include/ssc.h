@@ -206,11 +206,15 @@ int ssc_rulebook_conv_finish(const ssc_geometry *g, int64_t n_in, int32_t *n_out
  * Every row of out[n_out,Cout] is written (zeros where no pair lands).
  * ---------------------------------------------------------------------- */
 #define SSC_CONV_PAIRS_CANONICAL 2
-/* The rulebook is of a regular (not submanifold, not transposed) convolution of unit stride: may
- * be added to `kernel_volume` of ssc_conv_fwd_*, ssc_conv_plan_build and ssc_conv_run_*, and to
- * `elem_bytes` of ssc_rulebook_conv_begin / _finish.  It tells how many pairs to expect, which
- * decides what form the kernel takes, and is the same in all calls on one plan. */
-#define SSC_CONV_UNIT_STRIDE 0x10000
+/* What a rulebook's geometry tells of the number of its pairs, which decides what form the
+ * kernel takes (no counterpart in the reference): ssc_rulebook_kind gives a value for a
+ * geometry (host arithmetic only; 0: nothing is known), and ssc_conv_expect says of which kind
+ * the rulebook of the calling host thread's NEXT ssc_conv_fwd_*, ssc_conv_plan_build or
+ * ssc_conv_run_* call is.  That call takes the value and leaves 0 behind, also where it fails.
+ * The calls on one plan are told the same; ssc_rulebook_conv_finish builds its plan for the
+ * kind of the geometry it is given.  Returns SSC_OK. */
+int32_t ssc_rulebook_kind(const ssc_geometry *g);
+int ssc_conv_expect(int32_t kind);
 
 size_t ssc_conv_workspace_bytes(int64_t n_out, int32_t kernel_volume, int32_t c_in,
                                 int32_t c_out, int64_t pair_stride);

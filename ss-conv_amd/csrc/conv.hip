@@ -1273,10 +1273,14 @@ static int parts_block(int64_t n_in, int64_t n_out, int64_t pair_stride, bool un
   return in32 >= (unit ? 34.0 : 20.0) ? 32 : 0;
 }
 
-// unit: the rulebook is of a convolution of unit stride (SSC_CONV_UNIT_STRIDE).
+// What ssc_rulebook_kind says of a rulebook: of a regular convolution of unit stride, or nothing.
+constexpr int32_t kKindUnit = 1;
+
+// kind: of the rulebook (ssc_rulebook_kind).
 static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_out,
-                          int64_t pair_stride, int elem_bytes = 4, bool unit = false,
+                          int64_t pair_stride, int elem_bytes = 4, int32_t kind = 0,
                           bool allow_parts = true) {
+  const bool unit = kind == kKindUnit;
   ConvPlan p;
   p.ncb = (int)ceil_div(c_out, 16);
   p.nch = (int)ceil_div(c_in, kKC);
@@ -1367,7 +1371,7 @@ static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_ou
   plan_split(p, n_wg, pair ? 2 * n_wg : n_wg, n_out, K, pair_stride, n_in <= 0);
   // (a schedule of larger blocks that 32-bit offsets do not reach: the float form's may fit)
   if (p.parts && (uint64_t)p.grp_cap * 256 >= ((uint64_t)1 << 32))
-    return make_plan(n_in, n_out, K, c_in, c_out, pair_stride, elem_bytes, unit, false);
+    return make_plan(n_in, n_out, K, c_in, c_out, pair_stride, elem_bytes, kind, false);
   // (sizing calls: room for the parts form as well, which parts_block takes only where the
   // outputs are at most so many times the inputs)
   if (parts_can && n_in <= 0) {
@@ -1882,10 +1886,12 @@ static int conv_check_sizes(int K, int c_in, int c_out, int64_t n_in, int64_t n_
   return SSC_OK;
 }
 
-// SSC_CONV_UNIT_STRIDE rides on the kernel volume (or on the element size).
-static int strip_unit(int v, bool *unit) {
-  *unit = v > 0 && (v & SSC_CONV_UNIT_STRIDE) != 0;
-  return *unit ? v & ~SSC_CONV_UNIT_STRIDE : v;
+// The kind of the rulebook of this host thread's next call on a convolution (ssc_conv_expect).
+static thread_local int32_t g_expected_kind = 0;
+static int32_t take_expected() {
+  const int32_t kind = g_expected_kind;
+  g_expected_kind = 0;
+  return kind;
 }
 
 // The forward convolution for features, filters and output of element type IO.
@@ -1895,8 +1901,8 @@ static int conv_fwd(const IO *features, int64_t n_in, int32_t c_in, const IO *fi
                     const int32_t *pairs, int64_t pair_stride, const int32_t *pair_num,
                     int32_t kernel_volume, int32_t inverse, int32_t subm, IO *out, int64_t n_out,
                     void *workspace, size_t workspace_bytes, ssc_stream_t stream) {
-  bool unit;
-  const int K = strip_unit(kernel_volume, &unit);
+  const int32_t kind = take_expected();
+  const int K = kernel_volume;
   int rc = conv_check_sizes(K, c_in, c_out, n_in, n_out, pair_stride);
   if (rc != SSC_OK) return rc;
   if (n_out == 0) return SSC_OK;
@@ -1909,7 +1915,7 @@ static int conv_fwd(const IO *features, int64_t n_in, int32_t c_in, const IO *fi
   SSC_CHECK(workspace_bytes >= need, SSC_EWORKSPACE, "conv workspace too small: %zu < %zu",
             workspace_bytes, need);
 
-  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, (int)sizeof(IO), unit);
+  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, (int)sizeof(IO), kind);
   ConvWs w;
   conv_ws_walk(workspace, p, K, pair_stride, &w);
   const PackArgs pack = {filters, fs_k, fs_ci, fs_co, K, c_in, c_out, p.ncb, p.nch, w.packed, p.ns, p.parts_packed};
@@ -1941,16 +1947,15 @@ static int conv_pack(const IO *filters, int64_t fs_k, int64_t fs_ci, int64_t fs_
 template <typename IO>
 static int conv_planned(const IO *features, int64_t n_in, int32_t c_in, const void *packed,
                         size_t packed_bytes, const void *plan, size_t plan_bytes, int64_t pair_stride,
-                        int32_t kernel_volume, int32_t c_out, IO *out, int64_t n_out, hipStream_t s) {
-  bool unit;
-  const int K = strip_unit(kernel_volume, &unit);
+                        int32_t K, int32_t c_out, IO *out, int64_t n_out, hipStream_t s) {
+  const int32_t kind = take_expected();
   int rc = conv_check_sizes(K, c_in, c_out, n_in, n_out, pair_stride);
   if (rc != SSC_OK) return rc;
   if (n_out == 0) return SSC_OK;
   SSC_CHECK(out != nullptr, SSC_EINVAL, "out is NULL");
   if (pair_stride == 0 || n_in == 0) return fill_zero(out, n_out * c_out, s);
   SSC_CHECK(features && packed && plan, SSC_EINVAL, "NULL pointer argument");
-  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, (int)sizeof(IO), unit);
+  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, (int)sizeof(IO), kind);
   SSC_CHECK(packed_bytes >= conv_packed_bytes(p, K), SSC_EWORKSPACE,
             "buffer of the packed filters too small");
   SSC_CHECK(plan_bytes >= conv_plan_walk(nullptr, p, nullptr), SSC_EWORKSPACE,
@@ -1965,11 +1970,10 @@ static int conv_planned(const IO *features, int64_t n_in, int32_t c_in, const vo
 template <typename IO>
 static int conv_planned_epilogue(const IO *features, int64_t n_in, int32_t c_in,
                                  const void *packed, size_t packed_bytes, const void *plan,
-                                 size_t plan_bytes, int64_t pair_stride, int32_t kernel_volume,
-                                 int32_t c_cols, const ssc_conv_epilogue *e, IO *out,
-                                 int64_t n_out, hipStream_t s) {
-  bool unit;
-  const int K = strip_unit(kernel_volume, &unit);
+                                 size_t plan_bytes, int64_t pair_stride, int32_t K, int32_t c_cols,
+                                 const ssc_conv_epilogue *e, IO *out, int64_t n_out,
+                                 hipStream_t s) {
+  const int32_t kind = take_expected();
   int rc = conv_check_sizes(K, c_in, c_cols, n_in, n_out, pair_stride);
   if (rc != SSC_OK) return rc;
   SSC_CHECK(e != nullptr, SSC_EINVAL, "epilogue is NULL");
@@ -1985,7 +1989,7 @@ static int conv_planned_epilogue(const IO *features, int64_t n_in, int32_t c_in,
   SSC_CHECK(e->shift && e->scale && e->add && e->pre_bias && e->mode && e->gate && e->dest &&
                 e->gate_run,
             SSC_EINVAL, "NULL table in the epilogue");
-  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_cols, pair_stride, (int)sizeof(IO), unit);
+  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_cols, pair_stride, (int)sizeof(IO), kind);
   SSC_CHECK(packed_bytes >= conv_packed_bytes(p, K), SSC_EWORKSPACE,
             "buffer of the packed filters too small");
   SSC_CHECK(plan_bytes >= conv_plan_walk(nullptr, p, nullptr), SSC_EWORKSPACE,
@@ -2044,6 +2048,18 @@ int ssc_conv_fwd_f16(const void *features, int64_t n_in, int32_t c_in, const voi
                             static_cast<_Float16 *>(out), n_out, workspace, workspace_bytes, stream);
 }
 
+int32_t ssc_rulebook_kind(const ssc_geometry *g) {
+  if (g == nullptr || g->subm || g->transpose) return 0;
+  for (int a = 0; a < 3; ++a)
+    if (g->stride[a] != 1) return 0;
+  return kKindUnit;
+}
+
+int ssc_conv_expect(int32_t kind) {
+  g_expected_kind = kind;
+  return SSC_OK;
+}
+
 int ssc_conv_tile_cut(int32_t rows, int32_t c_in, int32_t c_out, int32_t *n_tiles, int32_t *height,
                       int32_t *window) {
   SSC_CHECK(rows >= 0 && c_in >= 1 && c_out >= 1 && n_tiles && height && window, SSC_EINVAL,
@@ -2089,14 +2105,14 @@ int ssc_conv_plan_build(const int32_t *pairs, int64_t pair_stride, const int32_t
                         int64_t n_out, int32_t c_in, int32_t c_out, int32_t elem_bytes, void *plan,
                         size_t plan_bytes, void *scratch, size_t scratch_bytes,
                         ssc_stream_t stream) {
-  bool unit;
-  const int K = strip_unit(kernel_volume, &unit);
+  const int32_t kind = take_expected();
+  const int K = kernel_volume;
   int rc = conv_check_sizes(K, c_in, c_out, n_in, n_out, pair_stride);
   if (rc != SSC_OK) return rc;
   SSC_CHECK(elem_bytes == 4 || elem_bytes == 2, SSC_EINVAL, "elem_bytes must be 4 or 2");
   if (n_out == 0 || pair_stride == 0 || n_in == 0) return SSC_OK;  // nothing to schedule
   SSC_CHECK(pairs && pair_num && plan && scratch, SSC_EINVAL, "NULL pointer argument");
-  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, elem_bytes, unit);
+  ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, pair_stride, elem_bytes, kind);
   SSC_CHECK(plan_bytes >= conv_plan_walk(nullptr, p, nullptr), SSC_EWORKSPACE,
             "plan buffer too small");
   SSC_CHECK(scratch_bytes >= conv_scratch_walk(nullptr, p, K, pair_stride, nullptr),
@@ -2153,9 +2169,8 @@ int ssc_rulebook_conv_begin(const int32_t *indices, int64_t n_in, const ssc_geom
   g_pending_layer = PendingLayer();
   SSC_CHECK(g != nullptr, SSC_EINVAL, "geometry is NULL");
   SSC_CHECK(c_in >= 1 && c_out >= 1, SSC_EINVAL, "channel counts must be positive");
-  bool unit;
-  elem_bytes = strip_unit(elem_bytes, &unit);
   SSC_CHECK(elem_bytes == 4 || elem_bytes == 2, SSC_EINVAL, "elem_bytes must be 4 or 2");
+  const int32_t kind = ssc_rulebook_kind(g);
   CombineJob job = {};
   if (filters != nullptr) {
     int rc = combine_job_of(filters->weight, filters->basis, filters->chan_out, filters->chan_in,
@@ -2178,9 +2193,9 @@ int ssc_rulebook_conv_begin(const int32_t *indices, int64_t n_in, const ssc_geom
     const size_t head = conv_scratch_head(scratch, &w);
     // (the form depends on the number of outputs as well, and with it the number of ranges of
     // layers with a lone last column group: the guess is a scattered cloud's)
-    const ConvPlan more = make_plan(n_in, 10 * n_in + 1, (int)K, c_in, c_out, n_in, elem_bytes, unit);
+    const ConvPlan more = make_plan(n_in, 10 * n_in + 1, (int)K, c_in, c_out, n_in, elem_bytes, kind);
     const ConvPlan fewer =
-        make_plan(n_in, n_in > 1 ? n_in - 1 : 1, (int)K, c_in, c_out, n_in, elem_bytes, unit);
+        make_plan(n_in, n_in > 1 ? n_in - 1 : 1, (int)K, c_in, c_out, n_in, elem_bytes, kind);
     const bool more_ok = !more.rebalance && !more.small;
     const bool fewer_ok = strided && n_in > 1 && !fewer.rebalance && !fewer.small &&
                           !(more_ok && fewer.n_rng == more.n_rng &&
@@ -2221,8 +2236,6 @@ int ssc_rulebook_conv_finish(const ssc_geometry *g, int64_t n_in, int32_t *n_out
   g_pending_layer = PendingLayer();
   int rc = ssc_rulebook_finish(g, n_in, n_out_host, in_order_host);
   if (rc != SSC_OK) return rc;
-  bool unit;
-  elem_bytes = strip_unit(elem_bytes, &unit);
   const int64_t n_out = *n_out_host;
   int K = 1;
   for (int a = 0; a < 3; ++a) K *= g->ksize[a];
@@ -2231,7 +2244,8 @@ int ssc_rulebook_conv_finish(const ssc_geometry *g, int64_t n_in, int32_t *n_out
   SSC_CHECK(elem_bytes == 4 || elem_bytes == 2, SSC_EINVAL, "elem_bytes must be 4 or 2");
   if (n_out == 0 || n_in == 0) return SSC_OK;  // nothing to schedule
   SSC_CHECK(pairs && pair_num && plan && scratch, SSC_EINVAL, "NULL pointer argument");
-  const ConvPlan p = make_plan(n_in, n_out, K, c_in, c_out, n_in, elem_bytes, unit);
+  const ConvPlan p =
+      make_plan(n_in, n_out, K, c_in, c_out, n_in, elem_bytes, ssc_rulebook_kind(g));
   SSC_CHECK(plan_bytes >= conv_plan_walk(nullptr, p, nullptr), SSC_EWORKSPACE,
             "plan buffer too small");
   SSC_CHECK(scratch_bytes >= conv_scratch_walk(nullptr, p, K, n_in, nullptr), SSC_EWORKSPACE,

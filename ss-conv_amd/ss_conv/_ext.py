@@ -58,6 +58,8 @@ _SIGNATURES = {
     "ssc_conv_plan_bytes": (_sz, [_i64, _i32, _i32, _i32, _i64]),
     "ssc_conv_plan_scratch_bytes": (_sz, [_i64, _i32, _i32, _i32, _i64]),
     "ssc_conv_packed_bytes": (_sz, [_i32, _i32, _i32]),
+    "ssc_rulebook_kind": (_i32, [_vp]),
+    "ssc_conv_expect": (ctypes.c_int, [_i32]),
     "ssc_conv_tile_cut": (ctypes.c_int, [_i32, _i32, _i32, ctypes.POINTER(_i32),
                                          ctypes.POINTER(_i32), ctypes.POINTER(_i32)]),
     "ssc_conv_plan_build": (ctypes.c_int, [_vp, _i64, _vp, _i32, _i32, _i32, _i64, _i64, _i32, _i32,
@@ -253,9 +255,6 @@ _ROWS_KEEP_BYTES = 64 << 20  # unused rows of such a buffer beyond which the res
 _PLAN_AHEAD_BYTES = 128 << 20
 
 
-_UNIT_STRIDE = 0x10000  # SSC_CONV_UNIT_STRIDE of include/ssc.h
-
-
 class RulebookMeta(object):
     """What the library knows about a rulebook it wrote itself: for which direction the pairs
     of every offset ascend in the rows that are accumulated into (`canonical`: (forward,
@@ -270,16 +269,16 @@ class RulebookMeta(object):
     origin.  A pairs tensor of other identity (a clone, a tensor that came back from a
     checkpoint) is bound to the same plans by adopt_meta once it has been compared with the
     tensor the plans were built over."""
-    __slots__ = ("version", "canonical", "plans", "pairs_ref", "unit")
+    __slots__ = ("version", "canonical", "plans", "pairs_ref", "kind")
     MAX_PLANS = 8
 
-    def __init__(self, version, canonical, plans=None, pairs_ref=None, unit=0):
+    def __init__(self, version, canonical, plans=None, pairs_ref=None, kind=0):
         import collections
         self.version = version
         self.canonical = canonical
         self.plans = collections.OrderedDict() if plans is None else plans
         self.pairs_ref = pairs_ref  # the tensor the plans were built over
-        self.unit = unit  # SSC_CONV_UNIT_STRIDE of a convolution of unit stride, or 0
+        self.kind = kind  # ssc_rulebook_kind of its geometry
 
     def get_plan(self, key):
         plan = self.plans.get(key)
@@ -321,7 +320,7 @@ def adopt_meta(indice_pairs, meta):
         if ref._version != meta.version or not bool(torch.equal(indice_pairs, ref)):
             return None
     bound = RulebookMeta(indice_pairs._version, meta.canonical, plans=meta.plans,
-                         pairs_ref=indice_pairs, unit=meta.unit)
+                         pairs_ref=indice_pairs, kind=meta.kind)
     indice_pairs._ssc_meta = bound
     return bound
 
@@ -482,7 +481,7 @@ class _PendingRulebook(object):
     """A rulebook between ssc_rulebook_begin and ssc_rulebook_finish: everything whose size
     does not depend on the number of outputs is queued, the host has not waited yet."""
     __slots__ = ("indices", "n", "geometry", "ws", "pairs", "num", "out_buf", "subm", "stream",
-                 "bound", "plan", "scratch", "conv", "main", "side", "unit")
+                 "bound", "plan", "scratch", "conv", "main", "side", "kind")
 
 
 def _rulebook_begin(indices, batch_size, out_spatial_shape, kernel_size, stride, padding, dilation,
@@ -512,7 +511,7 @@ def _rulebook_begin(indices, batch_size, out_spatial_shape, kernel_size, stride,
         nbytes = 256
     r = _PendingRulebook()
     r.indices, r.n, r.geometry, r.subm = indices, n, g, bool(subm)
-    r.unit = 0 if subm or transpose or any(int(v) != 1 for v in stride) else _UNIT_STRIDE
+    r.kind = _lib.ssc_rulebook_kind(gref)
     r.main = torch.cuda.current_stream(dev)
     if conv is None:
         worth = n * K >= _INDEX_STREAM_MIN_WORK
@@ -575,7 +574,7 @@ def _rulebook_queue(r, gref, K, nbytes, conv):
                 _ptr(indices), n, gref, r.ws.data_ptr(), r.ws.numel(), _ptr(r.pairs),
                 r.num.data_ptr(), _ptr(r.out_buf), 0 if r.out_buf is None else r.out_buf.size(0),
                 _ptr(clean), 0 if clean is None else clean.numel(),
-                r.conv[0], r.conv[1], r.conv[2] | r.unit, r.scratch.data_ptr(), r.scratch.numel(),
+                r.conv[0], r.conv[1], r.conv[2], r.scratch.data_ptr(), r.scratch.numel(),
                 ctypes.byref(job) if job is not None else None, r.stream))
         else:
             _check(_lib.ssc_rulebook_begin(_ptr(indices), n, gref, r.ws.data_ptr(), r.ws.numel(),
@@ -595,7 +594,7 @@ def _rulebook_conv_wait(r):
     in_order = _i32(0)
     _check(_lib.ssc_rulebook_conv_finish(
         ctypes.byref(r.geometry), r.n, ctypes.byref(n_out), ctypes.byref(in_order),
-        _ptr(r.pairs), r.num.data_ptr(), r.conv[0], r.conv[1], r.conv[2] | r.unit, r.plan.data_ptr(),
+        _ptr(r.pairs), r.num.data_ptr(), r.conv[0], r.conv[1], r.conv[2], r.plan.data_ptr(),
         r.plan.numel(), r.scratch.data_ptr(), r.scratch.numel(), r.stream))
     return n_out.value, bool(in_order.value)
 
@@ -632,7 +631,7 @@ def _rulebook_result(r, n_out, in_order):
     # (the first flag serves a call that accumulates into output rows, the second one
     # with `inverse`, which accumulates into input rows).
     r.pairs._ssc_meta = RulebookMeta(r.pairs._version, (in_order, True), pairs_ref=r.pairs,
-                                       unit=r.unit)
+                                     kind=r.kind)
     if r.side is not None:
         _mark_side_ready(outids)
     return [outids, r.pairs, r.num]
@@ -726,8 +725,9 @@ def _plan_of(meta, pairs, num, K, c_in, c_out, elem_bytes, n_in, n_out, inverse,
         plan = _workspace(_lib.ssc_conv_plan_bytes(n_out, K, c_in, c_out, stride), dev)
         scratch = _workspace(_lib.ssc_conv_plan_scratch_bytes(n_out, K, c_in, c_out, stride), dev)
         flags = 2 if meta.canonical[1 if inverse else 0] else 0
-        _check(_lib.ssc_conv_plan_build(_ptr(pairs), stride, num.data_ptr(), K | meta.unit,
-                                        int(bool(inverse)), flags, n_in, n_out, c_in, c_out, elem_bytes,
+        _lib.ssc_conv_expect(meta.kind)
+        _check(_lib.ssc_conv_plan_build(_ptr(pairs), stride, num.data_ptr(), K, int(bool(inverse)),
+                                        flags, n_in, n_out, c_in, c_out, elem_bytes,
                                         plan.data_ptr(), plan.numel(), scratch.data_ptr(),
                                         scratch.numel(), stream))
         meta.put_plan(key, plan)
@@ -763,12 +763,14 @@ class ConvEpilogue(object):
                                       int(act_gate), int(c_dest))
 
 
-def _run_planned(features, n_in, c_in, packed, plan, pair_stride, K, c_out, n_out, s, epilogue):
-    """Queue the kernel over packed filters and a plan (K: with the rulebook's _UNIT_STRIDE, as the
-    plan was built); with an epilogue the rows stored are those of the normalised, gated result."""
+def _run_planned(features, n_in, c_in, packed, plan, pair_stride, K, c_out, n_out, s, epilogue,
+                 kind):
+    """Queue the kernel over packed filters and a plan of a rulebook of `kind`; with an epilogue
+    the rows stored are those of the normalised, gated result."""
     dev = features.device
     if epilogue is None:
         out = torch.empty((n_out, c_out), dtype=features.dtype, device=dev)
+        _lib.ssc_conv_expect(kind)
         _check(_ENTRIES[features.dtype][2](_ptr(features), n_in, c_in, packed.data_ptr(),
                                            packed.numel(), plan.data_ptr(), plan.numel(),
                                            pair_stride, K, c_out, _ptr(out), n_out, s))
@@ -780,6 +782,7 @@ def _run_planned(features, n_in, c_in, packed, plan, pair_stride, K, c_out, n_ou
     # (looked up by name at every call: tests count the calls through these attributes)
     entry = (_lib.ssc_conv_run_epilogue_f32 if features.dtype == torch.float32
              else _lib.ssc_conv_run_epilogue_f16)
+    _lib.ssc_conv_expect(kind)
     _check(entry(_ptr(features), n_in, c_in, packed.data_ptr(), packed.numel(), plan.data_ptr(),
                  plan.numel(), pair_stride, K, c_out, ctypes.byref(epilogue.struct), _ptr(out),
                  n_out, s))
@@ -798,8 +801,8 @@ def _planned_conv(meta, features, owner, filters, fs, pairs, num, K, c_in, c_out
     packed = _packed_filters(owner, filters, fs, K, c_in, c_out, s)
     plan = _plan_of(meta, pairs, num, K, c_in, c_out, features.element_size(), n_in, n_out,
                     inverse, dev, s)
-    return _run_planned(features, n_in, c_in, packed, plan, pairs.size(2), K | meta.unit, c_out,
-                        n_out, s, epilogue)
+    return _run_planned(features, n_in, c_in, packed, plan, pairs.size(2), K, c_out, n_out, s,
+                        epilogue, meta.kind)
 
 
 def rulebook_conv(features, filters, indices, batch_size, out_spatial_shape, kernel_size, stride,
@@ -850,8 +853,8 @@ def rulebook_conv(features, filters, indices, batch_size, out_spatial_shape, ker
             plan = _plan_of(pairs._ssc_meta, pairs, num, K, c_in, c_out, eb, n_in, n_out, False,
                             dev, r.stream, beside=r.side is not None)
         _index_done(r, outids, pairs, num, plan)
-        out = _run_planned(features, n_in, c_in, packed, plan, n_in, K | r.unit, c_out, n_out, s,
-                           epilogue)
+        out = _run_planned(features, n_in, c_in, packed, plan, n_in, K, c_out, n_out, s, epilogue,
+                           r.kind)
         return out, outids, pairs, num
     n_out, in_order = _rulebook_conv_wait(r)
     if r.side is not None:
@@ -859,11 +862,11 @@ def rulebook_conv(features, filters, indices, batch_size, out_spatial_shape, ker
         # queued there)
         outids, pairs, num = _rulebook_result(r, n_out, in_order)
         _index_done(r, outids, pairs, num, r.plan)
-        out = _run_planned(features, n_in, c_in, packed, r.plan, n_in, K | r.unit, c_out, n_out, s,
-                           epilogue)
+        out = _run_planned(features, n_in, c_in, packed, r.plan, n_in, K, c_out, n_out, s,
+                           epilogue, r.kind)
     else:
-        out = _run_planned(features, n_in, c_in, packed, r.plan, n_in, K | r.unit, c_out, n_out, s,
-                           epilogue)
+        out = _run_planned(features, n_in, c_in, packed, r.plan, n_in, K, c_out, n_out, s,
+                           epilogue, r.kind)
         outids, pairs, num = _rulebook_result(r, n_out, in_order)
     if n_out > 0:
         pairs._ssc_meta.put_plan((False, c_in, c_out, eb, n_in, n_out, _tuning_now[0]), r.plan)

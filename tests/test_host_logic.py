@@ -125,6 +125,27 @@ def test_tile_cut_of_a_range():
                                  ctypes.byref(win)) == _ext.SSC_EINVAL
 
 
+def test_sizes_carry_no_flags():
+    """A kernel volume or an element size out of range is refused whatever bits it has; what a
+    caller expects of a rulebook has a call of its own."""
+    from ss_conv import _ext
+    lib = _ext._lib
+    for K in (257, 65536 + 27, 65600, 65536 + 256, (1 << 30) + 27, -27, 0):
+        calls = [lib.ssc_conv_fwd_f32(None, 0, 64, None, 1, 1, 1, 64, None, 0, None, K, 0, 0, None, 0,
+                                      None, 0, None),
+                 lib.ssc_conv_plan_build(None, 0, None, K, 0, 0, 0, 0, 64, 64, 4, None, 0, None, 0, None),
+                 lib.ssc_conv_run_f32(None, 0, 64, None, 0, None, 0, 0, K, 64, None, 0, None),
+                 lib.ssc_conv_run_epilogue_f32(None, 0, 64, None, 0, None, 0, 0, K, 64, None, None, 0,
+                                               None)]
+        assert calls == [_ext.SSC_ERUNTIME] * 4, (K, calls)
+    g = _ext._geometry(1, [8] * 3, [3] * 3, [1] * 3, [1] * 3, [1] * 3, 0, 0)
+    for eb in (65536 + 4, 65536 + 2, 3, 0):
+        assert lib.ssc_rulebook_conv_begin(None, 0, ctypes.byref(g), None, 0, None, None, None, 0, None,
+                                           0, 64, 64, eb, None, 0, None, None) == _ext.SSC_EINVAL
+    assert lib.ssc_rulebook_kind(None) == 0 and lib.ssc_rulebook_kind(ctypes.byref(g)) != 0
+    assert lib.ssc_conv_expect(0) == 0
+
+
 # ---- shape arithmetic and the tensor type ---------------------------------------------------
 @pytest.mark.parametrize("size,k,s,p,d", [(64, 3, 1, 1, 1), (64, 3, 2, 1, 1), (32, 2, 2, 0, 1),
                                           (17, 5, 1, 2, 1), (20, 3, 1, 2, 2), (9, 3, 3, 0, 1)])
