@@ -215,6 +215,13 @@ int ssc_rulebook_conv_finish(const ssc_geometry *g, int64_t n_in, int32_t *n_out
  * kind of the geometry it is given.  Returns SSC_OK. */
 int32_t ssc_rulebook_kind(const ssc_geometry *g);
 int ssc_conv_expect(int32_t kind);
+/* The form a plan over float rows would take (host arithmetic only, no GPU needed): the pairs
+ * of an offset to a block of its schedule -- 16: the float form; 32, 64: the form on bfloat16
+ * parts -- and the bytes of its plan and scratch, which are at most what ssc_conv_plan_bytes and
+ * ssc_conv_plan_scratch_bytes say for n_out rows or more. */
+int ssc_conv_form(int32_t kind, int64_t n_in, int64_t n_out, int32_t kernel_volume, int32_t c_in,
+                  int32_t c_out, int64_t pair_stride, int32_t *block, size_t *plan_bytes,
+                  size_t *scratch_bytes);
 
 size_t ssc_conv_workspace_bytes(int64_t n_out, int32_t kernel_volume, int32_t c_in,
                                 int32_t c_out, int64_t pair_stride);

@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(256)
 // segments for a regular grid of `granule` rows (grid_segments_kernel).
 // Also spill[t*K + k] = how far the last row block of tile t-1 may reach into tile t:
 // the first pair at or after segs[t*K + k], at most blk - 1 further, whose row is >=
-// spill_end[t] (blk: pairs of an offset to a block, 16 or 32).
+// spill_end[t] (blk: pairs of an offset to a block, 16, 32 or 64).
 __global__ void __launch_bounds__(256)
     tile_segments_kernel(const int32_t *__restrict__ flag, const int32_t *__restrict__ pairs,
                          const int32_t *__restrict__ sorted, int64_t pair_stride, int plane_s,
@@ -1239,29 +1239,47 @@ static void plan_split(ConvPlan &p, int n_wg, int n_rng, int64_t n_out, int K,
   p.grp_cap = plan_groups(p.n_tiles, n_out, K, pair_stride, p.blk);
 }
 
+// What ssc_rulebook_kind tells of a rulebook: in the upper bits how many of its input rows there are
+// to a pair of an offset, in the lower two how the pairs lie.  0: nothing is known.
+enum { kPairsEven = 1, kPairsStrided = 2, kPairsSubm = 3 };
+
 // Pairs of an offset to a block of the parts form for a convolution of n_out rows over n_wg
 // workgroups and tiles of tile32 / tile64 rows, 0: the float form.  What decides is how many pairs
 // an offset has in a tile (each offset's last block of a tile is padded), which the rows and the
-// kind of the rulebook tell: a convolution of unit stride pairs nearly every input row with
-// an output row under every offset, a strided one an eighth of them (stride 2).  Microseconds of
-// the kernel, float form / blocks of 32 / of 64, 3^3 offsets:
-//    pairs of an offset in a tile                                     channels
-//     11  (unit, gradient)  22 / 30 / 46       28  (unit)  290 / 338 / 561    64 -> 128
-//     24  (stride 2)        45 / 36 / 47       38  (unit)  158 / 155 / 228    64 -> 304
-//     28  (stride 2)       152 / 120 / 219     55  (unit)  419 / 312 / 452   128 -> 256
-//     35  (stride 2)       239 / 183 / 206     57  (unit)   46 /  39 /  43    64 -> 64
-//     57  (every row)       39 /  31 /  28     88  (stride 2) 1396 / 1057 / 943   128 -> 304
-//    110  (unit)          6880 / 5600 / 4520  216  (every row) 287 / 215 / 189   128 -> 64
-// Of a strided layer an output row has the offsets of its parity only, so that the pairs of a
-// tile bunch; where every row has every offset the blocks but the last one are full.
+// kind of the rulebook tell: a convolution of unit stride, and a transposed one, pair nearly every
+// input row with an output row under every offset, a strided one as many of them as the
+// product of its strides says (1 in 8, 1 in 27).  Submanifold rulebooks pair 1 in 2 to 1 in 7 on
+// surfaces, 1 in 22 (kernel 3) to 1 in 65 (kernel 5) on scattered voxels; they, and rulebooks of
+// which nothing is known, count as strided by 2 -- the latter with no fewer pairs than their
+// output rows need.  Microseconds of the kernel, float form / blocks of 32 / of 64:
+//   pairs expected of an offset in a tile                            offsets  channels
+//     10  (stride 3, gradient)   25 /  30 /  46                           27  128 -> 128
+//     13  (stride 2)            219 / 257 / 443    8  (stride 3) 85 / 113 / 195   125   64 -> 128
+//     15  (stride 2, gradient)   80 /  65 / 102   17  (stride 3) 40 /  33 /  47   27  304, 128 -> 128
+//     21  (stride 2)             95 / 129 / 210                          125   64 -> 128
+//     26  (stride 2)             49 /  45 /  66   34  (stride 2) 83 /  70 / 103   27   64 -> 128
+//     26  (unit)                301 / 349 / 527   34  (unit)    576 / 524 / 743   27   64 -> 128
+//     26  (unit)               1435 / 1320 / 2052                         27  128 -> 304
+//     31  (transposed by 2)    1019 / 739 / 744                           27  128 -> 128
+//     51  (stride 2)             42 /  37 /  35                           27   64 -> 128
+//    147  (stride 2)           1839 / 1382 / 1223                         27  128 -> 304
+//    296  (every row)           282 / 213 / 185                           27  128 -> 64
+//     37  (submanifold)          53 /  47 /  60   37  (same, scattered) 32 / 34 / 51  27   64 -> 128
+// With one chunk of channels to a group every 64 pairs cost a read and a write of the
+// accumulators, so padding costs more than with several (23 against 14 pairs).  Of a strided layer
+// an output row has the offsets of its parity only, so that the pairs of a tile bunch, and blocks
+// fill better than under unit stride (34); where every row has every offset the blocks but the last
+// one are full.
 constexpr int kPartsMost32 = 10, kPartsMost64 = 4;
-static int parts_block(int64_t n_in, int64_t n_out, int64_t pair_stride, bool unit, int n_wg,
-                       int tile32, int tile64) {
+static int parts_block(int64_t n_in, int64_t n_out, int K, int64_t pair_stride, int32_t kind,
+                       int nch, int n_wg, int tile32, int tile64) {
   const bool inverse = pair_stride == n_out && n_in != n_out;
   const int64_t rb_in = pair_stride, rb_out = inverse ? n_in : n_out;
   if (n_out > kPartsMost32 * rb_in) return 0;  // (what buffers are sized for; no rule below comes near)
-  if (rb_out > 4 * rb_in) unit = true;  // (a stride of 2 makes 3.4 rows of one at most)
-  const double fill = std::min(1.0, (unit ? 1.0 : 0.125) * (double)rb_in / (double)n_out);
+  const double per_pair = (kind >> 2) > 0
+                              ? (double)(kind >> 2)
+                              : std::min(8.0, (double)K * (double)rb_in / (double)rb_out);
+  const double fill = std::min(1.0, (double)rb_in / (per_pair * (double)n_out));
   const double rows = (double)n_out / n_wg;
   const double in32 = fill * std::min(rows, (double)tile32), in64 = fill * std::min(rows, (double)tile64);
   if (fill >= 0.8 && rows < tile64) {
@@ -1270,17 +1288,15 @@ static int parts_block(int64_t n_in, int64_t n_out, int64_t pair_stride, bool un
   } else if (in64 >= 72.0 && n_out <= kPartsMost64 * rb_in) {
     return 64;
   }
-  return in32 >= (unit ? 34.0 : 20.0) ? 32 : 0;
+  const int lie = kind & 3;
+  const double least = lie == kPairsEven ? 34.0 : lie == kPairsStrided ? (nch > 1 ? 14.0 : 23.0) : 20.0;
+  return in32 >= least ? 32 : 0;
 }
-
-// What ssc_rulebook_kind says of a rulebook: of a regular convolution of unit stride, or nothing.
-constexpr int32_t kKindUnit = 1;
 
 // kind: of the rulebook (ssc_rulebook_kind).
 static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_out,
                           int64_t pair_stride, int elem_bytes = 4, int32_t kind = 0,
                           bool allow_parts = true) {
-  const bool unit = kind == kKindUnit;
   ConvPlan p;
   p.ncb = (int)ceil_div(c_out, 16);
   p.nch = (int)ceil_div(c_in, kKC);
@@ -1314,7 +1330,7 @@ static ConvPlan make_plan(int64_t n_in, int64_t n_out, int K, int c_in, int c_ou
     const int cols = (int)ceil_div(p.ncb, p.ncw);
     const int blk = g_conv_parts_blk > 0
                         ? g_conv_parts_blk
-                        : parts_block(n_in, n_out, pair_stride, unit,
+                        : parts_block(n_in, n_out, K, pair_stride, kind, p.nch,
                                       std::min(256, std::max(1, device_cu_count() / cols)),
                                       pick_tile(64, 32, true) - kSpillRowsParts,
                                       pick_tile(64, 64, true) - kSpillRowsParts);
@@ -2049,14 +2065,32 @@ int ssc_conv_fwd_f16(const void *features, int64_t n_in, int32_t c_in, const voi
 }
 
 int32_t ssc_rulebook_kind(const ssc_geometry *g) {
-  if (g == nullptr || g->subm || g->transpose) return 0;
-  for (int a = 0; a < 3; ++a)
-    if (g->stride[a] != 1) return 0;
-  return kKindUnit;
+  if (g == nullptr) return 0;
+  if (g->subm) return 8 << 2 | kPairsSubm;
+  int64_t strides = 1;
+  for (int a = 0; a < 3; ++a) {
+    if (g->stride[a] < 1) return 0;
+    strides = std::min<int64_t>(strides * g->stride[a], 1 << 20);
+  }
+  return (int32_t)(g->transpose ? 1 : strides) << 2 | (strides > 1 ? kPairsStrided : kPairsEven);
 }
 
 int ssc_conv_expect(int32_t kind) {
   g_expected_kind = kind;
+  return SSC_OK;
+}
+
+int ssc_conv_form(int32_t kind, int64_t n_in, int64_t n_out, int32_t kernel_volume, int32_t c_in,
+                  int32_t c_out, int64_t pair_stride, int32_t *block, size_t *plan_bytes,
+                  size_t *scratch_bytes) {
+  int rc = conv_check_sizes(kernel_volume, c_in, c_out, n_in, n_out, pair_stride);
+  if (rc != SSC_OK) return rc;
+  SSC_CHECK(n_in > 0 && n_out > 0 && pair_stride > 0 && block && plan_bytes && scratch_bytes,
+            SSC_EINVAL, "bad argument");
+  const ConvPlan p = make_plan(n_in, n_out, kernel_volume, c_in, c_out, pair_stride, 4, kind);
+  *block = p.blk;
+  *plan_bytes = conv_plan_walk(nullptr, p, nullptr);
+  *scratch_bytes = conv_scratch_walk(nullptr, p, kernel_volume, pair_stride, nullptr);
   return SSC_OK;
 }
 
@@ -2192,8 +2226,9 @@ int ssc_rulebook_conv_begin(const int32_t *indices, int64_t n_in, const ssc_geom
     ConvWs w = {};
     const size_t head = conv_scratch_head(scratch, &w);
     // (the form depends on the number of outputs as well, and with it the number of ranges of
-    // layers with a lone last column group: the guess is a scattered cloud's)
-    const ConvPlan more = make_plan(n_in, 10 * n_in + 1, (int)K, c_in, c_out, n_in, elem_bytes, kind);
+    // layers with a lone last column group: the guess is the float form, a scattered cloud's)
+    const ConvPlan more =
+        make_plan(n_in, n_in + 1, (int)K, c_in, c_out, n_in, elem_bytes, kind, false);
     const ConvPlan fewer =
         make_plan(n_in, n_in > 1 ? n_in - 1 : 1, (int)K, c_in, c_out, n_in, elem_bytes, kind);
     const bool more_ok = !more.rebalance && !more.small;

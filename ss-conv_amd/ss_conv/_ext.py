@@ -60,6 +60,8 @@ _SIGNATURES = {
     "ssc_conv_packed_bytes": (_sz, [_i32, _i32, _i32]),
     "ssc_rulebook_kind": (_i32, [_vp]),
     "ssc_conv_expect": (ctypes.c_int, [_i32]),
+    "ssc_conv_form": (ctypes.c_int, [_i32, _i64, _i64, _i32, _i32, _i32, _i64, ctypes.POINTER(_i32),
+                                     ctypes.POINTER(_sz), ctypes.POINTER(_sz)]),
     "ssc_conv_tile_cut": (ctypes.c_int, [_i32, _i32, _i32, ctypes.POINTER(_i32),
                                          ctypes.POINTER(_i32), ctypes.POINTER(_i32)]),
     "ssc_conv_plan_build": (ctypes.c_int, [_vp, _i64, _vp, _i32, _i32, _i32, _i64, _i64, _i32, _i32,

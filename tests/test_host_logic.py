@@ -146,6 +146,87 @@ def test_sizes_carry_no_flags():
     assert lib.ssc_conv_expect(0) == 0
 
 
+def _rulebook_sizes(idx, grid, k, s):
+    """Rows and pairs of an offset (mean) of a convolution of kernel k, stride s, padding k // 2."""
+    out = (grid + 2 * (k // 2) - k) // s + 1
+    keys = []
+    for off in np.ndindex(k, k, k):
+        o = idx[:, 1:] + k // 2 - np.array(off)
+        ok = (o % s == 0).all(1) & (o >= 0).all(1) & (o // s < out).all(1)
+        o = o[ok] // s
+        keys.append(((idx[ok, 0] * out + o[:, 0]) * out + o[:, 1]) * out + o[:, 2])
+    keys = np.concatenate(keys)
+    return len(np.unique(keys)), len(keys) / k ** 3
+
+
+def _conv_form(geometry, n_in, n_out, K, c_in, c_out, stride):
+    from ss_conv import _ext
+    kind = 0 if geometry is None else _ext._lib.ssc_rulebook_kind(ctypes.byref(geometry))
+    blk, plan, scratch = ctypes.c_int32(), ctypes.c_size_t(), ctypes.c_size_t()
+    assert _ext._lib.ssc_conv_form(kind, n_in, n_out, K, c_in, c_out, stride, ctypes.byref(blk),
+                                   ctypes.byref(plan), ctypes.byref(scratch)) == 0
+    return blk.value, plan.value, scratch.value
+
+
+@pytest.mark.parametrize("clouds,points,grid", [(16, 1024, 64), (16, 2048, 128), (32, 4096, 32),
+                                                (8, 4096, 20)])
+def test_form_follows_the_pairs_of_an_offset(clouds, points, grid):
+    """The form a plan takes against the pairs that an offset really has in a workgroup's tile:
+    the float form where they are few, whatever kernel and stride made them few; larger blocks
+    where they are many; in both directions."""
+    import synth
+    from ss_conv import _ext
+    pts, _, ids = synth.make_clouds(clouds, points, seed=1)
+    idx = synth.voxel_indices(pts, ids, grid)
+    n_in, seen = len(idx), set()
+    for k, s in [(3, 1), (3, 2), (3, 3), (3, 4), (5, 1), (5, 2), (5, 3), (5, 4), (2, 2), (4, 4)]:
+        n_out, pairs = _rulebook_sizes(idx, grid, k, s)
+        out = (grid + 2 * (k // 2) - k) // s + 1
+        g = _ext._geometry(clouds, [out] * 3, [k] * 3, [s] * 3, [k // 2] * 3, [1] * 3, 0, 0)
+        for ci, co in ((64, 128), (128, 64)):
+            for a, b, rows_in, rows in ((ci, co, n_in, n_out), (co, ci, n_out, n_in)):
+                per_wg = rows / (256 // -(-b // 64))
+                in_tile = pairs / rows * min(per_wg, 296)
+                blk = _conv_form(g, rows_in, rows, k ** 3, a, b, n_in)[0]
+                seen.add(blk)
+                if in_tile < 12:
+                    assert blk == 16, (k, s, a, b, in_tile)
+                if in_tile < 40:
+                    assert blk < 64, (k, s, a, b, in_tile)
+                if in_tile > 60:
+                    assert blk > 16, (k, s, a, b, in_tile)
+    assert 16 in seen and max(seen) > 16
+
+
+def test_no_plan_outgrows_what_callers_allocate():
+    """Every form's plan fits the sizes that follow from the number of output rows alone, also at
+    the ratios of rows up to which the rule takes a form."""
+    from ss_conv import _ext
+    lib = _ext._lib
+    rng = np.random.default_rng(3)
+    kinds = [None] + [_ext._geometry(1, [64] * 3, [3] * 3, [s] * 3, [1] * 3, [1] * 3, sub, tr)
+                      for s in (1, 2, 3) for sub, tr in ((0, 0), (0, 1), (1, 0))]
+    seen = set()
+    for it in range(1500):
+        stride = int(np.exp(rng.uniform(0, np.log(3e6))))
+        ratio = [3.999, 4.0, 4.001, 9.999, 10.0, 10.001, rng.uniform(0.02, 27)][rng.integers(7)]
+        rows = max(1, int(stride * ratio) + int(rng.integers(-1, 2)))
+        K = int(rng.choice([8, 27, 27, 125]))
+        ci, co = (int(rng.choice([4, 64, 64, 72, 128, 128, 200, 256, 608])) for _ in range(2))
+        bound = rows + int(rng.integers(0, 3)) * rows // 2
+        room = (lib.ssc_conv_plan_bytes(bound, K, ci, co, stride),
+                lib.ssc_conv_plan_scratch_bytes(bound, K, ci, co, stride))
+        for n_in, n_out in ((stride, rows), (rows, stride)):
+            if n_out == stride:
+                room = (lib.ssc_conv_plan_bytes(n_out, K, ci, co, stride),
+                        lib.ssc_conv_plan_scratch_bytes(n_out, K, ci, co, stride))
+            blk, plan, scratch = _conv_form(kinds[rng.integers(len(kinds))], n_in, n_out, K, ci, co,
+                                            stride)
+            seen.add(blk)
+            assert plan <= room[0] and scratch <= room[1], (n_in, n_out, K, ci, co, stride, blk)
+    assert seen == {16, 32, 64}
+
+
 # ---- shape arithmetic and the tensor type ---------------------------------------------------
 @pytest.mark.parametrize("size,k,s,p,d", [(64, 3, 1, 1, 1), (64, 3, 2, 1, 1), (32, 2, 2, 0, 1),
                                           (17, 5, 1, 2, 1), (20, 3, 1, 2, 2), (9, 3, 3, 0, 1)])
