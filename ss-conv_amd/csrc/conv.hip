@@ -1283,8 +1283,16 @@ static int parts_block(int64_t n_in, int64_t n_out, int K, int64_t pair_stride, 
   const double rows = (double)n_out / n_wg;
   const double in32 = fill * std::min(rows, (double)tile32), in64 = fill * std::min(rows, (double)tile64);
   if (fill >= 0.8 && rows < tile64) {
+    // (with many offsets the ranges differ by more rows -- what the grid's border cuts off counts
+    // for more -- and the longest sets the pace.  Microseconds, 64 -> 64 channels, gradient:
+    //   60 rows to a range:  27 offsets 39 / 32 / 29, 125 offsets 161 / 169 / 210
+    //   57 rows              27          42 / 39 / 41, 125         162 / 161 / 211
+    //   53 rows              27          38 / 32 / 28, 125         160 / 128 / 144)
+    auto full64 = [](int64_t n) {
+      return ceil_div(n, 64) * 64 * 5 <= ceil_div(n, 32) * 32 * 6;
+    };
     const int64_t whole = (int64_t)in64 + 1;
-    if (whole >= 32 && ceil_div(whole, 64) * 64 * 5 <= ceil_div(whole, 32) * 32 * 6) return 64;
+    if (whole >= 32 && full64(whole) && (K <= 64 || full64(whole + 8))) return 64;
   } else if (in64 >= 72.0 && n_out <= kPartsMost64 * rb_in) {
     return 64;
   }

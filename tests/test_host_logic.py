@@ -198,6 +198,17 @@ def test_form_follows_the_pairs_of_an_offset(clouds, points, grid):
     assert 16 in seen and max(seen) > 16
 
 
+def test_form_of_ranges_of_about_64_rows():
+    """Where every row has every offset a block of 64 pairs must hold the longest range: with 125
+    offsets, whose ranges differ more, not where they are 64 rows long in the mean but for a few."""
+    from ss_conv import _ext
+    for k, rows, want in ((3, 59.6, 64), (5, 59.6, 32), (5, 56.9, 32), (5, 52.6, 64), (5, 114.3, 64),
+                          (5, 26.0, 16)):
+        n = int(rows * 256)
+        g = _ext._geometry(16, [64] * 3, [k] * 3, [1] * 3, [k // 2] * 3, [1] * 3, 0, 0)
+        assert _conv_form(g, 20 * n, n, k ** 3, 64, 64, n)[0] == want, (k, rows)
+
+
 def test_no_plan_outgrows_what_callers_allocate():
     """Every form's plan fits the sizes that follow from the number of output rows alone, also at
     the ratios of rows up to which the rule takes a form."""
