@@ -192,26 +192,25 @@ struct ConvEpilogue {
 };
 
 // ---- bfloat16 parts ---------------------------------------------------------------------
-// An element of a float matrix as three bfloat16 parts that add up to it: the element rounded,
-// what is left rounded, and the rest.  The matrix cores multiply bfloat16 sixteen times as fast
-// as floats; of the nine products of parts six are taken (the ones left out are below 2^-24 of
-// the product).
+// An element of a float matrix, times 2^16, as three bfloat16 parts that add up to it: the element
+// rounded, what is left rounded, and the rest (the last bit of a float is 2^-149, that of a bfloat16
+// 2^-133).  The matrix cores multiply bfloat16 sixteen times as fast as floats; of the nine products
+// of parts six are taken (the ones left out are below 2^-24 of the product).
 // What the parts cannot do (PartsCheck::odd) and what then happens: see the parts form below.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 struct PartsCheck {
   float nan;       // NaN once a sum was not finite (0 times it is NaN)
   uint32_t least;  // smallest magnitude of a sum that is not zero: (bits << 1) - 1
-  uint32_t rest;   // OR of the words of which third parts were made
   __device__ __forceinline__ void sum(float v) {
     least = min(least, (__builtin_bit_cast(uint32_t, v) << 1) - 1u);
     nan = __builtin_fmaf(v, 0.f, nan);
   }
   __device__ __forceinline__ bool odd() const {
-    return nan != 0.f || (rest & 0xFFFFu) != 0 || least < ((127u - 95u) << 24) - 1u;
+    return nan != 0.f || least < ((127u - 94u) << 24) - 1u;
   }
 };
-// Two elements' parts, each pair of parts packed into a word.  (What a part leaves by the dot
+// Elements' parts, each two of them packed into a word.  (What a part leaves by the dot
 // product of a bfloat16 pair: it holds the matrix cores up for its time, which shift, mask and
 // subtraction do not -- 48 matrix instructions of a wave beside 112 others of another one: 812
 // cycles alone, 1392 with dot products, 900 with subtractions -- but those are twice as many, and
@@ -226,18 +225,33 @@ struct PartsCut {
     m0 = __builtin_bit_cast(bf16x2, minus0);
     m1 = __builtin_bit_cast(bf16x2, minus1);
   }
-  __device__ __forceinline__ void two(float u, float v, int &hi, int &mid, int &lo,
-                                      uint32_t &rest) const {
-    const bf16x2 a = __builtin_convertvector(float2v{u, v}, bf16x2);
-    hi = __builtin_bit_cast(int, a);
-    u = __builtin_amdgcn_fdot2_f32_bf16(a, m0, u, false);
-    v = __builtin_amdgcn_fdot2_f32_bf16(a, m1, v, false);
-    const bf16x2 b = __builtin_convertvector(float2v{u, v}, bf16x2);
-    mid = __builtin_bit_cast(int, b);
-    u = __builtin_amdgcn_fdot2_f32_bf16(b, m0, u, false);
-    v = __builtin_amdgcn_fdot2_f32_bf16(b, m1, v, false);
-    rest |= __builtin_bit_cast(uint32_t, u) | __builtin_bit_cast(uint32_t, v);
-    lo = __builtin_bit_cast(int, __builtin_convertvector(float2v{u, v}, bf16x2));
+  // (step by step over all of them: a pair's own steps each wait for the one before, and one pair
+  // after the other makes the kernel 7-9 % slower)
+  template <int N>
+  __device__ __forceinline__ void all(const float4v (&v)[N], int2v (&p)[N][3]) const {
+    float4v u[N];
+    bf16x2 part[N][2];
+#pragma unroll
+    for (int j = 0; j < N; ++j) u[j] = v[j] * kPartsScale;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        part[j][0] = __builtin_convertvector(float2v{u[j].x, u[j].y}, bf16x2);
+        part[j][1] = __builtin_convertvector(float2v{u[j].z, u[j].w}, bf16x2);
+        p[j][i] = int2v{__builtin_bit_cast(int, part[j][0]), __builtin_bit_cast(int, part[j][1])};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (i == 2) break;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        u[j].x = __builtin_amdgcn_fdot2_f32_bf16(part[j][0], m0, u[j].x, false);
+        u[j].y = __builtin_amdgcn_fdot2_f32_bf16(part[j][0], m1, u[j].y, false);
+        u[j].z = __builtin_amdgcn_fdot2_f32_bf16(part[j][1], m0, u[j].z, false);
+        u[j].w = __builtin_amdgcn_fdot2_f32_bf16(part[j][1], m1, u[j].w, false);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 };
 // Staged rows in LDS: two stages of 2 blk pairs x 32 channels x 3 parts (blk: pairs to a block).
@@ -340,7 +354,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
   const int col0 = col_base + cblk * kCN;
   static_assert(FORM == 0 || (NCW == 4 && !kHalf), "the other forms are built for float");
   static_assert(!PARTS || (NS == 16 && GATHER != 0), "the parts form: whole chunks, buffer loads");
-  PartsCheck check = {0.f, 0xFFFFFFFFu, 0u};  // (the parts form: what its sums and elements showed)
+  PartsCheck check = {0.f, 0xFFFFFFFFu};  // (the parts form: what its sums showed)
+  float unscale = PARTS ? 1.f / (kPartsScale * kPartsScale) : 1.f;  // of the accumulators
 
   {
     float4v z = {0.f, 0.f, 0.f, 0.f};
@@ -506,8 +521,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
               check.sum(x0);
               check.sum(x1);
             }
-            a0[e.gcl] = gate_act(x0);
-            if (two) a1[e.gcl] = gate_act(x1);
+            a0[e.gcl] = gate_act(PARTS ? x0 * unscale : x0);
+            if (two) a1[e.gcl] = gate_act(PARTS ? x1 * unscale : x1);
           }
           __builtin_amdgcn_sched_barrier(0);
           float4v v0 = own ? *reinterpret_cast<float4v *>(a0 + c_t) : z, v1 = z, g1 = z;
@@ -523,6 +538,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
               const bool stored = (e.mg[i] & 15) != 3;
               check.sum(stored ? v0[i] : 0.f);
               check.sum(stored ? v1[i] : 0.f);
+              v0[i] *= unscale;
+              v1[i] *= unscale;
             }
           }
           __builtin_amdgcn_sched_barrier(0);  // the clears stay behind every read above
@@ -600,7 +617,10 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
             *ap = z;
             if constexpr (PARTS) {
 #pragma unroll
-              for (int i = 0; i < 4; ++i) check.sum(v[u][i]);
+              for (int i = 0; i < 4; ++i) {
+                check.sum(v[u][i]);
+                v[u][i] *= unscale;
+              }
             }
           }
 #pragma unroll
@@ -618,7 +638,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
         if (sl >= T) sl -= T;
         if constexpr (PARTS) check.sum(acc[sl * kAS + c]);
         if (col0 + c < cout)
-          __builtin_nontemporal_store((IO)acc[sl * kAS + c], out + (int64_t)(row0 + r) * cout + col0 + c);
+          __builtin_nontemporal_store((IO)(PARTS ? acc[sl * kAS + c] * unscale : acc[sl * kAS + c]),
+                                      out + (int64_t)(row0 + r) * cout + col0 + c);
         acc[sl * kAS + c] = 0.f;
       }
     }
@@ -653,11 +674,13 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
   //
   // What the parts cannot do is worked out again with float instructions: a workgroup that has
   // met one of the following walks its groups a second time (see the end of the form).
-  //  - Infinities, NaN, and floats that round to an infinity as bfloat16: a sum not finite.
-  //  - Elements with bits below 2^-133, the last of a bfloat16: of a row, what is left for the
-  //    third part is a bfloat16 then and only then if the lower half of its word is zero; of
-  //    the filters, a NaN stands in their place.
-  //  - Sums that are not zero and below 2^-95: six products of parts, each rounded at 2^-150.
+  //  - Infinities, NaN, elements of 2^111 and sums of 2^95 or more (an infinity among the scaled
+  //    parts): a sum not finite.
+  //  - Sums that are not zero and below 2^-126 (scaled: 2^-94): six products of parts, each rounded
+  //    at 2^-150.
+  // (Without the scale elements with bits below 2^-133 and sums below 2^-95 went that way too, and
+  // one such element sent a workgroup through its range a second time: 128 -> 64 channels, every row,
+  // 756 us with a single one and 936 with one in every workgroup, where the float form takes 283.)
   //
   // What bounds it (128 -> 64 channels, 216 stages of 48 matrix instructions a wave, 185 us): a
   // stage is 788 cycles of matrix instructions and takes about 1800; LDS (48 reads of a KiB at 4-8
@@ -728,18 +751,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
       };
       auto store_rows = [&](int buf, const float4v (&v)[NB]) __attribute__((always_inline)) {
         int2v p[NB][3];
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          int h, m, l;
-          cut.two(v[j].x, v[j].y, h, m, l, check.rest);
-          p[j][0].x = h;
-          p[j][1].x = m;
-          p[j][2].x = l;
-          cut.two(v[j].z, v[j].w, h, m, l, check.rest);
-          p[j][0].y = h;
-          p[j][1].y = m;
-          p[j][2].y = l;
-        }
+        cut.all(v, p);
         char *dst = st_base + buf * kStageB;
 #pragma unroll
         for (int j = 0; j < NB; ++j)
@@ -1000,6 +1012,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
     if (check.odd()) odd_s[0] = 1;
     __syncthreads();
     if (odd_s[0] == 0) return;
+    unscale = 1.f;
     // The workgroup's tiles again, on float instructions: consumer wave w has columns 16 w .. of
     // the 64 and walks the row blocks in order, operands straight from memory.  Rare, and slower
     // than the float form.

@@ -26,25 +26,25 @@ struct PackArgs {
 // of step s has the channels 32 s + 4 g .. + 3 and 32 s + 16 + 4 g .. + 3 of the chunk, the ones it
 // has in the float fragments 2 s and 2 s + 1.
 constexpr int kPartFragBytes = 2 * 3 * 1024;
-// Element idx of the packed filters, value v.  An element that is not the sum of its parts (bits
-// below 2^-133; floats that round to an infinity) gets a NaN for its first part: every sum it
-// is in is refused and worked out again with the float fragments (infinities and NaN do so by
-// themselves).
+// Rows and filters are scaled by this before they are cut, the sums by its inverse squared: parts
+// then hold every bit of every float.  All exact.
+constexpr float kPartsScale = 0x1p16f;
+// Element idx of the packed filters, value v.  (What is too large for it is an infinity, and every
+// sum it is in is refused and worked out again with the float fragments.)
 __device__ __forceinline__ void pack_parts_element(const PackArgs &a, int64_t idx, float v) {
   const int64_t frag = idx >> 10;
   const int f = (int)(idx & 1023), q = f >> 8, lane = (f >> 2) & 63, j = f & 3;
   __bf16 *dst = reinterpret_cast<__bf16 *>(static_cast<char *>(a.packed_out) +
                                            (int64_t)a.K * a.ncb * a.nch * 4096 + frag * kPartFragBytes) +
                 ((q >> 1) * 3 * 64 + lane) * 8 + (q & 1) * 4 + j;
-  __bf16 hi = (__bf16)v;
+  v *= kPartsScale;
+  const __bf16 hi = (__bf16)v;
   float left = v - (float)hi;
   const __bf16 mid = (__bf16)left;
   left -= (float)mid;
-  const __bf16 lo = (__bf16)left;
-  if ((float)lo != left) hi = (__bf16)__builtin_nanf("");
   dst[0] = hi;
   dst[64 * 8] = mid;
-  dst[2 * 64 * 8] = lo;
+  dst[2 * 64 * 8] = (__bf16)left;
 }
 
 // Offset k, input channel ci and output channel co of element idx of the packed filters

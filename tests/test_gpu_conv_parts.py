@@ -130,6 +130,39 @@ def test_parts_cannot(what, blk, device):
 
 
 @pytest.mark.parametrize("blk", [32, 64])
+@pytest.mark.parametrize("where", ["rows", "filters", "scaled"])
+def test_parts_hold_every_bit(where, blk, device):
+    """Elements with bits down to the last one of a float, and sums far below those of ordinary
+    layers, are no reason to leave the form (whose sums differ from the float form's in their last
+    bits), and lose nothing in it."""
+    n_in, o_idx, pairs, num = _rulebook(700, 12, 3, 1, 7, device)
+    n_out = o_idx.shape[0]
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn(n_in, 64, generator=g), torch.randn(3, 3, 3, 64, 72, generator=g)
+    plain = _conv(x.to(device), w.to(device), pairs, num, n_out, False, BLOCKS[blk])
+    if where == "scaled":  # elements with bits below 2^-133, sums of 2^-100
+        for a, b in ((-105, 0), (0, -105), (-52, -53)):
+            y = _conv((x * 2.0 ** a).to(device), (w * 2.0 ** b).to(device), pairs, num, n_out, False,
+                      BLOCKS[blk])
+            assert torch.equal(y * 2.0 ** 105, plain), (a, b)
+        return
+    some = torch.rand((n_in, 64) if where == "rows" else w.shape, generator=g) < 0.01
+    (x if where == "rows" else w)[some] = 0.0
+    none = _conv(x.to(device), w.to(device), pairs, num, n_out, False, BLOCKS[blk])
+    assert not torch.equal(none, _conv(x.to(device), w.to(device), pairs, num, n_out, False, FLOAT))
+    (x if where == "rows" else w)[some] = 2.0 ** -130 * 1.2345  # next to nothing beside the others
+    assert torch.equal(none, _conv(x.to(device), w.to(device), pairs, num, n_out, False, BLOCKS[blk]))
+    # rows (columns) of nothing but such elements, far from where the others' sums are
+    (x if where == "rows" else w.view(-1, 72))[::2] = 2.0 ** -148 * torch.randint(1, 1 << 20, (64 if where == "rows" else 72,), generator=g)
+    if where == "filters":
+        w[:] = w.view(-1, 72)[0]
+        x = x.abs()
+    y = _conv(x.to(device), w.to(device), pairs, num, n_out, False, BLOCKS[blk]).cpu()
+    ref = _reference(x, w, pairs, num, n_out, False)
+    assert ((y.double() - ref).norm(dim=1) <= TOL * ref.norm(dim=1) + 64 * 27 * 2.0 ** -150).all()
+
+
+@pytest.mark.parametrize("blk", [32, 64])
 @pytest.mark.parametrize("odd", [False, True])
 def test_parts_with_epilogue(blk, odd, device):
     """Batch norm and gate on the way out, also where the rows are worked out a second time."""
