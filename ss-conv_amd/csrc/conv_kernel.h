@@ -1014,8 +1014,9 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
     if (odd_s[0] == 0) return;
     unscale = 1.f;
     // The workgroup's tiles again, on float instructions: consumer wave w has columns 16 w .. of
-    // the 64 and walks the row blocks in order, operands straight from memory.  Rare, and slower
-    // than the float form.
+    // the 64 and walks the row blocks in order, operands straight from memory.  Rare, and 3.4 times
+    // as slow as the float form; its sums are no further off (128 -> 64 channels, every row: 1.8e-7
+    // against 2.0e-7; with all chunks of a group in one chain 2.3e-7).
     {
       const int g = lane >> 4, l16 = lane & 15;
       const int w_base = min(col0 / 16 + (producer ? 0 : wave), ncb - 1) * nch * 4096;
@@ -1034,7 +1035,7 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
           for (int cc = 0; cc < nch; ++cc)
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-              float4v av[4], wv[4];
+              float4v av[4], wv[4], t = {0.f, 0.f, 0.f, 0.f};  // (a chunk's products by themselves)
 #pragma unroll
               for (int q = 0; q < 4; ++q) {
                 int off = in_off[b];
@@ -1046,7 +1047,8 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
               for (int q = 0; q < 4; ++q)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                  d[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q][j], av[q][j], d[b], 0, 0, 0);
+                  t = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q][j], av[q][j], t, 0, 0, 0);
+              d[b] += t;
             }
 #pragma unroll
           for (int b = 0; b < 4; ++b) {

@@ -130,6 +130,26 @@ def test_parts_cannot(what, blk, device):
 
 
 @pytest.mark.parametrize("blk", [32, 64])
+@pytest.mark.parametrize("ci,co", [(128, 64), (512, 72)])
+def test_second_walk_is_no_further_off(ci, co, blk, device):
+    """Rows that are worked out again because others of their workgroup are not finite: against
+    64 bits no further off than the float form's."""
+    n_in, o_idx, pairs, num = _rulebook(3000, 16, 3, 1, 9, device)
+    n_out = o_idx.shape[0]
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(n_in, ci, generator=g), torch.randn(3, 3, 3, ci, co, generator=g)
+    x[::100, 3] = float("inf")
+    x, w = x.to(device), w.to(device)
+    y = _conv(x, w, pairs, num, n_out, False, BLOCKS[blk]).cpu()
+    old = _conv(x, w, pairs, num, n_out, False, FLOAT).cpu()
+    ref = _reference(x, w, pairs, num, n_out, False)
+    fine = torch.isfinite(ref)
+    assert torch.equal(fine, torch.isfinite(y)) and 0.1 < fine.float().mean() < 0.99
+    err, was = (rel_l2(v[fine].numpy(), ref[fine].numpy()) for v in (y, old))
+    assert err <= 1.05 * was, (err, was)
+
+
+@pytest.mark.parametrize("blk", [32, 64])
 @pytest.mark.parametrize("where", ["rows", "filters", "scaled"])
 def test_parts_hold_every_bit(where, blk, device):
     """Elements with bits down to the last one of a float, and sums far below those of ordinary
