@@ -282,6 +282,18 @@ class RulebookMeta(object):
         self.pairs_ref = pairs_ref  # the tensor the plans were built over
         self.kind = kind  # ssc_rulebook_kind of its geometry
 
+    # Plans stay out of files (a SparseTensor saved whole brings its plan_dict): the form of a plan
+    # belongs to the library and the device that built it.  They are built anew on first use.
+    def __getstate__(self):
+        return {"version": self.version, "canonical": self.canonical,
+                "pairs_ref": self.pairs_ref, "kind": self.kind}
+
+    def __setstate__(self, state):
+        if isinstance(state, tuple):  # (files from before records had a state of their own)
+            state = state[1]
+        self.__init__(state["version"], state["canonical"], pairs_ref=state["pairs_ref"],
+                      kind=state.get("kind", 0))
+
     def get_plan(self, key):
         plan = self.plans.get(key)
         if plan is not None:

@@ -611,3 +611,29 @@ def test_modules_saved_whole_before_their_tables_grew():
     del ker._tables, norm._layout_cpu, norm._layout_dev  # files from before there were any
     assert pickle.loads(pickle.dumps(ker))._tables is None
     assert set(pickle.loads(pickle.dumps(norm)).layout("cpu")) == set(bnact.field_layout(rs))
+
+
+def test_rulebook_records_come_back_without_plans():
+    """What a SparseTensor keeps with a rulebook goes into files without the plans, whose form
+    belongs to the library that built them; records of earlier forms come back, also without
+    their plans, as rulebooks of which nothing is known."""
+    import pickle
+    from ss_conv import _ext
+    pairs = torch.zeros(27, 2, 5, dtype=torch.int32)
+    meta = _ext.RulebookMeta(0, (True, True), pairs_ref=pairs, kind=5)
+    meta.put_plan((False, 64, 64, 4, 5, 5, 1), torch.zeros(8, dtype=torch.uint8))
+    again = pickle.loads(pickle.dumps(meta))
+    assert len(again.plans) == 0 and again.kind == 5 and again.canonical == (True, True)
+    assert torch.equal(again.pairs_ref, pairs) and len(meta.plans) == 1
+    slots = {"version": 0, "canonical": (True, False), "plans": meta.plans, "pairs_ref": pairs}
+    for more in ({}, {"unit": 65536}):
+        old = _ext.RulebookMeta.__new__(_ext.RulebookMeta)
+        state = (None, dict(slots, **more))  # what pickle kept of an object with slots
+        if hasattr(old, "__setstate__"):
+            old.__setstate__(state)
+        else:
+            for k, v in state[1].items():
+                setattr(old, k, v)
+        assert len(old.plans) == 0 and old.kind == 0 and old.canonical == (True, False)
+        old.put_plan("key", pairs)
+        assert old.get_plan("key") is pairs
