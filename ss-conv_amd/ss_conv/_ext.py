@@ -339,6 +339,24 @@ def adopt_meta(indice_pairs, meta):
     return bound
 
 
+class _PackedCopies(tuple):
+    """(version of the tensor, {way of reading it: packed filters}), kept on the tensor.  A
+    parameter saved whole brings its attributes into the file: this one leaves it as None, since
+    the packed order belongs to the library that wrote it."""
+    __slots__ = ()
+
+    def __reduce_ex__(self, protocol):
+        return (type(None), ())
+
+
+def _packed_copies(owner):
+    """The packed copies that hold for a tensor's present values, by way of reading it."""
+    held = getattr(owner, "_ssc_packed", None)
+    if type(held) is not _PackedCopies or held[0] != owner._version:
+        held = owner._ssc_packed = _PackedCopies((owner._version, {}))
+    return held[1]
+
+
 def forget_packed(filters):
     """Drop the packed copy of `filters` that the convolution keeps with the tensor.  The
     copy is reused while the tensor's version counter stands still, and an edit through
@@ -699,16 +717,13 @@ def _packed_filters(owner, filters, fs, K, c_in, c_out, stream):
     layers, whose kernel is synthesised once, pack once."""
     flush_combine()
     key = (filters.data_ptr(), tuple(fs), K, c_in, c_out)
-    held = getattr(owner, "_ssc_packed", None)
-    if held is None or held[0] != owner._version:
-        held = (owner._version, {})
-        owner._ssc_packed = held
-    packed = held[1].get(key)
+    held = _packed_copies(owner)
+    packed = held.get(key)
     if packed is None:
         packed = _workspace(_lib.ssc_conv_packed_bytes(K, c_in, c_out), filters.device)
         _check(_ENTRIES[filters.dtype][1](_ptr(filters), fs[0], fs[1], fs[2], K, c_in, c_out,
                                          packed.data_ptr(), packed.numel(), stream))
-        held[1][key] = packed
+        held[key] = packed
     return packed
 
 
@@ -1467,8 +1482,8 @@ def attach_packed(filters, c_in, c_out, packed):
     K = 1
     for d in base.shape[:-2]:
         K *= d
-    filters._ssc_packed = (filters._version,
-                           {(base.data_ptr(), (fs_k, fs_ci, fs_co), K, c_in, c_out): packed})
+    filters._ssc_packed = _PackedCopies(
+        (filters._version, {(base.data_ptr(), (fs_k, fs_ci, fs_co), K, c_in, c_out): packed}))
 
 
 def voxel_coords(points, batch_ids, half_extent, unit):

@@ -637,3 +637,23 @@ def test_rulebook_records_come_back_without_plans():
         assert len(old.plans) == 0 and old.kind == 0 and old.canonical == (True, False)
         old.put_plan("key", pairs)
         assert old.get_plan("key") is pairs
+
+
+def test_packed_filters_stay_out_of_files():
+    """The packed copies that ride on a layer's filters do not come back from a module saved
+    whole, and those of a file from before are not used: another library packs them otherwise."""
+    import pickle
+    from ss_conv import _ext
+    from ss_conv.sp_ops.conv import SparseConvolution
+    layer = SparseConvolution(3, 8, 8, 3, bias=False)
+    held = _ext._packed_copies(layer.weight)
+    held["way"] = torch.zeros(4, dtype=torch.uint8)
+    assert _ext._packed_copies(layer.weight) is held and layer.weight._ssc_packed[1] is held
+    again = pickle.loads(pickle.dumps(layer))
+    assert torch.equal(again.weight, layer.weight) and not getattr(again.weight, "_ssc_packed", None)
+    assert _ext._packed_copies(again.weight) == {}
+    again.weight._ssc_packed = (again.weight._version, dict(held))  # the plain tuple of before
+    assert _ext._packed_copies(again.weight) == {}
+    with torch.no_grad():
+        layer.weight.add_(1)
+    assert _ext._packed_copies(layer.weight) == {}
