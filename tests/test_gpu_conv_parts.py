@@ -70,6 +70,76 @@ def test_parts_match_sums_in_64_bits(case, blk, device):
         assert torch.equal(y, _conv(x, w, pairs, num, out_rows, inverse, BLOCKS[blk]))
 
 
+# rulebooks other than a regular one in key order: stride, submanifold, transposed, what else
+OTHERS = {"stride 3": (3, 0, 0, ""), "stride 4": (4, 0, 0, ""), "submanifold": (1, 1, 0, ""),
+          "transposed": (2, 0, 1, ""), "rows in any order": (1, 0, 0, "rows"),
+          "pairs in any order": (1, 0, 0, "pairs"), "two ranges": (1, 0, 0, 128),
+          "second split": (1, 0, 0, 32)}
+
+
+@pytest.mark.parametrize("blk", [32, 64])
+@pytest.mark.parametrize("what", list(OTHERS))
+def test_parts_over_other_rulebooks(what, blk, device):
+    """Strides whose offsets have few pairs, submanifold and transposed rulebooks, input rows and
+    pairs in any order, two ranges of rows to a workgroup and the second split of the work: both
+    directions against sums in 64 bits."""
+    from ss_conv.sp_ops.ops import get_indice_pairs
+    s, subm, transpose, more = OTHERS[what]
+    rng = np.random.default_rng(11)
+    idx = random_voxels(rng, 2, 24, 6000)
+    if more == "rows":
+        idx = idx[rng.permutation(len(idx))]
+    idx = torch.from_numpy(idx).to(device)
+    o_idx, pairs, num = get_indice_pairs(idx, 2, [24] * 3, 3, s, 1, 1, 0, bool(subm), bool(transpose))
+    if more == "pairs":  # a tensor the library knows nothing of, each offset's pairs shuffled
+        pairs = pairs.clone()
+        for k, m in enumerate(num.cpu().tolist()):
+            pairs[k, :, :m] = pairs[k, :, torch.from_numpy(rng.permutation(m)).to(device)]
+    flags = BLOCKS[blk] | (more if isinstance(more, int) else 0)
+    g = torch.Generator().manual_seed(2)
+    w = torch.randn(3, 3, 3, 64, 72, generator=g).to(device)
+    n_in, n_out = idx.shape[0], o_idx.shape[0]
+    for inverse, rows, out_rows, c in ((False, n_in, n_out, 64), (True, n_out, n_in, 72)):
+        x = torch.randn(rows, c, generator=g).to(device)
+        y = _conv(x, w, pairs, num, out_rows, inverse, flags)
+        assert rel_l2(y.cpu().numpy(), _reference(x, w, pairs, num, out_rows, inverse).numpy()) < TOL
+        assert torch.equal(y, _conv(x, w, pairs, num, out_rows, inverse, flags))
+        if c == 64:  # (whole chunks: the form is taken)
+            assert not torch.equal(y, _conv(x, w, pairs, num, out_rows, inverse, FLOAT))
+
+
+def _without_plans(st):
+    """The same rows and rulebook under a record without plans: they are built from the pairs."""
+    from ss_conv import _ext
+    from ss_conv.sp_ops.tensor import SparseTensor
+    t = SparseTensor(st.features, st.indices, st.spatial_shape, st.batch_size)
+    t.indice_dict, t.plan_dict = st.indice_dict, {}
+    pairs, meta = st.indice_dict["a"][2], st.plan_dict["a"]
+    pairs._ssc_meta = _ext.RulebookMeta(pairs._version, meta.canonical, pairs_ref=pairs, kind=meta.kind)
+    return t
+
+
+def test_layer_over_a_rulebook_from_a_file(device):
+    """A sparse tensor saved whole and loaded again: its rulebook serves a layer as before."""
+    import io
+    from ss_conv.sp_ops.conv import SparseConvolution
+    from ss_conv.sp_ops.tensor import SparseTensor
+    torch.manual_seed(1)
+    layer = SparseConvolution(3, 64, 64, 3, padding=1, bias=False, indice_key="a").to(device).eval()
+    idx = torch.from_numpy(random_voxels(np.random.default_rng(4), 2, 20, 8000)).to(device)
+    st = SparseTensor(torch.randn(idx.shape[0], 64, device=device), idx, [20] * 3, 2)
+    with torch.no_grad():
+        y = layer(st)
+        file = io.BytesIO()
+        torch.save((st, layer), file)
+        file.seek(0)
+        st2, layer2 = torch.load(file, weights_only=False)
+        assert len(st2.plan_dict["a"].plans) == 0 < len(st.plan_dict["a"].plans)
+        z = layer2(st2)
+        assert rel_l2(z.features.cpu().numpy(), y.features.cpu().numpy()) < TOL
+        assert torch.equal(z.features, layer(_without_plans(st)).features)
+
+
 @pytest.mark.parametrize("blk", [32, 64])
 def test_parts_by_the_rule(blk, device):
     """Sizes at which the rule itself takes the form: the same bits as when it is forced."""
@@ -83,11 +153,12 @@ def test_parts_by_the_rule(blk, device):
 
 
 @pytest.mark.parametrize("blk", [32, 64])
-@pytest.mark.parametrize("what", ["inf", "nan", "both", "large", "tiny", "subnormal", "filter inf",
+@pytest.mark.parametrize("what", ["inf", "nan", "both", "large", "tiny", "tinier", "subnormal", "filter inf",
                                   "filter subnormal", "filter large"])
 def test_parts_cannot(what, blk, device):
-    """Elements that parts do not add up to, and sums that are not finite or next to nothing: the
-    workgroup that meets one works its rows out with float instructions."""
+    """Elements too large for the scaled parts, and sums that are not finite or next to nothing: the
+    workgroup that meets one works its rows out with float instructions.  Elements and sums that
+    only the scale keeps in reach of the parts."""
     n_in, o_idx, pairs, num = _rulebook(700, 12, 3, 1, 7, device)
     n_out = o_idx.shape[0]
     g = torch.Generator().manual_seed(3)
@@ -99,12 +170,15 @@ def test_parts_cannot(what, blk, device):
         x[torch.rand(n_in, 64, generator=g) < 2e-3] = -float("inf")
     if what == "nan":
         x[some] = float("nan")
-    if what == "large":  # rounds to an infinity as a bfloat16
+    if what == "large":  # an infinity as a scaled bfloat16
         x[some] = 3.4e38
         w *= 1e-3
-    if what == "tiny":  # sums below 2^-95 that are not zero
+    if what == "tiny":  # sums of 2^-110, whose parts' products are not rounded thanks to the scale
         x *= 2.0 ** -70
         w *= 2.0 ** -40
+    if what == "tinier":  # sums some of which are below 2^-126 and not zero
+        x *= 2.0 ** -64
+        w *= 2.0 ** -62
     if what == "subnormal":  # bits below 2^-133, next to nothing but times 2^100
         x *= 2.0 ** -125
         w *= 2.0 ** 100
@@ -183,9 +257,11 @@ def test_parts_hold_every_bit(where, blk, device):
 
 
 @pytest.mark.parametrize("blk", [32, 64])
-@pytest.mark.parametrize("odd", [False, True])
+@pytest.mark.parametrize("odd", [None, "inf", "nan", "large", "filter inf", "gate inf", "gate large"])
 def test_parts_with_epilogue(blk, odd, device):
-    """Batch norm and gate on the way out, also where the rows are worked out a second time."""
+    """Batch norm and gate on the way out, also where the rows are worked out a second time: sums
+    that are not finite, in a column that is stored and in a gate's, which relu and sigmoid may
+    hide (an infinity's parts are an infinity and NaNs)."""
     from ss_conv import _ext
     from ss_conv.activation import Activation
     from ss_conv.batchnorm import BatchNorm
@@ -199,17 +275,37 @@ def test_parts_with_epilogue(blk, odd, device):
                                     Activation(rs, (torch.relu, torch.sigmoid))).to(device).eval()
     idx = torch.from_numpy(random_voxels(np.random.default_rng(8), 2, 16, 1500)).to(device)
     x = torch.randn(idx.shape[0], 64, device=device)
-    if odd:
-        x[3, 5] = 2.0 ** -130 * 1.2345
+    with torch.no_grad():
+        w = block.conv.eval_weight(x)
+        if odd in ("inf", "nan"):
+            x[::200, 5] = float(odd)
+        if odd == "large":  # an infinity once scaled, the sums are none
+            x[::200, 5] = 3e38
+            w *= 1e-3
+        if odd == "filter inf":
+            w[1, 1, 2, 7, 40] = float("inf")
+        if odd == "gate inf":
+            w[1, 1, 2, 7, 128 + 3] = float("inf")
+        if odd == "gate large":
+            w[1, 1, 2, 7, 128 + 3] = 3e38
+            x *= 1e-3
     got = []
     for flags in (BLOCKS[blk], FLOAT):
         try:
             assert _ext._lib.ssc_conv_tuning(flags) == 0
             with torch.no_grad():
-                got.append(block(SparseTensor(x, idx, [16] * 3, 2)).features.cpu().numpy())
+                got.append(block(SparseTensor(x, idx, [16] * 3, 2)).features.cpu())
         finally:
             _ext._lib.ssc_conv_tuning(1)
-    assert rel_l2(got[0], got[1]) < 2e-6
+    assert torch.equal(torch.isnan(got[0]), torch.isnan(got[1]))
+    assert torch.equal(torch.isinf(got[0]) * got[0].sign(), torch.isinf(got[1]) * got[1].sign())
+    fine = torch.isfinite(got[1]) & (got[1].abs() < 1e4)
+    assert fine.float().mean() > 0.3 and rel_l2(got[0][fine].numpy(), got[1][fine].numpy()) < 2e-6
+    huge = torch.isfinite(got[1]) & ~fine
+    if odd in (None, "large"):
+        assert bool(huge.any()) == (odd == "large")
+    if huge.any():
+        assert rel_l2(got[0][huge].double().numpy(), got[1][huge].double().numpy()) < 2e-6
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
