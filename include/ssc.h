@@ -255,12 +255,13 @@ int ssc_conv_fwd_f16(const void *features /* [n_in,c_in] half */, int64_t n_in, 
  * its backward pass walks the same pairs again, src/conv/indice_conv.h:344-426):
  *   ssc_conv_plan_build: the row-block schedule of the kernel (what ssc_conv_fwd_* derives
  *     from the pairs on every call).  The plan stays valid while pairs, pair_num, n_out,
- *     kernel_volume, c_in, c_out, elem_bytes (4: float, 2: half), `inverse` and the number
- *     of feature rows n_in stay the same; `scratch` is needed during the call only.
+ *     kernel_volume, c_in, c_out, elem_bytes (4: float, 2: half), `inverse`, the number of
+ *     feature rows n_in and what ssc_conv_expect was told stay the same; `scratch` is needed during the call only.
  *     flags: SSC_CONV_PAIRS_CANONICAL as for ssc_conv_fwd_f32.
  *   ssc_conv_pack_filters_*: the filters in the kernel's fragment order; valid while the
  *     filter values stay the same.
- *   ssc_conv_run_*: the MFMA kernel alone.  Results are bit-identical to ssc_conv_fwd_*.
+ *   ssc_conv_run_*: the MFMA kernel alone.  Results are bit-identical to ssc_conv_fwd_* told
+ *     the same by ssc_conv_expect.
  * Pairs with one scatter row twice inside an offset are not supported by either form (a
  * rulebook never has them). */
 /* Both sizes grow with n_out (and never shrink for a smaller one): buffers sized for an

@@ -1252,19 +1252,28 @@ enum { kPairsEven = 1, kPairsStrided = 2, kPairsSubm = 3 };
 // surfaces, 1 in 22 (kernel 3) to 1 in 65 (kernel 5) on scattered voxels; they, and rulebooks of
 // which nothing is known, count as strided by 2 -- the latter with no fewer pairs than their
 // output rows need.  Microseconds of the kernel, float form / blocks of 32 / of 64:
-//   pairs expected of an offset in a tile                            offsets  channels
-//     10  (stride 3, gradient)   25 /  30 /  46                           27  128 -> 128
-//     13  (stride 2)            219 / 257 / 443    8  (stride 3) 85 / 113 / 195   125   64 -> 128
-//     15  (stride 2, gradient)   80 /  65 / 102   17  (stride 3) 40 /  33 /  47   27  304, 128 -> 128
-//     21  (stride 2)             95 / 129 / 210                          125   64 -> 128
-//     26  (stride 2)             49 /  45 /  66   34  (stride 2) 83 /  70 / 103   27   64 -> 128
-//     26  (unit)                301 / 349 / 527   34  (unit)    576 / 524 / 743   27   64 -> 128
-//     26  (unit)               1435 / 1320 / 2052                         27  128 -> 304
-//     31  (transposed by 2)    1019 / 739 / 744                           27  128 -> 128
-//     51  (stride 2)             42 /  37 /  35                           27   64 -> 128
-//    147  (stride 2)           1839 / 1382 / 1223                         27  128 -> 304
-//    296  (every row)           282 / 213 / 185                           27  128 -> 64
-//     37  (submanifold)          53 /  47 /  60   37  (same, scattered) 32 / 34 / 51  27   64 -> 128
+//   pairs expected of an offset in a tile                 offsets   channels
+//     8  (stride 3)                95 /  117 /  188           125   128 ->  64
+//    10  (stride 3, gradient)      25 /   31 /   47            27   128 -> 128
+//    13  (stride 2)               221 /  262 /  438           125    64 -> 128
+//    15  (stride 2, gradient)      81 /   64 /  104            27   304 -> 128
+//    17  (stride 3)                41 /   33 /   48            27   128 -> 128
+//    21  (stride 2)                93 /  130 /  207           125    64 -> 128
+//    26  (stride 2)                48 /   44 /   66            27    64 -> 128
+//    28  (stride 2, gradient)      47 /   42 /   47            27   128 ->  64
+//    28  (unit)                   280 /  336 /  496            27    64 -> 128
+//    26  (unit)                  1434 / 1302 / 2042            27   128 -> 304
+//    34  (unit)                   573 /  537 /  740            27    64 -> 128
+//    31  (transposed by 2)       1002 /  757 /  772            27   128 -> 128
+//    37  (stride 2, gradient)    1511 / 1201 / 1329            27   304 -> 128
+//    51  (stride 2)                42 /   38 /   36            27    64 -> 128
+//   121  (stride 2)              1342 / 1039 /  955            27   128 -> 304
+//   144  (stride 2)              1645 / 1195 / 1114            27   256 -> 608
+//   156  (unit)                  6623 / 5492 / 4540            27   512 -> 608
+//   223  (unit, every row)        274 /  207 /  187            27   128 ->  64
+//   296  (unit, every row)       6334 / 4509 / 4364            27   608 -> 512
+//    37  (submanifold)             52 /   46 /   59            27    64 -> 128
+//    32  (same, scattered)         33 /   37 /   49            27   128 ->  64
 // With one chunk of channels to a group every 64 pairs cost a read and a write of the
 // accumulators, so padding costs more than with several (23 against 14 pairs).  Of a strided layer
 // an output row has the offsets of its parity only, so that the pairs of a tile bunch, and blocks
@@ -1275,7 +1284,9 @@ static int parts_block(int64_t n_in, int64_t n_out, int K, int64_t pair_stride, 
                        int nch, int n_wg, int tile32, int tile64) {
   const bool inverse = pair_stride == n_out && n_in != n_out;
   const int64_t rb_in = pair_stride, rb_out = inverse ? n_in : n_out;
-  if (n_out > kPartsMost32 * rb_in) return 0;  // (what buffers are sized for; no rule below comes near)
+  // (what buffers are sized for; a transposed rulebook may have more output rows: 2133 / 1598 / 1877
+  // at 10.5 of them to an input row, 128 -> 128)
+  if (n_out > kPartsMost32 * rb_in) return 0;
   const double per_pair = (kind >> 2) > 0
                               ? (double)(kind >> 2)
                               : std::min(8.0, (double)K * (double)rb_in / (double)rb_out);

@@ -299,7 +299,9 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
   constexpr int kAS = kCN + (FIVE || WIDE ? 16 : 0) + 4;
   constexpr int NT = (NCW + 4) * 64;
   // threads that write a tile out (the parts form over blocks of 64 with the epilogue: the
-  // consumers only, the producers have no registers for it)
+  // consumers only.  With all waves 50 registers of the producers were spilled, 512 -> 608 channels
+  // 5.3 ms instead of 4.4; that was before rows were scaled, whose cut takes fewer of them, and has
+  // not been measured since)
   constexpr bool kProducersFlush = !(EPI && FORM == 5);
   constexpr int NTF = kProducersFlush ? NT : NCW * 64;
   constexpr int NP = 256;  // producer threads
@@ -685,17 +687,13 @@ __global__ void __launch_bounds__((NCW + 4) * 64)
   // What bounds it (128 -> 64 channels, 216 stages of 48 matrix instructions a wave, 185 us): a
   // stage is 788 cycles of matrix instructions and takes about 1800; LDS (48 reads of a KiB at 4-8
   // cycles, 48 writes of 512 bytes at 8) and the vector memory path (40 KiB at 64 bytes a cycle)
-  // are busy 600-700 cycles each, the producers' cutting 450, which share the SIMDs with the
+  // are busy 600-700 cycles each, the producers' cutting 450-500, which share the SIMDs with the
   // products; none of them alone sets the pace.  Blocks of 64 halve the fragment loads of a product
   // and the barriers, and pad more; four row blocks leave registers for two stages of fragments.
-  // Microseconds, float form -> blocks of 32 / of 64, and the error against 64 bits:
-  //   128 -> 64,  1.54M pairs, every row   287 ->  210 /  185    2.0e-7 -> 1.5e-7
-  //   128 -> 304, 1.69M pairs, stride 2   1396 -> 1063 /  934    1.8e-7 -> 1.3e-7
-  //   256 -> 608, 0.51M pairs, stride 2   1710 -> 1216 / 1095    2.1e-7 -> 1.4e-7
-  //   512 -> 608, 1.03M pairs             6880 -> 5513 / 4465    2.6e-7 -> 1.6e-7
-  //   608 -> 512, 1.03M pairs, every row  6580 -> 4720 / 4277    3.3e-7 -> 1.8e-7
-  //   304 -> 128, 1.69M pairs, stride 2   1523 -> 1235 / 1312    1.7e-7 -> 1.2e-7
-  //    64 -> 128, 1.54M pairs, 1 in 10     290 ->  328 /  500    (stays with the float form)
+  // Error against 64 bits, float form -> parts (times stand at parts_block, conv.hip):
+  //   128 -> 64   2.0e-7 -> 1.5e-7      512 -> 608   2.6e-7 -> 1.6e-7
+  //   128 -> 304  1.8e-7 -> 1.3e-7      608 -> 512   3.3e-7 -> 1.8e-7
+  //   256 -> 608  2.1e-7 -> 1.4e-7      304 -> 128   1.7e-7 -> 1.2e-7
   // With the sums of all chunks in one chain the error of the wide ones is 2.7e-7 to 4.1e-7.
   if constexpr (PARTS) {
     constexpr int NB = FORM == 5 ? 4 : 2;
